@@ -153,9 +153,8 @@ extern "C" int cpfft_destroy(cpfft_ctx* c) {
   if (c->f2d_cos) (void)hipFree(c->f2d_cos);
   {
     MlpBuffers& b = c->mlp;
-    void* mb[] = {b.params, b.pbf, b.grads, b.m, b.v, b.norm, b.logX, b.logT, b.Xb, b.Xf, b.Tb,
-                  b.H1, b.H2, b.Y, b.dY, b.dZ1, b.dZ2, b.H1b, b.H2b, b.dYb, b.dZ1b, b.dZ2b,
-                  b.part, b.Xv, b.ws};
+    void* mb[] = {b.params, b.pbf, b.grads, b.m, b.v, b.norm, b.logX, b.logT, b.Xf, b.Tb, b.Y,
+                  b.pk, b.gT, b.fT, b.part, b.stat, b.Xv, b.ws};
     for (void* q : mb)
       if (q) (void)hipFree(q);
   }
@@ -1075,17 +1074,14 @@ extern "C" int cpfft_mlp_init(cpfft_ctx* c, uint64_t seed, long capacity, int ba
     HIP_OK(hipMalloc(&b.norm, d.nnorm * sizeof(float)));
     HIP_OK(hipMalloc(&b.logX, capacity * d.nin * sizeof(float)));
     HIP_OK(hipMalloc(&b.logT, capacity * d.nout * sizeof(float)));
-    HIP_OK(hipMalloc(&b.Xb, (long)rows * d.nin * sizeof(uint16_t)));
     HIP_OK(hipMalloc(&b.Xf, (long)rows * d.nin * sizeof(float)));
     HIP_OK(hipMalloc(&b.Tb, (long)rows * d.nout * sizeof(float)));
-    float** f32[] = {&b.H1, &b.H2, &b.dZ1, &b.dZ2};
-    for (float** q : f32) HIP_OK(hipMalloc(q, (long)rows * kMlpHid * sizeof(float)));
     HIP_OK(hipMalloc(&b.Y, (long)rows * d.nout * sizeof(float)));
-    HIP_OK(hipMalloc(&b.dY, (long)rows * d.nout * sizeof(float)));
-    uint16_t** b16[] = {&b.H1b, &b.H2b, &b.dZ1b, &b.dZ2b};
-    for (uint16_t** q : b16) HIP_OK(hipMalloc(q, (long)rows * kMlpHid * sizeof(uint16_t)));
-    HIP_OK(hipMalloc(&b.dYb, (long)rows * d.nout * sizeof(uint16_t)));
-    HIP_OK(hipMalloc(&b.part, (long)mlp_loss_parts(b, rows) * sizeof(double)));
+    HIP_OK(hipMalloc(&b.pk, mlp_pack_len(d) * sizeof(uint16_t)));
+    HIP_OK(hipMalloc(&b.gT, mlp_grad_bf16(d, rows) * sizeof(uint16_t)));
+    HIP_OK(hipMalloc(&b.fT, mlp_grad_f32(d, rows) * sizeof(float)));
+    HIP_OK(hipMalloc(&b.part, (long)mlp_row_blocks(rows) * sizeof(double)));
+    HIP_OK(hipMalloc(&b.stat, mlp_stat_doubles() * sizeof(double)));
     HIP_OK(hipMalloc(&b.Xv, c->V * mlp_nin_pad(d.nin) * sizeof(uint16_t)));
     HIP_OK(hipMalloc(&b.ws, (long)d.nout * c->V * sizeof(float)));
     c->mlp_ready = true;
@@ -1156,16 +1152,13 @@ extern "C" int cpfft_mlp_train(cpfft_ctx* c, int iters, double lr, uint64_t seed
   MlpBuffers& b = c->mlp;
   const int rows = std::min<long>(4096, b.rows);
   mlp_stats(b, c->mlp_count, c->stream);
-  for (int it = 0; it < iters; ++it) {
-    mlp_weights_to_bf16(b, c->stream);
-    mlp_gather_batch(b, rows, c->mlp_count, (uint32_t)seed, (uint32_t)(c->mlp_steps + it), c->stream);
-    mlp_forward(b, rows, b.Xb, b.Y, c->stream);
-    mlp_backward(b, rows, b.Xb, b.Tb, b.grads, b.part, c->stream);
-    mlp_adam(b, (float)lr, c->mlp_steps + it + 1, c->stream);
-  }
+  mlp_pack_weights(b, c->stream);
+  for (int it = 0; it < iters; ++it)
+    mlp_train_step(b, rows, c->mlp_count, (uint32_t)seed, (uint32_t)(c->mlp_steps + it), (float)lr,
+                   c->mlp_steps + it + 1, c->stream);
   HIP_OK(hipGetLastError());
   c->mlp_steps += iters;
-  const int np = mlp_loss_parts(b, rows);
+  const int np = mlp_row_blocks(rows);
   std::vector<double> hp(np);
   HIP_OK(hipMemcpyAsync(hp.data(), b.part, np * sizeof(double), hipMemcpyDeviceToHost, c->stream));
   HIP_OK(hipStreamSynchronize(c->stream));
@@ -1211,11 +1204,10 @@ static int mlp_upload_batch(cpfft_ctx* c, const float* Xn, const float* Tn, int 
   MlpBuffers& b = c->mlp;
   if (n < 1 || n > b.rows) return fail(-1, "cpfft_mlp: batch size out of range");
   HIP_OK(hipMemcpyAsync(b.Xf, Xn, (long)n * b.d.nin * sizeof(float), hipMemcpyHostToDevice, c->stream));
-  mlp_to_bf16((long)n * b.d.nin, b.Xf, b.Xb, c->stream);
   if (Tn)
     HIP_OK(hipMemcpyAsync(b.Tb, Tn, (long)n * b.d.nout * sizeof(float), hipMemcpyHostToDevice,
                           c->stream));
-  mlp_weights_to_bf16(b, c->stream);
+  mlp_pack_weights(b, c->stream);
   HIP_OK(hipStreamSynchronize(c->stream));
   return 0;
 }
@@ -1224,7 +1216,7 @@ extern "C" int cpfft_mlp_forward(cpfft_ctx* c, const float* Xn, int n, float* Y)
   if (!c || !c->mlp_ready) return fail(-1, "cpfft_mlp_forward: cpfft_mlp_init first");
   int rc = mlp_upload_batch(c, Xn, nullptr, n);
   if (rc) return rc;
-  mlp_forward(c->mlp, n, c->mlp.Xb, c->mlp.Y, c->stream);
+  mlp_forward(c->mlp, n, c->mlp.Xf, c->mlp.Y, c->stream);
   HIP_OK(hipGetLastError());
   HIP_OK(hipStreamSynchronize(c->stream));
   HIP_OK(hipMemcpyAsync(Y, c->mlp.Y, (long)n * c->mlp.d.nout * sizeof(float), hipMemcpyDeviceToHost,
@@ -1239,11 +1231,10 @@ extern "C" int cpfft_mlp_grad(cpfft_ctx* c, const float* Xn, const float* Tn, in
   int rc = mlp_upload_batch(c, Xn, Tn, n);
   if (rc) return rc;
   MlpBuffers& b = c->mlp;
-  mlp_forward(b, n, b.Xb, b.Y, c->stream);
-  mlp_backward(b, n, b.Xb, b.Tb, b.grads, b.part, c->stream);
+  mlp_grad(b, n, b.Xf, b.Tb, c->stream);
   HIP_OK(hipGetLastError());
   HIP_OK(hipStreamSynchronize(c->stream));
-  const int np = mlp_loss_parts(b, n);
+  const int np = mlp_row_blocks(n);
   std::vector<double> hp(np);
   HIP_OK(hipMemcpyAsync(grad, b.grads, b.d.nparam * sizeof(float), hipMemcpyDeviceToHost, c->stream));
   HIP_OK(hipMemcpyAsync(hp.data(), b.part, np * sizeof(double), hipMemcpyDeviceToHost, c->stream));

@@ -48,34 +48,43 @@ struct MlpBuffers {
   float* logT = nullptr;    // logged converged slip increments [cap][nout]
   long cap = 0;
   int rows = 0;             // batch capacity of the training buffers
-  uint16_t* Xb = nullptr;   // [rows][nin] normalised BF16 inputs
-  float* Xf = nullptr;      // [rows][nin] FP32 inputs staged from the host
+  float* Xf = nullptr;      // [rows][nin] normalised FP32 inputs staged from the host
   float* Tb = nullptr;      // [rows][nout] normalised targets
-  float *H1 = nullptr, *H2 = nullptr, *Y = nullptr, *dY = nullptr, *dZ1 = nullptr, *dZ2 = nullptr;
-  uint16_t *H1b = nullptr, *H2b = nullptr, *dYb = nullptr, *dZ1b = nullptr, *dZ2b = nullptr;
-  double* part = nullptr;   // loss partial sums
+  float* Y = nullptr;       // [rows][nout] network outputs
+  uint16_t* pk = nullptr;   // packed BF16 weights of the training step (mlp_pack_len)
+  uint16_t* gT = nullptr;   // operands of the weight gradients (mlp_grad_bf16)
+  float* fT = nullptr;      // back-propagated errors for the bias gradients (mlp_grad_f32)
+  double* part = nullptr;   // loss partial sums [mlp_row_blocks(rows)]
+  double* stat = nullptr;   // column statistics (mlp_stat_doubles)
   uint16_t* Xv = nullptr;   // normalised BF16 inputs of every voxel [V][mlp_nin_pad(nin)]
   float* ws = nullptr;      // predicted slip increments for the warm start [nout][V]
 };
 
-void mlp_to_bf16(long n, const float* x, uint16_t* y, hipStream_t s);
+// BF16 copy of the weights for the inference kernel (pbf)
 void mlp_weights_to_bf16(const MlpBuffers& b, hipStream_t s);
-// Y[rows][nout] = network(Xb) (normalised units); H1, H2 kept for mlp_backward
-void mlp_forward(const MlpBuffers& b, int rows, const uint16_t* Xb, float* Y, hipStream_t s);
-// gradient of mean((Y - T)^2) over rows x nout into grads (b.Y from
-// mlp_forward); part[0..mlp_loss_parts(b, rows)) receives partial sums of
-// (Y - T)^2
-void mlp_backward(const MlpBuffers& b, int rows, const uint16_t* Xb, const float* T, float* grads,
-                  double* part, hipStream_t s);
-int mlp_loss_parts(const MlpBuffers& b, int rows);
-void mlp_adam(const MlpBuffers& b, float lr, long t, hipStream_t s);
-void mlp_gather_batch(const MlpBuffers& b, int rows, long count, uint32_t seed, uint32_t step,
-                      hipStream_t s);
+// packed BF16 copies for the training step (pk); mlp_train_step keeps them
+// current, so once before the first step after a change of params
+long mlp_pack_len(const MlpDims& d);
+void mlp_pack_weights(const MlpBuffers& b, hipStream_t s);
+// rows per launch are split into blocks of 32, each with a partial loss
+int mlp_row_blocks(int rows);
+long mlp_grad_bf16(const MlpDims& d, int rows);
+long mlp_grad_f32(const MlpDims& d, int rows);
+// Y[rows][nout] = network(Xf) (normalised units)
+void mlp_forward(const MlpBuffers& b, int rows, const float* Xf, float* Y, hipStream_t s);
+// gradient of mean((Y - T)^2) over rows x nout into b.grads, partial sums of
+// (Y - T)^2 into b.part[0..mlp_row_blocks(rows))
+void mlp_grad(const MlpBuffers& b, int rows, const float* Xf, const float* Tf, hipStream_t s);
+// one Adam step (step number t, learning rate lr) on rows drawn from the
+// log's first count pairs; partial losses as mlp_grad's
+void mlp_train_step(const MlpBuffers& b, int rows, long count, uint32_t seed, uint32_t step,
+                    float lr, long t, hipStream_t s);
+long mlp_stat_doubles();
 void mlp_stats(const MlpBuffers& b, long count, hipStream_t s);
 // Inference over all voxels in one launch: ws[k][e] = the network's output
 // k for the normalised inputs Xv[e] (row stride mlp_nin_pad(nin)),
 // denormalised (the weights must be in pbf).  BF16 operands, FP32
-// accumulation, the same rounding points as mlp_forward.
+// accumulation, the the rounding points of mlp_forward.
 void mlp_infer(const MlpBuffers& b, long V, hipStream_t s);
 
 }  // namespace cpfft

@@ -183,3 +183,55 @@ def test_fused_inference_matches_oracle_network(slip_set):
     assert ws.shape == (nout, N ** 3)
     assert err <= 2e-3
     s.close()
+
+
+@pytest.mark.parametrize("slip_set", [1, 80])
+@pytest.mark.parametrize("n", [1, 31, 32, 33, 255, 4096])
+def test_training_blocks_match_oracle(n, slip_set):
+    """Row counts around the training kernels' 32-row blocks and 16-row MFMA
+    steps; the tolerances of test_mlp_forward_and_gradient_match_oracle."""
+    s, _ = _solver(slip_set=slip_set)
+    s.mlp_init(seed=4, capacity=1024, batch=4096)
+    nin, nout, npar, _ = C.mlp_sizes(s.nslip)
+    p = s.mlp_params()[:npar]
+    rng = np.random.default_rng(n)
+    X = rng.standard_normal((n, nin)).astype(np.float32)
+    T = rng.standard_normal((n, nout)).astype(np.float32)
+    Yo, _ = M.forward(p, X, nout=nout)
+    Y = s.mlp_forward(X)
+    assert np.linalg.norm(Y - Yo) <= 2e-3 * np.linalg.norm(Yo)
+    g, loss = s.mlp_grad(X, T)
+    lo, go = M.loss_and_grad(p, X, T)
+    assert abs(loss - lo) <= 1e-3 * lo
+    off = M.offsets(nin, nout)
+    for a, b in zip(off[:-1], off[1:]):
+        assert np.linalg.norm(g[a:b] - go[a:b]) <= 1e-2 * np.linalg.norm(go[a:b]), (a, b)
+    s.close()
+
+
+@pytest.mark.parametrize("slip_set", [1, 80])
+@pytest.mark.parametrize("capacity", [1, 63, 200, 512])
+def test_log_statistics(capacity, slip_set):
+    """mean and deviation of the logged inputs (FP64 sums of FP32 values,
+    rounded once to FP32), log sizes around the blocks' row runs"""
+    s, _ = _solver(slip_set=slip_set)
+    s.drive_eps_sig(1, 0)
+    s.fill9(C.DFM, np.array([5e-4, 0, 0, 0, -2.5e-4, 0, 0, 0, -2.5e-4]))
+    s.daxpy(1.0, C.DFM, C.FN1)
+    s.drive_eps_sig(1, 1)
+    s.mlp_init(seed=4, capacity=capacity, batch=64)
+    X, _ = s.mlp_predict(1)
+    assert C.lib().cpfft_mlp_log(s.h, 1, 1) == 0
+    s.mlp_train(1)
+    nin, _, npar, _ = C.mlp_sizes(s.nslip)
+    norm = s.mlp_params()[npar:]
+    X = X[:capacity].astype(np.float64)
+    mean, sd = X.mean(0), X.std(0)
+    scale = abs(X).max(0)
+    assert (abs(norm[:nin] - mean) <= 1e-7 * scale + 1e-12).all()
+    # a column whose spread is below the rounding of its FP64 sums may round
+    # to zero, which the kernel replaces by one
+    got, tiny = norm[nin:2 * nin], sd <= 1e-12 * scale
+    assert (abs(got - sd) <= 1e-6 * sd + 1e-30)[~tiny].all()
+    assert (got[tiny & (sd == 0.0)] > 0).all()
+    s.close()
