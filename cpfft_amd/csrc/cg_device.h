@@ -15,9 +15,10 @@ struct CGScalars {
   double alpha, beta;
   double tolb, tol;
   double resnorm;  // |r| after the last update
+  double n2b;      // |b|
   int k;           // iterations completed
   int maxit;
-  int done;        // 0 running, 1 converged, 2 iteration limit reached
+  int done;        // 0 running, 1 converged, 2 iteration limit reached, 3 zero right-hand side
   int pad;
 };
 

@@ -52,19 +52,20 @@ struct cpfft_ctx {
   double* r = nullptr;   // CG residual
   double* p = nullptr;   // CG direction
   double* q = nullptr;   // CG operator image
-  double* tmp9 = nullptr;  // tangent_homo right-hand side
+  double* tmp9 = nullptr;  // second direction buffer (fft_grid.hip, reference operator)
   double* tan6 = nullptr;  // per-voxel material tangent [36][V]
   double* partials = nullptr;
   double* dpart = nullptr;  // p.q partial sums of the fused passes A or D
   double* rpart = nullptr;  // r.r partial sums of pass D in its update mode
   double* dres = nullptr;  // device results of reductions (16 doubles)
   double* hres = nullptr;  // pinned host mirror
-  CGScalars* dcg = nullptr;  // device scalars of the running CG solve
+  CGScalars* dcg = nullptr;  // device scalars of the running CG solve (two, see enqueue_pcg_grid)
   CGScalars* hcg = nullptr;  // pinned host mirror
   // tangent_homo's nine simultaneous solves: x, r, p, q per right-hand side
   double* th[4][9] = {};
   CGScalars* dcg9 = nullptr;
-  // on the planned path tangent_homo keeps no x: per right-hand side i,
+  int homo_group = 1;  // systems per launch of tangent_homo on fft_grid.hip's edges
+  // tangent_homo keeps no x: per right-hand side i,
   // hdc[9i..9i+9) receives the voxel sums of K4:p_i from pass C and
   // hm[9i..9i+9) the running sum of alpha * mean(K4:p_i) = mean(K4:x_i)
   double* hdc = nullptr;
@@ -122,6 +123,19 @@ static int upload_orients(cpfft_ctx* c, const std::vector<std::array<double, 3>>
   HIP_OK(hipMalloc(&c->orients, h.size() * sizeof(Orient<NS>)));
   HIP_OK(hipMemcpy(c->orients, h.data(), h.size() * sizeof(Orient<NS>), hipMemcpyHostToDevice));
   return 0;
+}
+
+// Right-hand sides of tangent_homo per launch on fft_grid.hip's kernels: as
+// many as 700 MB of spectra hold, so all nine up to 96^3.  (That the spectra
+// outgrow the 256 MB memory-side cache costs less than the launches: at 96^3
+// one, three and nine a launch took 85.0, 73.3 and 69.4 ms a call.)
+static int homo_group(const SpecGeom& g) {
+  const long one = 9 * g.S1 * (long)sizeof(cplx);
+  return (int)std::max(1L, std::min(9L, (700L << 20) / one));
+}
+// whether tangent_homo runs on fft_grid.hip's kernels
+static bool homo_grid(const SpecGeom& g) {
+  return gkdf_grid_edge(g.N) || (gkdf_slab_edge(g.N) && g.gamma_mode == 1);
 }
 
 static void drop_graphs(cpfft_ctx* c);
@@ -192,9 +206,7 @@ extern "C" int cpfft_create(int N, const cpfft_material* m, const double* angles
   c->V = (long)N * N * N;
   const long V = c->V;
   // geometry
-  int maxlds = 65536;
-  (void)hipDeviceGetAttribute(&maxlds, hipDeviceAttributeMaxSharedMemoryPerBlock, c->dev);
-  if (const char* why = make_spec_geom(N, gamma_mode, maxlds, c->geom)) {
+  if (const char* why = make_spec_geom(N, gamma_mode, c->geom)) {
     cpfft_destroy(c);
     return fail(-3, (std::string("cpfft_create: ") + why).c_str());
   }
@@ -237,7 +249,12 @@ extern "C" int cpfft_create(int N, const cpfft_material* m, const double* angles
     c->field_len[f] = lens[f];
     HIP_OK(hipMalloc(&c->fields[f], lens[f] * sizeof(double)));
   }
-  HIP_OK(hipMalloc(&c->spec, 2 * 9 * c->geom.S1 * sizeof(cplx)));
+  c->homo_group = homo_group(c->geom);
+  const bool grid = gkdf_grid_edge(N);
+  const long nspec = homo_grid(c->geom)
+                         ? std::max(18 * c->geom.S1, c->homo_group * grid_spec_len(c->geom))
+                         : 18 * c->geom.S1;
+  HIP_OK(hipMalloc(&c->spec, nspec * sizeof(cplx)));
   HIP_OK(hipMalloc(&c->r, 9 * V * sizeof(double)));
   HIP_OK(hipMalloc(&c->p, 9 * V * sizeof(double)));
   HIP_OK(hipMalloc(&c->q, 9 * V * sizeof(double)));
@@ -245,17 +262,19 @@ extern "C" int cpfft_create(int N, const cpfft_material* m, const double* angles
   HIP_OK(hipMalloc(&c->tan6, 36 * V * sizeof(double)));
   HIP_OK(hipMalloc(&c->partials, reduce_partials_count(9 * V) * sizeof(double)));
   // p.q partial sums: pass D's (gkdf_dot_parts) or pass A's (N*N/2, one per
-  // pencil pair)
-  HIP_OK(hipMalloc(&c->dpart, std::max({1, gkdf_dot_parts(N), N * N}) * sizeof(double)));
+  // pencil pair); on fft_grid.hip's edges of up to nine systems
+  HIP_OK(hipMalloc(&c->dpart,
+                   (grid ? 9 * grid_parts(N) : std::max(gkdf_dot_parts(N), N * N)) * sizeof(double)));
+  const int nrr = std::max({grid ? grid_rr_parts(N, false) : gkdf_dot_parts(N), grid_parts(N)});
   // r.r partial sums of up to nine systems (tangent_homo's right-hand sides)
-  HIP_OK(hipMalloc(&c->rpart, 9 * (size_t)std::max(1, gkdf_dot_parts(N)) * sizeof(double)));
+  HIP_OK(hipMalloc(&c->rpart, 9 * (size_t)nrr * sizeof(double)));
   HIP_OK(hipMalloc(&c->dres, 16 * sizeof(double)));
   HIP_OK(hipHostMalloc(&c->hres, 16 * sizeof(double), hipHostMallocDefault));
-  HIP_OK(hipMalloc(&c->dcg, sizeof(CGScalars)));
+  HIP_OK(hipMalloc(&c->dcg, 2 * sizeof(CGScalars)));
   HIP_OK(hipHostMalloc(&c->hcg, sizeof(CGScalars), hipHostMallocDefault));
   for (int a = 0; a < 4; ++a)
     for (int i = 0; i < 9; ++i) HIP_OK(hipMalloc(&c->th[a][i], 9 * V * sizeof(double)));
-  HIP_OK(hipMalloc(&c->dcg9, 9 * sizeof(CGScalars)));
+  HIP_OK(hipMalloc(&c->dcg9, 18 * sizeof(CGScalars)));
   HIP_OK(hipMalloc(&c->hdc, 81 * sizeof(double)));
   HIP_OK(hipMalloc(&c->hm, 81 * sizeof(double)));
   HIP_OK(hipMalloc(&c->hpq, 9L * k4_contract_multi_blocks(V) * sizeof(double)));
@@ -500,25 +519,72 @@ extern "C" int cpfft_f2disp(cpfft_ctx* c, const double* F, const double lengths[
 // CG iterations enqueued per host round trip
 static constexpr int kChunk = 8;
 
+// Whether p.q is formed as p.(K4:p): with the textbook operator, a symmetric
+// projection.  (The reference's is one too for odd N, but its solves take
+// p.q as fftPcg does: at a tolerance below the rounding floor, as in the
+// reference's example deck, the two differ in the iterations they spend there.)
+static bool projection(const cpfft_ctx* c) { return c->geom.gamma_mode == 1; }
+
+// kChunk CG iterations on fft_grid.hip's edges.  The convergence test of an
+// iteration is part of the next one's first kernel where grid_fused_check
+// says so; blocks then read the old state while one of them writes the new,
+// so the state alternates between two copies (kChunk is even: the first one
+// holds it between chunks) and the chunk ends with a test of its own.  The
+// direction alternates between two fields for the same reason: blocks read
+// all of the old one to form their component of the new.
+static_assert(kChunk % 2 == 0, "the state ends a chunk where it began");
+static void enqueue_pcg_grid(cpfft_ctx* c, double* x, int base) {
+  const bool pr = projection(c), fchk = grid_fused_check(c->N);
+  const int np = grid_rr_parts(c->N, pr);
+  double* pd[2] = {c->p, pr ? c->q : c->tmp9};
+  CGScalars* cs[2] = {c->dcg, fchk ? c->dcg + 1 : c->dcg};
+  GridCG k{};
+  k.nrhs = 1;
+  k.r[0] = c->r;
+  k.x[0] = x;
+  k.out[0] = pr ? nullptr : c->q;
+  k.K4 = c->fields[CPFFT_K4];
+  k.spec = c->spec;
+  k.tw = c->tw;
+  k.pq = c->dpart;
+  k.rr = c->rpart;
+  for (int j = 0; j < kChunk; ++j) {
+    k.p_old[0] = pd[j & 1];
+    k.p_new[0] = pd[(j & 1) ^ 1];
+    k.cs_old = cs[j & 1];
+    k.cs_new = cs[(j & 1) ^ 1];
+    k.chk = fchk && j > 0;
+    c->ev_cur = base + j;
+    tstart(c, 0);
+    launch_cg_grid(c->geom, k, 0, c->stream);
+    tstop(c, 0);
+    tstart(c, 2);
+    launch_cg_grid(c->geom, k, 1, c->stream);
+    if (!fchk || j == kChunk - 1) launch_cg_check(c->rpart, np, c->dcg, c->stream);
+    tstop(c, 2);
+  }
+  c->ev_cur = -1;
+}
+
 // kChunk CG iterations of cpfft_pcg on the solution x: q = A p (pass A also
-// forms p = r + beta p, pass D the p.q partial sums on the planned path),
-// alpha, x and r updates, convergence test.  Every kernel reads the scalars
-// in c->dcg and returns at once after convergence, so the chunk has no
-// host-side control flow and can be replayed from a graph.
+// forms p = r + beta p, pass D the p.q partial sums), alpha, x and r updates,
+// convergence test.  Every kernel reads the scalars in c->dcg and returns at
+// once after convergence, so the chunk has no host-side control flow and can
+// be replayed from a graph.
 // base: the solve's iteration number of the chunk's first iteration (only
 // labels timing events)
 static void enqueue_pcg_chunk(cpfft_ctx* c, double* x, int base = 0) {
+  if (gkdf_grid_edge(c->N)) return enqueue_pcg_grid(c, x, base);
   const long n = 9 * c->V;
   SpecGeom g = c->geom;
   g.skip = &c->dcg->done;
-  const bool fused = gkdf_pencil_supported(c->N);
   const int ndp = gkdf_dot_parts(c->N);
   // The textbook operator is a symmetric projection and p lies in its
   // range, so p.q = p.(K4:p): pass A forms it, alpha follows pass A, and
   // pass D applies x += alpha p, r -= alpha q without storing q.  The
   // reference's even-N operator is not a projection: there pass D forms p.q
   // and a separate kernel updates x and r.
-  const bool apq = fused && c->geom.gamma_mode == 1;
+  const bool apq = projection(c);
   CGFuse fz{c->p, c->r, c->dcg, c->p, c->dpart, nullptr, nullptr, 0, nullptr, nullptr, nullptr};
   if (apq) {
     fz.dot_p = nullptr;
@@ -532,23 +598,16 @@ static void enqueue_pcg_chunk(cpfft_ctx* c, double* x, int base = 0) {
   for (int j = 0; j < kChunk; ++j) {
     c->ev_cur = base + j;
     tstart(c, 0);
-    if (fused) {
-      launch_gkdf_pencil(g, c->p, c->fields[CPFFT_K4], c->q, c->spec, c->tw, c->stream, &fz);
-    } else {
-      launch_gkdf(g, c->p, c->fields[CPFFT_K4], c->q, c->spec, c->tw, c->stream);
-    }
+    launch_gkdf_pencil(g, c->p, c->fields[CPFFT_K4], c->q, c->spec, c->tw, c->stream, &fz);
     tstop(c, 0);
     tstart(c, 2);
     if (apq) {
       launch_cg_check(c->rpart, ndp, c->dcg, c->stream);
-    } else if (fused) {
+    } else {
       launch_cg_alpha(c->dpart, ndp, c->dcg, c->stream);
       launch_cg_update_check(n, c->dcg, c->p, c->q, x, c->r, c->partials, c->stream);
-    } else {
-      launch_cg_tail(n, c->dcg, c->p, c->q, x, c->r, c->partials, c->stream);
     }
     tstop(c, 2);
-    if (!fused) launch_cg_dir_dev(n, c->dcg, c->r, c->p, c->stream);
   }
   c->ev_cur = -1;
 }
@@ -624,6 +683,11 @@ static void drop_graphs(cpfft_ctx* c) {
 static std::mutex g_tune_mu;
 static std::map<std::pair<int, int>, PencilTune> g_tune;
 
+// value of candidate v of pass p, 0 if there is none
+static int tune_value(int N, int p, int v) {
+  return gkdf_grid_edge(N) ? grid_candidate(N, p, v) : pencil_candidate(N, p, v);
+}
+
 static void apply_tune(cpfft_ctx* c, const PencilTune& t) {
   const bool changed = t.a != c->geom.tune.a || t.a0 != c->geom.tune.a0 || t.b != c->geom.tune.b ||
                        t.c != c->geom.tune.c;
@@ -636,7 +700,7 @@ static void apply_tune(cpfft_ctx* c, const PencilTune& t) {
 
 extern "C" int cpfft_autotune(cpfft_ctx* c, int reps, int force) {
   if (!c) return fail(-1, "cpfft_autotune: null context");
-  if (!gkdf_pencil_supported(c->N)) return 1;
+  if (!tune_value(c->N, 0, 0)) return 1;
   if (reps < 1) reps = 10;
   const std::pair<int, int> key(c->dev, c->N);
   if (!force) {
@@ -660,11 +724,16 @@ extern "C" int cpfft_autotune(cpfft_ctx* c, int reps, int force) {
     float best = 0.f;
     int bi = 0;
     for (int v = 0; v < kPencilCands; ++v) {
-      if (!pencil_candidate(c->N, pass, v)) continue;
-      launch_pencil_pass(c->geom, pass, v, F, K4, c->spec, c->tw, c->stream);  // warm-up
+      if (!tune_value(c->N, pass, v)) continue;
+      auto one = [&] {
+        if (gkdf_grid_edge(c->N))
+          launch_grid_pass(c->geom, pass, v, F, K4, c->spec, c->tw, c->stream);
+        else
+          launch_pencil_pass(c->geom, pass, v, F, K4, c->spec, c->tw, c->stream);
+      };
+      one();  // warm-up
       HIP_OK(hipEventRecord(e0, c->stream));
-      for (int r = 0; r < reps; ++r)
-        launch_pencil_pass(c->geom, pass, v, F, K4, c->spec, c->tw, c->stream);
+      for (int r = 0; r < reps; ++r) one();
       HIP_OK(hipEventRecord(e1, c->stream));
       HIP_OK(hipEventSynchronize(e1));
       float ms = 0.f;
@@ -689,19 +758,19 @@ extern "C" int cpfft_get_tune(cpfft_ctx* c, int out[4]) {
   if (!c) return fail(-1, "cpfft_get_tune: null context");
   const PencilTune& t = c->geom.tune;
   const int idx[4] = {t.a, t.a0, t.b, t.c};
-  for (int p = 0; p < 4; ++p) out[p] = pencil_candidate(c->N, p, idx[p]);
+  for (int p = 0; p < 4; ++p) out[p] = tune_value(c->N, p, idx[p]);
   return 0;
 }
 
 extern "C" int cpfft_set_tune(cpfft_ctx* c, const int in[4]) {
   if (!c) return fail(-1, "cpfft_set_tune: null context");
-  if (!gkdf_pencil_supported(c->N)) return fail(-1, "cpfft_set_tune: no tunable shapes for this N");
+  if (!tune_value(c->N, 0, 0)) return fail(-1, "cpfft_set_tune: no tunable shapes for this N");
   PencilTune t;
   int* knob[4] = {&t.a, &t.a0, &t.b, &t.c};
   for (int p = 0; p < 4; ++p) {
     int found = -1;
     for (int v = 0; v < kPencilCands && found < 0; ++v)
-      if (pencil_candidate(c->N, p, v) == in[p] && in[p] > 0) found = v;
+      if (tune_value(c->N, p, v) == in[p] && in[p] > 0) found = v;
     if (found < 0) return fail(-1, "cpfft_set_tune: shape is not among the candidates for this N");
     *knob[p] = found;
   }
@@ -748,32 +817,18 @@ extern "C" int cpfft_pcg(cpfft_ctx* c, const double* b, double* x, double tol, i
                          double* relres) {
   if (!c) return fail(-1, "cpfft_pcg: null context");
   const long n = 9 * c->V;
-  const int maxIter = c->cg_maxit;
   const double eps = 2.220446049250313e-16;
+  int rc;
   if (iters) *iters = 0;
   if (relres) *relres = 0.0;
-  launch_fill(n, 0.0, x, c->stream);
-  double bb;
-  int rc = dot_host(c, b, b, &bb);
-  if (rc) return rc;
-  double n2b = sqrt(bb), tolb = tol * n2b;
-  if (tol <= eps || tol >= 1.0) return fail(-1, "cpfft_pcg: improper tolerance");
-  if (n2b <= eps) return 1;
-  launch_copy(n, b, c->r, c->stream);
-  launch_copy(n, b, c->p, c->stream);
+  const bool bad_tol = tol <= eps || tol >= 1.0;
+  if (bad_tol || x == b) launch_fill(n, 0.0, x, c->stream);
+  if (bad_tol) return fail(-1, "cpfft_pcg: improper tolerance");
   // Iterations run on the device with their scalars in c->dcg; the host
   // enqueues them in chunks and reads the state once per chunk.  Kernels of
   // iterations enqueued after convergence return at once.
-  CGScalars h{};
-  h.rr = bb;
-  h.tolb = tolb;
-  h.tol = tol;
-  h.resnorm = n2b;
-  h.k = 0;
-  h.maxit = maxIter;
-  h.done = 0;
-  *c->hcg = h;
-  HIP_OK(hipMemcpyAsync(c->dcg, c->hcg, sizeof(CGScalars), hipMemcpyHostToDevice, c->stream));
+  launch_cg_start(n, b, x, c->r, gkdf_grid_edge(c->N) ? nullptr : c->p, c->partials, c->stream);
+  launch_cg_init(c->partials, cg_start_parts(), tol, c->cg_maxit, 3, c->dcg, nullptr, 1, c->stream);
   const bool graph = c->use_graphs && !c->timing;
   hipGraphExec_t ge = nullptr;
   if (graph) {
@@ -800,13 +855,20 @@ extern "C" int cpfft_pcg(cpfft_ctx* c, const double* b, double* x, double tol, i
     if (c->hcg->done) break;
   }
   const int k = c->hcg->k;
+  if (c->hcg->done == 3) {  // zero right-hand side
+    if (c->timing)
+      for (int f : {0, 2}) {
+        while (c->ev_n[f] > 0 && c->ev_it[f][c->ev_n[f] - 1] >= 0) c->ev_n[f]--;
+      }
+    return 1;
+  }
   if (c->timing)  // drop the events of the no-op iterations at the end
     for (int f : {0, 2})
       while (c->ev_n[f] > 0 && c->ev_it[f][c->ev_n[f] - 1] >= k) c->ev_n[f]--;
   c->cg_iters += k;
   c->gkdf_calls += k;
   if (iters) *iters = k;
-  if (relres) *relres = c->hcg->resnorm / n2b;
+  if (relres) *relres = c->hcg->resnorm / c->hcg->n2b;
   if (c->hcg->done == 2) return fail(-2, "cpfft_pcg: no convergence within the iteration limit");
   return 0;
 }
@@ -879,7 +941,96 @@ extern "C" int cpfft_drive_eps_sig(cpfft_ctx* c, int step, int iiter) {
 // path first p_i = r_i + beta_i p_i), then each solve applies the operator
 // without K4 in place and its own alpha, update and test.  Kernels of
 // finished solves return at once, so the chunk can be replayed from a graph.
+// Whether tangent_homo's K4:p_i are formed by a launch of their own, which
+// reads r and p once instead of once per component: from 40^3 on (48^3:
+// 10.7 against 12.8 ms a call; 32^3: 3.7 against 3.5, its blocks too few to
+// fill the chip).
+static bool homo_contract(const cpfft_ctx* c) {
+  return c->N >= 40 && gkdf_slab_edge(c->N);
+}
+
+// With fft_grid.hip's kernels the systems share every launch.
+static void enqueue_homo_slab(cpfft_ctx* c) {
+  const long V = c->V;
+  const bool pr = projection(c);
+  const int nb = k4_contract_multi_blocks(V);
+  const int npq = pr ? nb : grid_parts(c->N), np = grid_rr_parts(c->N, pr);
+  double* const pq = pr ? c->hpq : c->dpart;
+  Ptr9 pp;
+  Ptr9r rr;
+  for (int i = 0; i < 9; ++i) {
+    pp.p[i] = c->th[2][i];
+    pp.q[i] = c->th[3][i];
+    rr.r[i] = c->th[1][i];
+  }
+  for (int j = 0; j < kChunk; ++j) {
+    launch_k4_contract_multi(V, c->fields[CPFFT_K4], pp, c->dcg9, 9, c->stream, &rr,
+                             pr ? c->hpq : nullptr);
+    for (int i0 = 0; i0 < 9; i0 += c->homo_group) {
+      GridCG k{};
+      k.nrhs = std::min(c->homo_group, 9 - i0);
+      for (int i = 0; i < k.nrhs; ++i) {
+        k.q[i] = c->th[3][i0 + i];
+        k.r[i] = c->th[1][i0 + i];
+        k.p_new[i] = c->th[2][i0 + i];
+        k.out[i] = pr ? nullptr : c->th[3][i0 + i];
+      }
+      k.npq = nb;
+      k.spec = c->spec;
+      k.tw = c->tw;
+      k.cs_old = k.cs_new = c->dcg9 + i0;
+      k.pq = pq + (long)i0 * npq;
+      k.rr = c->rpart + (long)i0 * np;
+      k.dc = c->hdc + 9 * i0;
+      launch_cg_grid(c->geom, k, 0, c->stream);
+      launch_cg_grid(c->geom, k, 1, c->stream);
+    }
+    launch_cg_check(c->rpart, np, c->dcg9, c->stream, c->hdc, c->hm, 1.0 / (double)V, 9, np);
+  }
+}
+
+// The same with K4:p_i formed by the forward pass (see enqueue_pcg_grid for
+// the two copies of the state and of the direction).
+static void enqueue_homo_grid(cpfft_ctx* c) {
+  const bool pr = projection(c), fchk = grid_fused_check(c->N);
+  const int npq = grid_parts(c->N), np = grid_rr_parts(c->N, pr);
+  const double sc = 1.0 / (double)c->V;
+  double* const* R = c->th[1];
+  double* const* Q = c->th[3];
+  double* const* pd[2] = {c->th[2], pr ? c->th[3] : c->th[0]};
+  CGScalars* cs[2] = {c->dcg9, fchk ? c->dcg9 + 9 : c->dcg9};
+  for (int j = 0; j < kChunk; ++j) {
+    for (int i0 = 0; i0 < 9; i0 += c->homo_group) {
+      GridCG k{};
+      k.nrhs = std::min(c->homo_group, 9 - i0);
+      for (int i = 0; i < k.nrhs; ++i) {
+        k.p_old[i] = pd[j & 1][i0 + i];
+        k.p_new[i] = pd[(j & 1) ^ 1][i0 + i];
+        k.r[i] = R[i0 + i];
+        k.out[i] = pr ? nullptr : Q[i0 + i];
+      }
+      k.K4 = c->fields[CPFFT_K4];
+      k.spec = c->spec;
+      k.tw = c->tw;
+      k.cs_old = cs[j & 1] + i0;
+      k.cs_new = cs[(j & 1) ^ 1] + i0;
+      k.chk = fchk && j > 0;
+      k.pq = c->dpart + (long)i0 * npq;
+      k.rr = c->rpart + (long)i0 * np;
+      k.dc = c->hdc + 9 * i0;
+      k.m = c->hm + 9 * i0;
+      k.scale = sc;
+      launch_cg_grid(c->geom, k, 0, c->stream);
+      launch_cg_grid(c->geom, k, 1, c->stream);
+    }
+    if (!fchk || j == kChunk - 1)
+      launch_cg_check(c->rpart, np, c->dcg9, c->stream, c->hdc, c->hm, sc, 9, np);
+  }
+}
+
 static void enqueue_homo_chunk(cpfft_ctx* c) {
+  if (homo_grid(c->geom))
+    return homo_contract(c) ? enqueue_homo_slab(c) : enqueue_homo_grid(c);
   const long V = c->V, n = 9 * V;
   double* const* X = c->th[0];
   double* const* R = c->th[1];
@@ -893,93 +1044,75 @@ static void enqueue_homo_chunk(cpfft_ctx* c) {
     pp.q[i] = Q[i];
     rr.r[i] = R[i];
   }
-  const bool fused = gkdf_pencil_supported(c->N);
   const int ndp = gkdf_dot_parts(c->N);
   // textbook operator: p_i . q_i = p_i . (K4:p_i) from the K4 pass, alpha
   // before the operator, pass D updates r_i without storing q_i (see
   // enqueue_pcg_chunk); the reference's even-N operator: p.q from pass D
-  const bool apq = fused && c->geom.gamma_mode == 1;
+  const bool apq = projection(c);
   const int nb = k4_contract_multi_blocks(V);
+  const double sc = 1.0 / (double)V;
   for (int j = 0; j < kChunk; ++j) {
-    launch_k4_contract_multi(V, K4, pp, c->dcg9, 9, c->stream, fused ? &rr : nullptr,
-                             apq ? c->hpq : nullptr);
+    launch_k4_contract_multi(V, K4, pp, c->dcg9, 9, c->stream, &rr, apq ? c->hpq : nullptr);
     // the nine alphas in one launch (one block per right-hand side)
     if (apq) launch_cg_alpha(c->hpq, nb, c->dcg9, c->stream, 9, nb);
     for (int i = 0; i < 9; ++i) {
       SpecGeom g = c->geom;
       g.skip = &c->dcg9[i].done;
       // in place: pass A reads all of Q[i] before pass D writes it
-      if (fused) {
-        // pass C: voxel sums of K4:p_i, from which the check accumulates
-        // mean(K4:x_i); x_i itself is never formed
-        double* const dc = c->hdc + 9 * i;
-        double* const m = c->hm + 9 * i;
-        const double sc = 1.0 / (double)V;
-        if (apq) {
-          const CGFuse fz{nullptr, nullptr, c->dcg9 + i, nullptr, nullptr, dc, nullptr, 0,
-                          R[i], nullptr, c->rpart + (long)i * ndp};
-          launch_gkdf_pencil(g, Q[i], nullptr, Q[i], c->spec, c->tw, c->stream, &fz);
-        } else {
-          const CGFuse fz{nullptr, nullptr, c->dcg9 + i, Pd[i], c->dpart, dc, nullptr, 0,
-                          nullptr, nullptr, nullptr};
-          launch_gkdf_pencil(g, Q[i], nullptr, Q[i], c->spec, c->tw, c->stream, &fz);
-          launch_cg_alpha(c->dpart, ndp, c->dcg9 + i, c->stream);
-          launch_cg_update_check(n, c->dcg9 + i, Pd[i], Q[i], X[i], R[i], c->partials, c->stream,
-                                 false, dc, m, sc);
-        }
+      // pass C: voxel sums of K4:p_i, from which the check accumulates
+      // mean(K4:x_i); x_i itself is never formed
+      double* const dc = c->hdc + 9 * i;
+      double* const m = c->hm + 9 * i;
+      if (apq) {
+        const CGFuse fz{nullptr, nullptr, c->dcg9 + i, nullptr, nullptr, dc, nullptr, 0,
+                        R[i], nullptr, c->rpart + (long)i * ndp};
+        launch_gkdf_pencil(g, Q[i], nullptr, Q[i], c->spec, c->tw, c->stream, &fz);
       } else {
-        launch_gkdf(g, Q[i], nullptr, Q[i], c->spec, c->tw, c->stream);
-        launch_cg_tail(n, c->dcg9 + i, Pd[i], Q[i], X[i], R[i], c->partials, c->stream);
-        launch_cg_dir_dev(n, c->dcg9 + i, R[i], Pd[i], c->stream);
+        const CGFuse fz{nullptr, nullptr, c->dcg9 + i, Pd[i], c->dpart, dc, nullptr, 0,
+                        nullptr, nullptr, nullptr};
+        launch_gkdf_pencil(g, Q[i], nullptr, Q[i], c->spec, c->tw, c->stream, &fz);
+        launch_cg_alpha(c->dpart, ndp, c->dcg9 + i, c->stream);
+        launch_cg_update_check(n, c->dcg9 + i, Pd[i], Q[i], X[i], R[i], c->partials, c->stream,
+                               false, dc, m, sc);
       }
     }
     // the nine convergence tests in one launch, after all nine operators
-    if (apq)
-      launch_cg_check(c->rpart, ndp, c->dcg9, c->stream, c->hdc, c->hm, 1.0 / (double)V, 9, ndp);
+    if (apq) launch_cg_check(c->rpart, ndp, c->dcg9, c->stream, c->hdc, c->hm, sc, 9, ndp);
   }
 }
 
 extern "C" int cpfft_tangent_homo(cpfft_ctx* c, double tol, double C_homo[81]) {
   if (!c) return fail(-1, "cpfft_tangent_homo: null context");
   const long V = c->V, n = 9 * V;
-  const int maxIter = c->cg_maxit;
   const double eps = 2.220446049250313e-16;
   if (tol <= eps || tol >= 1.0) return fail(-1, "cpfft_tangent_homo: improper tolerance");
-  const bool fused = gkdf_pencil_supported(c->N);
-  double* const* X = c->th[0];
   double* const* R = c->th[1];
-  double* const* Pd = c->th[2];
   double* const* Q = c->th[3];
   const double* K4 = c->fields[CPFFT_K4];
-  // right-hand sides b_i = -G(K4 : E_i) in R[i]
-  for (int i = 0; i < 9; ++i) {
-    launch_gather_k4_col(V, i, K4, Q[i], c->stream);
-    tstart(c, 3);
-    launch_gkdf(c->geom, Q[i], nullptr, R[i], c->spec, c->tw, c->stream);
-    tstop(c, 3);
-    c->gkdf_calls++;
-    launch_scal(n, -1.0, R[i], c->stream);
-    launch_dot(R[i], R[i], n, c->partials, c->dres + i, c->stream);
+  int rc;
+  // right-hand sides b_i = -G(K4 : E_i) in R[i]; a zero one needs no
+  // iterations (dF_i = 0)
+  if (homo_grid(c->geom)) {
+    const int np = grid_parts(c->N);
+    for (int i0 = 0; i0 < 9; i0 += c->homo_group) {
+      tstart(c, 3);
+      launch_homo_rhs_grid(c->geom, K4, i0, std::min(c->homo_group, 9 - i0), R + i0, c->spec, c->tw,
+                           c->rpart + (long)i0 * np, c->stream);
+      tstop(c, 3);
+    }
+    launch_cg_init(c->rpart, np, tol, c->cg_maxit, 1, c->dcg9, c->hm, 9, c->stream);
+  } else {
+    for (int i = 0; i < 9; ++i) {
+      launch_gather_k4_col(V, i, K4, Q[i], c->stream);
+      tstart(c, 3);
+      launch_gkdf(c->geom, Q[i], nullptr, R[i], c->spec, c->tw, c->stream);
+      tstop(c, 3);
+      launch_scal(n, -1.0, R[i], c->stream);
+      launch_dot(R[i], R[i], n, c->partials, c->dres + i, c->stream);
+    }
+    launch_cg_init(c->dres, 1, tol, c->cg_maxit, 1, c->dcg9, c->hm, 9, c->stream);
   }
-  int rc = read_res(c, 9);
-  if (rc) return rc;
-  double n2b[9];
-  for (int i = 0; i < 9; ++i) {
-    const double bb = c->hres[i];
-    n2b[i] = sqrt(bb);
-    CGScalars h{};
-    h.rr = bb;
-    h.tolb = tol * n2b[i];
-    h.tol = tol;
-    h.resnorm = n2b[i];
-    h.maxit = maxIter;
-    h.done = (n2b[i] <= eps) ? 1 : 0;  // zero right-hand side: dF_i = 0
-    c->hcg9[i] = h;
-    if (!fused) launch_fill(n, 0.0, X[i], c->stream);
-    launch_copy(n, R[i], Pd[i], c->stream);
-  }
-  HIP_OK(hipMemcpyAsync(c->dcg9, c->hcg9, 9 * sizeof(CGScalars), hipMemcpyHostToDevice, c->stream));
-  if (fused) launch_fill(81, 0.0, c->hm, c->stream);
+  c->gkdf_calls += 9;
   const bool graph = c->use_graphs && !c->timing;
   if (graph && !c->homo_graph &&
       (rc = capture_chunk(c, 1, [&] { enqueue_homo_chunk(c); }, &c->homo_graph)))
@@ -1002,24 +1135,13 @@ extern "C" int cpfft_tangent_homo(cpfft_ctx* c, double tol, double C_homo[81]) {
     c->gkdf_calls += c->hcg9[i].k;
     if (c->hcg9[i].done == 2) return fail(-2, "cpfft_tangent_homo: CG did not converge within the iteration limit");
   }
-  if (fused) {
-    // C_homo(9(j-1)+i) = mean(K4 : E_i)_j + mean(K4 : x_i)_j, the first
-    // term the mean of K4 component 9j+i, the second accumulated above
-    double* hm = c->hhm;
-    HIP_OK(hipMemcpyAsync(hm, c->hm, 81 * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-    for (int j = 0; j < 9; ++j) {
-      launch_mean9(K4 + (long)9 * j * V, V, c->partials, c->dres, c->stream);
-      if ((rc = read_res(c, 9))) return rc;
-      for (int i = 0; i < 9; ++i) C_homo[9 * j + i] = c->hres[i] + hm[9 * i + j];
-    }
-    return 0;
-  }
-  for (int i = 0; i < 9; ++i) {
-    launch_add_identity_comp(V, i, X[i], c->stream);
-    launch_k4_dot9(V, K4, X[i], c->partials, c->dres, c->stream);
-    if ((rc = read_res(c, 9))) return rc;
-    for (int j = 0; j < 9; ++j) C_homo[9 * j + i] = c->hres[j];
-  }
+  // C_homo(9(j-1)+i) = mean(K4 : E_i)_j + mean(K4 : x_i)_j, the first term
+  // the mean of K4 component 9j+i, the second accumulated above
+  launch_mean81(K4, V, c->hm, c->partials, c->hdc, c->stream);
+  HIP_OK(hipGetLastError());
+  HIP_OK(hipMemcpyAsync(c->hhm, c->hdc, 81 * sizeof(double), hipMemcpyDeviceToHost, c->stream));
+  HIP_OK(hipStreamSynchronize(c->stream));
+  for (int i = 0; i < 81; ++i) C_homo[i] = c->hhm[i];
   return 0;
 }
 

@@ -1,16 +1,5 @@
 // cpfft_kernels.hip -- CDNA4 (gfx950) kernels of the CPFFT solver step.
 //
-//  * G_K_dF (src/G_K_dF.f:11-87) as five passes over an R2C half spectrum
-//    held in HBM, [9][N][N][N/2+1] complex (x slowest):
-//      1. z: fused K4:F contraction (ddot42n, G_K_dF.f:241-268) + real-to-
-//         complex FFT along z, one workgroup per (x,y) pencil
-//      2. y: complex FFT along y, one workgroup per (c, x, kz tile)
-//      3. x: forward FFT along x, Green projection for all nine
-//         components, inverse FFT along x, one workgroup per (ky, kz tile)
-//      4. y: inverse complex FFT
-//      5. z: complex-to-real FFT with the 1/N^3 scale
-//    FFTs run in LDS as mixed-radix (4,2,3,5,generic) Stockham stages with
-//    ping-pong buffers; twiddles come from a table of N-th roots of unity.
 //  * BLAS-1 and reductions for CG, Newton norms and volume averages
 //    (FFT_nr3.f:85-147, tangent_homo.f:62-66): deterministic two-stage
 //    block reductions (fixed order, no floating-point atomics).
@@ -24,276 +13,30 @@ namespace cpfft {
 
 static constexpr int kBlock = 256;
 
-// ------------------------------------------------------------------ FFT
-// Twiddle for exponent e (0 <= e < N: every caller's exponent t*k*N/(Ns*r)
-// with t < r, k < Ns, or ((q t) mod r) * N/r, stays below N) of the N-th
-// root table, conjugated for the inverse transform.
-__device__ inline cplx tw_get(const cplx* __restrict__ tw, int, int e, double sgn) {
-  cplx w = tw[e];
-  w.im *= sgn;  // table holds exp(-2 pi i k/N); sgn=+1 forward, -1 inverse
-  return w;
-}
-
-__device__ inline cplx cmul(cplx a, cplx b) {
-  return cplx{a.re * b.re - a.im * b.im, a.re * b.im + a.im * b.re};
-}
-
-// Batched in-LDS complex FFT.  Line L, element n lives at
-// buf[L*ls + n*es]; tmp has the same layout.  fwd: +1 forward, -1 inverse
-// (unscaled).  Result in buf.  All threads of the block must call it.
-__device__ void lds_fft(cplx* buf, cplx* tmp, int nlines, int ls, int es, const FftPlan& pl,
-                        const cplx* __restrict__ tw, double fwd) {
-  const int N = pl.n;
-  const int T = blockDim.x, tid = threadIdx.x;
-  int Ns = 1;
-  cplx* src = buf;
-  cplx* dst = tmp;
-  for (int st = 0; st < pl.nst; ++st) {
-    const int r = pl.rad[st];
-    const int nb = N / r;
-    const int total = nlines * nb;
-    const int tstride = N / (Ns * r);  // twiddle exponent step: exp(-2pi i t k/(Ns r))
-    for (int b = tid; b < total; b += T) {
-      const int line = b / nb;
-      const int j = b - line * nb;
-      const int k = j % Ns;
-      const cplx* s = src + line * ls;
-      cplx* d = dst + line * ls;
-      const int o = (j / Ns) * Ns * r + k;
-      if (r == 2) {
-        cplx a0 = s[j * es];
-        cplx a1 = cmul(s[(j + nb) * es], tw_get(tw, N, k * tstride, fwd));
-        d[o * es] = cplx{a0.re + a1.re, a0.im + a1.im};
-        d[(o + Ns) * es] = cplx{a0.re - a1.re, a0.im - a1.im};
-      } else if (r == 4) {
-        cplx a0 = s[j * es];
-        cplx a1 = cmul(s[(j + nb) * es], tw_get(tw, N, k * tstride, fwd));
-        cplx a2 = cmul(s[(j + 2 * nb) * es], tw_get(tw, N, 2 * k * tstride, fwd));
-        cplx a3 = cmul(s[(j + 3 * nb) * es], tw_get(tw, N, 3 * k * tstride, fwd));
-        cplx b0{a0.re + a2.re, a0.im + a2.im}, b1{a0.re - a2.re, a0.im - a2.im};
-        cplx b2{a1.re + a3.re, a1.im + a3.im}, b3{a1.re - a3.re, a1.im - a3.im};
-        // multiply b3 by -i (forward) or +i (inverse)
-        cplx b3r{fwd * b3.im, -fwd * b3.re};
-        d[o * es] = cplx{b0.re + b2.re, b0.im + b2.im};
-        d[(o + Ns) * es] = cplx{b1.re + b3r.re, b1.im + b3r.im};
-        d[(o + 2 * Ns) * es] = cplx{b0.re - b2.re, b0.im - b2.im};
-        d[(o + 3 * Ns) * es] = cplx{b1.re - b3r.re, b1.im - b3r.im};
-      } else {
-        // generic radix r (3, 5, or a prime factor): direct DFT of size r
-        cplx x[16];
-#pragma unroll
-        for (int t = 0; t < 16; ++t) {
-          if (t < r) {
-            cplx v = s[(j + t * nb) * es];
-            x[t] = t ? cmul(v, tw_get(tw, N, t * k * tstride, fwd)) : v;
-          }
-        }
-        const int rstep = N / r;  // r-th roots from the N-th root table
-#pragma unroll
-        for (int q = 0; q < 16; ++q) {
-          if (q < r) {
-            cplx acc = x[0];
-#pragma unroll
-            for (int t = 1; t < 16; ++t) {
-              if (t < r) {
-                cplx w = tw_get(tw, N, ((q * t) % r) * rstep, fwd);
-                cplx m = cmul(x[t], w);
-                acc.re += m.re;
-                acc.im += m.im;
-              }
-            }
-            d[(o + q * Ns) * es] = acc;
-          }
-        }
-      }
-    }
-    __syncthreads();
-    cplx* t2 = src;
-    src = dst;
-    dst = t2;
-    Ns *= r;
-  }
-  if (src != buf) {
-    for (int b = tid; b < nlines * N; b += T) {
-      int line = b / N, n = b - line * N;
-      buf[line * ls + n * es] = src[line * ls + n * es];
-    }
-    __syncthreads();
-  }
-}
-
-// pass 1: (x,y) pencils. out spec[c][x][y][kz]
-__global__ __launch_bounds__(kBlock) void k_fft_z_fwd(SpecGeom g, const double* __restrict__ F,
-                                                      const double* __restrict__ K4,
-                                                      cplx* __restrict__ spec,
-                                                      const cplx* __restrict__ tw) {
-  if (g.skip && *g.skip) return;
-  extern __shared__ cplx lds[];
-  const int N = g.N, Nz = g.Nz;
-  const long V = g.V;
-  const long line0 = blockIdx.x;  // x*N + y
-  cplx* buf = lds;
-  cplx* tmp = lds + 9 * N;
-  const long e0 = line0 * N;
-  for (int z = threadIdx.x; z < N; z += blockDim.x) {
-    const long e = e0 + z;
-    double f[9];
-#pragma unroll
-    for (int c = 0; c < 9; ++c) f[c] = F[c * V + e];
-    if (K4) {
-      // ddot42n: C_r = t1 + (((t2+t6)+(t4+t8)) + ((t3+t7)+(t5+t9)))
-#pragma unroll
-      for (int r = 0; r < 9; ++r) {
-        double k[9];
-#pragma unroll
-        for (int c = 0; c < 9; ++c) k[c] = K4[(9 * r + c) * V + e];
-        buf[r * N + z] = cplx{ddot42n_row(k, f), 0.0};
-      }
-    } else {
-#pragma unroll
-      for (int r = 0; r < 9; ++r) buf[r * N + z] = cplx{f[r], 0.0};
-    }
-  }
-  __syncthreads();
-  lds_fft(buf, tmp, 9, N, 1, g.plan, tw, 1.0);
-  for (int i = threadIdx.x; i < 9 * Nz; i += blockDim.x) {
-    int c = i / Nz, kz = i - c * Nz;
-    spec[c * g.S1 + line0 * Nz + kz] = buf[c * N + kz];
-  }
-}
-
-// pass 2 / 4: y transforms. grid: (ceil(Nz/ty), N, 9)
-__global__ __launch_bounds__(kBlock) void k_fft_y(SpecGeom g, cplx* __restrict__ spec,
-                                                  const cplx* __restrict__ tw, double fwd) {
-  if (g.skip && *g.skip) return;
-  extern __shared__ cplx lds[];
-  const int N = g.N, Nz = g.Nz, ty = g.ty;
-  const int kz0 = blockIdx.x * ty;
-  const int x = blockIdx.y, c = blockIdx.z;
-  const int nt = min(ty, Nz - kz0);
-  cplx* base = spec + c * g.S1 + (long)x * N * Nz;
-  cplx* buf = lds;
-  cplx* tmp = lds + ty * N;
-  // line t = kz column, element n = y; layout buf[t*N + n]
-  for (int i = threadIdx.x; i < N * nt; i += blockDim.x) {
-    int y = i / nt, t = i - y * nt;
-    buf[t * N + y] = base[(long)y * Nz + kz0 + t];
-  }
-  __syncthreads();
-  lds_fft(buf, tmp, nt, N, 1, g.plan, tw, fwd);
-  for (int i = threadIdx.x; i < N * nt; i += blockDim.x) {
-    int y = i / nt, t = i - y * nt;
-    base[(long)y * Nz + kz0 + t] = buf[t * N + y];
-  }
-}
-
-// pass 3: x transforms + projection. grid: (ceil(Nz/tz), N)
-__global__ __launch_bounds__(kBlock) void k_proj_x(SpecGeom g, cplx* __restrict__ spec,
-                                                   const cplx* __restrict__ tw) {
-  if (g.skip && *g.skip) return;
-  extern __shared__ cplx lds[];
-  const int N = g.N, Nz = g.Nz, tz = g.tz;
-  const int kz0 = blockIdx.x * tz;
-  const int y = blockIdx.y;
-  const int nt = min(tz, Nz - kz0);
-  const int nl = 9 * nt;
-  cplx* buf = lds;
-  cplx* tmp = lds + 9 * tz * N;
-  // line (c*nt + t), element x; layout buf[(c*nt+t)*N + x]
-  for (int i = threadIdx.x; i < 9 * N * nt; i += blockDim.x) {
-    int t = i % nt;
-    int rest = i / nt;
-    int x = rest % N, c = rest / N;
-    buf[(c * nt + t) * N + x] = spec[c * g.S1 + ((long)x * N + y) * Nz + kz0 + t];
-  }
-  __syncthreads();
-  lds_fft(buf, tmp, nl, N, 1, g.plan, tw, 1.0);
-  // projection at every (x, kz) point of the tile
-  for (int i = threadIdx.x; i < N * nt; i += blockDim.x) {
-    int x = i / nt, t = i - x * nt;
-    cplx A[9], out[9];
-#pragma unroll
-    for (int c = 0; c < 9; ++c) A[c] = buf[(c * nt + t) * N + x];
-    project9(N, g.gamma_mode, x, y, kz0 + t, A, out);
-#pragma unroll
-    for (int c = 0; c < 9; ++c) buf[(c * nt + t) * N + x] = out[c];
-  }
-  __syncthreads();
-  lds_fft(buf, tmp, nl, N, 1, g.plan, tw, -1.0);
-  for (int i = threadIdx.x; i < 9 * N * nt; i += blockDim.x) {
-    int t = i % nt;
-    int rest = i / nt;
-    int x = rest % N, c = rest / N;
-    spec[c * g.S1 + ((long)x * N + y) * Nz + kz0 + t] = buf[(c * nt + t) * N + x];
-  }
-}
-
-// pass 5: complex-to-real along z, scale 1/N^3
-__global__ __launch_bounds__(kBlock) void k_fft_z_inv(SpecGeom g, const cplx* __restrict__ spec,
-                                                      double* __restrict__ out,
-                                                      const cplx* __restrict__ tw) {
-  if (g.skip && *g.skip) return;
-  extern __shared__ cplx lds[];
-  const int N = g.N, Nz = g.Nz;
-  const long V = g.V;
-  const long line0 = blockIdx.x;
-  cplx* buf = lds;
-  cplx* tmp = lds + 9 * N;
-  for (int i = threadIdx.x; i < 9 * N; i += blockDim.x) {
-    int c = i / N, z = i - c * N;
-    cplx v;
-    if (z < Nz) {
-      v = spec[c * g.S1 + line0 * Nz + z];
-    } else {
-      cplx w = spec[c * g.S1 + line0 * Nz + (N - z)];
-      v = cplx{w.re, -w.im};
-    }
-    buf[c * N + z] = v;
-  }
-  __syncthreads();
-  lds_fft(buf, tmp, 9, N, 1, g.plan, tw, -1.0);
-  const double sc = 1.0 / (double)V;
-  for (int i = threadIdx.x; i < 9 * N; i += blockDim.x) {
-    int c = i / N, z = i - c * N;
-    out[c * V + line0 * N + z] = buf[c * N + z].re * sc;
-  }
-}
-
-const char* make_spec_geom(int N, int gamma_mode, int lds, SpecGeom& g) {
-  const int maxlds = lds > 65536 ? 65536 : lds;
+// ------------------------------------------------------------- operator
+const char* make_spec_geom(int N, int gamma_mode, SpecGeom& g) {
   g = SpecGeom{};
   g.N = N;
   g.Nz = N / 2 + 1;
   g.V = (long)N * N * N;
   g.S1 = (long)N * N * g.Nz;
-  g.plan = make_plan(N);
   g.gamma_mode = gamma_mode;
-  g.ty = 8;
-  g.tz = 1;
-  while (g.tz < 4 && 2 * 9 * (long)(2 * g.tz) * N * (long)sizeof(cplx) <= maxlds) g.tz *= 2;
-  if (!gkdf_pencil_supported(N)) {  // limits of the generic runtime-plan path
-    if (2 * 9 * (long)N * (long)sizeof(cplx) > maxlds)
-      return "grid edge too large for the LDS of this device";
-    for (int s = 0; s < g.plan.nst; ++s)
-      if (g.plan.rad[s] > 16) return "N has a prime factor above 16";
+  if (gkdf_grid_edge(N)) {
+    if (N > 227) return "grid edge too large for the LDS of this device";
+    int m = N;
+    for (int p : {2, 3, 5, 7, 11})
+      while (m % p == 0) m /= p;
+    if (m > 13) return "N has a prime factor above 16";
   }
   return nullptr;
 }
 
 void launch_gkdf(const SpecGeom& g, const double* F, const double* K4, double* out, cplx* spec,
                  const cplx* tw, hipStream_t s) {
-  if (launch_gkdf_pencil(g, F, K4, out, spec, tw, s)) return;
-  const int N = g.N;
-  size_t lz = 2 * 9 * (size_t)N * sizeof(cplx);
-  k_fft_z_fwd<<<dim3((unsigned)((long)N * N)), kBlock, lz, s>>>(g, F, K4, spec, tw);
-  size_t ly = 2 * (size_t)g.ty * N * sizeof(cplx);
-  dim3 gy((g.Nz + g.ty - 1) / g.ty, N, 9);
-  k_fft_y<<<gy, kBlock, ly, s>>>(g, spec, tw, 1.0);
-  size_t lx = 2 * 9 * (size_t)g.tz * N * sizeof(cplx);
-  dim3 gx((g.Nz + g.tz - 1) / g.tz, N);
-  k_proj_x<<<gx, kBlock, lx, s>>>(g, spec, tw);
-  k_fft_y<<<gy, kBlock, ly, s>>>(g, spec, tw, -1.0);
-  k_fft_z_inv<<<dim3((unsigned)((long)N * N)), kBlock, lz, s>>>(g, spec, out, tw);
+  if (gkdf_grid_edge(g.N))
+    launch_gkdf_grid(g, F, K4, out, spec, tw, s);
+  else
+    launch_gkdf_pencil(g, F, K4, out, spec, tw, s);
 }
 
 // ------------------------------------------------------------ reductions
@@ -363,28 +106,32 @@ void launch_mean9(const double* x, long V, double* partials, double* d_out, hipS
   k_scale9<<<1, 64, 0, s>>>(d_out, 1.0 / (double)V);
 }
 
-// tangent_homo: out[j] = sum over (m,e) of K4[9j+m][e] C[m][e]
-__global__ __launch_bounds__(kBlock) void k_k4dot9_part(const double* __restrict__ K4,
-                                                        const double* __restrict__ C, long V,
-                                                        double* __restrict__ part) {
+// tangent_homo's end: means of the 81 rows of K4, kMeanBlocks partial sums
+// a row, then one wave a row
+static constexpr int kMeanBlocks = 64;
+__global__ __launch_bounds__(kBlock) void k_sum81_part(const double* __restrict__ K4, long V,
+                                                       double* __restrict__ part) {
   __shared__ double sh[kBlock];
-  long n = 9 * V;
-  long chunk = (n + gridDim.x - 1) / gridDim.x;
-  long a = blockIdx.x * chunk, b = min(n, a + chunk);
-  for (int j = 0; j < 9; ++j) {
-    const double* Kj = K4 + (long)9 * j * V;
-    double acc = 0.0;
-    for (long i = a + threadIdx.x; i < b; i += blockDim.x) acc += Kj[i] * C[i];
-    double s = block_sum(acc, sh);
-    if (threadIdx.x == 0) part[j * gridDim.x + blockIdx.x] = s;
-  }
+  const double* x = K4 + blockIdx.y * V;
+  const long chunk = (V + gridDim.x - 1) / gridDim.x;
+  const long a = blockIdx.x * chunk, b = min(V, a + chunk);
+  double acc = 0.0;
+  for (long i = a + threadIdx.x; i < b; i += kBlock) acc += __builtin_nontemporal_load(x + i);
+  const double s = tree_sum0<kBlock>(acc, sh);
+  if (threadIdx.x == 0) part[blockIdx.y * kMeanBlocks + blockIdx.x] = s;
 }
-
-void launch_k4_dot9(long V, const double* K4, const double* C, double* partials, double* d_out,
-                    hipStream_t s) {
-  k_k4dot9_part<<<kRedBlocks, kBlock, 0, s>>>(K4, C, V, partials);
-  k_sum_parts<<<1, kBlock, 0, s>>>(partials, kRedBlocks, 9, d_out);
-  k_scale9<<<1, 64, 0, s>>>(d_out, 1.0 / (double)V);
+__global__ __launch_bounds__(64) void k_mean81(const double* __restrict__ part, double sc,
+                                               const double* __restrict__ m,
+                                               double* __restrict__ out) {
+  const int row = blockIdx.x, j = row / 9, i = row - 9 * j;
+  const double s = tree_sum0<64>(part[row * kMeanBlocks + threadIdx.x], nullptr);
+  if (threadIdx.x == 0) out[row] = s * sc + m[9 * i + j];
+}
+void launch_mean81(const double* K4, long V, const double* m, double* partials, double* out,
+                   hipStream_t s) {
+  static_assert(81 * kMeanBlocks <= 9 * kRedBlocks, "partial sums buffer");
+  k_sum81_part<<<dim3(kMeanBlocks, 81), kBlock, 0, s>>>(K4, V, partials);
+  k_mean81<<<81, 64, 0, s>>>(partials, 1.0 / (double)V, m, out);
 }
 
 // --------------------------------------------------------------- BLAS-1
@@ -421,38 +168,12 @@ __global__ void k_state_init(long V, int W, double tt0, double* __restrict__ st)
     st[i] = v;
   }
 }
-__global__ void k_add1(long V, double* __restrict__ x) {
-  for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < V; i += (long)gridDim.x * blockDim.x)
-    x[i] = x[i] + 1.0;
-}
 __global__ void k_gather_col(long V, int col, const double* __restrict__ K4, double* __restrict__ C) {
   for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < 9 * V; i += (long)gridDim.x * blockDim.x) {
     long j = i / V, e = i - j * V;
     C[i] = K4[(9 * j + col) * V + e];
   }
 }
-__global__ __launch_bounds__(kBlock) void k_cg_update(long n, double a, const double* __restrict__ p,
-                                                      const double* __restrict__ q,
-                                                      double* __restrict__ x, double* __restrict__ r,
-                                                      double* __restrict__ part) {
-  __shared__ double sh[kBlock];
-  long chunk = (n + gridDim.x - 1) / gridDim.x;
-  long lo = blockIdx.x * chunk, hi = min(n, lo + chunk);
-  double acc = 0.0;
-  for (long i = lo + threadIdx.x; i < hi; i += blockDim.x) {
-    x[i] = x[i] + a * p[i];
-    double ri = r[i] - a * q[i];
-    r[i] = ri;
-    acc += ri * ri;
-  }
-  double s = block_sum(acc, sh);
-  if (threadIdx.x == 0) part[blockIdx.x] = s;
-}
-__global__ void k_cg_dir(long n, double b, const double* __restrict__ r, double* __restrict__ p) {
-  for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x)
-    p[i] = r[i] + b * p[i];
-}
-
 static inline unsigned grid_for(long n) {
   long g = (n + kBlock - 1) / kBlock;
   return (unsigned)(g > 8192 ? 8192 : (g < 1 ? 1 : g));
@@ -485,34 +206,63 @@ void launch_fill_f32(long n, float v, float* x, hipStream_t s) {
 void launch_state_init(long V, int W, double tt0, double* state, hipStream_t s) {
   k_state_init<<<grid_for((long)W * V), kBlock, 0, s>>>(V, W, tt0, state);
 }
-void launch_add_identity_comp(long V, int comp, double* x, hipStream_t s) {
-  k_add1<<<grid_for(V), kBlock, 0, s>>>(V, x + (long)comp * V);
-}
 void launch_gather_k4_col(long V, int i, const double* K4, double* C, hipStream_t s) {
   k_gather_col<<<grid_for(9 * V), kBlock, 0, s>>>(V, i, K4, C);
 }
-void launch_cg_update(long n, double a, const double* p, const double* q, double* x, double* r,
-                      double* partials, double* d_out, hipStream_t s) {
-  k_cg_update<<<kRedBlocks, kBlock, 0, s>>>(n, a, p, q, x, r, partials);
-  k_sum_parts<<<1, kBlock, 0, s>>>(partials, kRedBlocks, 1, d_out);
-}
-void launch_cg_dir(long n, double b, const double* r, double* p, hipStream_t s) {
-  k_cg_dir<<<grid_for(n), kBlock, 0, s>>>(n, b, r, p);
-}
-
 // ------------------------------------------------- device-scalar CG
-__global__ __launch_bounds__(kBlock) void k_dot_part_s(const double* __restrict__ x,
-                                                       const double* __restrict__ y, long n,
-                                                       double* __restrict__ part,
-                                                       const CGScalars* __restrict__ cs) {
-  if (cs->done) return;
+// Start of a solve: x = 0, r = b (and p = b), partial sums of b.b over the
+// contiguous ranges of k_dot_part
+template <bool P>
+__global__ __launch_bounds__(kBlock) void k_cg_start(long n, const double* __restrict__ b,
+                                                     double* __restrict__ x,
+                                                     double* __restrict__ r,
+                                                     double* __restrict__ p,
+                                                     double* __restrict__ part) {
   __shared__ double sh[kBlock];
-  long chunk = (n + gridDim.x - 1) / gridDim.x;
-  long a = blockIdx.x * chunk, b = min(n, a + chunk);
+  const long chunk = (n + gridDim.x - 1) / gridDim.x;
+  const long lo = blockIdx.x * chunk, hi = min(n, lo + chunk);
   double acc = 0.0;
-  for (long i = a + threadIdx.x; i < b; i += blockDim.x) acc += x[i] * y[i];
-  double s = block_sum(acc, sh);
+  for (long i = lo + threadIdx.x; i < hi; i += kBlock) {
+    const double v = b[i];
+    x[i] = 0.0;
+    r[i] = v;
+    if constexpr (P) p[i] = v;
+    acc += v * v;
+  }
+  const double s = block_sum(acc, sh);
   if (threadIdx.x == 0) part[blockIdx.x] = s;
+}
+// block b: system b
+__global__ __launch_bounds__(kBlock) void k_cg_init(const double* __restrict__ part, int np,
+                                                    double tol, int maxit, int zero_code,
+                                                    CGScalars* __restrict__ cs,
+                                                    double* __restrict__ m) {
+  __shared__ double sh[kBlock];
+  const double bb = ordered_sum<kBlock>(part + (long)blockIdx.x * np, np, sh);
+  if (m && threadIdx.x < 9) m[9 * blockIdx.x + threadIdx.x] = 0.0;
+  if (threadIdx.x == 0) {
+    CGScalars c{};
+    c.rr = bb;
+    c.n2b = sqrt(bb);
+    c.tolb = tol * c.n2b;
+    c.tol = tol;
+    c.resnorm = c.n2b;
+    c.maxit = maxit;
+    c.done = c.n2b <= 2.220446049250313e-16 ? zero_code : 0;
+    cs[blockIdx.x] = c;
+  }
+}
+void launch_cg_start(long n, const double* b, double* x, double* r, double* p, double* partials,
+                     hipStream_t s) {
+  if (p)
+    k_cg_start<true><<<kRedBlocks, kBlock, 0, s>>>(n, b, x, r, p, partials);
+  else
+    k_cg_start<false><<<kRedBlocks, kBlock, 0, s>>>(n, b, x, r, p, partials);
+}
+int cg_start_parts() { return kRedBlocks; }
+void launch_cg_init(const double* part, int np, double tol, int maxit, int zero_code,
+                    CGScalars* cs, double* m, int nsys, hipStream_t s) {
+  k_cg_init<<<nsys, kBlock, 0, s>>>(part, np, tol, maxit, zero_code, cs, m);
 }
 // alpha = rr / (p.q) from the partial sums (same order as k_sum_parts)
 // block b serves system b: partial sums part + b pstride, scalars cs + b
@@ -591,14 +341,6 @@ __global__ __launch_bounds__(kBlock) void k_cg_check(const double* __restrict__ 
     cg_check(cs, rr1);
   }
 }
-__global__ void k_cg_dir_s(long n, const CGScalars* __restrict__ cs, const double* __restrict__ r,
-                           double* __restrict__ p) {
-  if (cs->done) return;
-  const double b = cs->beta;
-  for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x)
-    p[i] = r[i] + b * p[i];
-}
-
 void launch_cg_update_check(long n, CGScalars* cs, const double* p, const double* q, double* x,
                             double* r, double* partials, hipStream_t s, bool xupd,
                             const double* dc, double* m, double scale) {
@@ -615,17 +357,6 @@ void launch_cg_alpha(const double* part, int np, CGScalars* cs, hipStream_t s, i
 void launch_cg_check(const double* part, int np, CGScalars* cs, hipStream_t s, const double* dc,
                      double* m, double scale, int nsys, long pstride) {
   k_cg_check<<<nsys, kBlock, 0, s>>>(part, np, cs, dc, m, scale, pstride);
-}
-
-void launch_cg_tail(long n, CGScalars* cs, const double* p, const double* q, double* x,
-                    double* r, double* partials, hipStream_t s) {
-  k_dot_part_s<<<kRedBlocks, kBlock, 0, s>>>(p, q, n, partials, cs);
-  k_cg_alpha<<<1, kBlock, 0, s>>>(partials, kRedBlocks, cs, 0);
-  k_cg_update_s<true><<<kRedBlocks, kBlock, 0, s>>>(n, cs, p, q, x, r, partials);
-  k_cg_check<<<1, kBlock, 0, s>>>(partials, kRedBlocks, cs, nullptr, nullptr, 0.0, 0);
-}
-void launch_cg_dir_dev(long n, const CGScalars* cs, const double* r, double* p, hipStream_t s) {
-  k_cg_dir_s<<<grid_for(n), kBlock, 0, s>>>(n, cs, r, p);
 }
 
 // ------------------------------------------ multi-RHS K4 contraction
@@ -670,7 +401,8 @@ __global__ __launch_bounds__(kBlock) void k_k4_contract_multi(long V, const doub
       double* pw = const_cast<double*>(pp.p[i]);
 #pragma unroll
       for (int c = 0; c < 9; ++c) {
-        f[c] = rb[i & 1][c] + beta * pb[i & 1][c];
+        // (the first direction is r, whatever p holds)
+        f[c] = beta == 0.0 ? rb[i & 1][c] : rb[i & 1][c] + beta * pb[i & 1][c];
         if (valid) __builtin_nontemporal_store(f[c], pw + c * V + e);
       }
     } else {

@@ -69,9 +69,8 @@ extern "C" int cpfft_gkdf_noalloc(int N, int gamma_mode, const double* F, const 
   if (!F || !GKF) return nfail(-1, "null field pointer");
   if (F == GKF) return nfail(-1, "F and GKF must not alias");
   SpecGeom g;
-  // the geometry of a context (cpfft_create clamps the LDS per block to
-  // 64 KiB), so the results are bit-identical to cpfft_gkdf's
-  if (const char* why = make_spec_geom(N, gamma_mode, 65536, g)) return nfail(-3, why);
+  // a context's geometry and kernels, so the results are cpfft_gkdf's
+  if (const char* why = make_spec_geom(N, gamma_mode, g)) return nfail(-3, why);
   if (2 * 9 * g.S1 > kSpecMax) return nfail(-1, "spectrum exceeds the scratch array");
   cplx* sp = nullptr;
   if (int rc = noalloc_scratch_current_device(&sp)) return rc;

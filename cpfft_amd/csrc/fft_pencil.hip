@@ -1,5 +1,6 @@
 // fft_pencil.hip -- G_K_dF (src/G_K_dF.f:11-87) for grid edges with a
-// compile-time radix plan (16, 32, 48, 64, 96, 128, 256).
+// compile-time radix plan and large planes (64, 96, 128, 256; fft_grid.hip
+// serves the others).
 //
 // Five passes over two half-spectrum buffers in HBM, each pass reading and
 // writing contiguous runs (whole lines or >= 64-byte tiles):
@@ -800,7 +801,6 @@ constexpr int dot_parts() { return (N / tile_z(N)) * N * 9; }
 
 bool gkdf_pencil_supported(int N) {
   switch (N) {
-    case 16: case 32: case 48: case 64: case 96: case 128: case 256: return true;
     default: return false;
   }
 }
@@ -810,9 +810,6 @@ bool launch_gkdf_pencil(const SpecGeom& g, const double* F, const double* K4, do
   cplx* T1 = spec;
   cplx* T2 = spec + 9 * g.S1;
   switch (g.N) {
-    case 16: fp::launch<16>(g, F, K4, out, T1, T2, tw, s, fuse); return true;
-    case 32: fp::launch<32>(g, F, K4, out, T1, T2, tw, s, fuse); return true;
-    case 48: fp::launch<48>(g, F, K4, out, T1, T2, tw, s, fuse); return true;
     case 64: fp::launch<64>(g, F, K4, out, T1, T2, tw, s, fuse); return true;
     case 96: fp::launch<96>(g, F, K4, out, T1, T2, tw, s, fuse); return true;
     case 128: fp::launch<128>(g, F, K4, out, T1, T2, tw, s, fuse); return true;
@@ -824,9 +821,6 @@ bool launch_gkdf_pencil(const SpecGeom& g, const double* F, const double* K4, do
 int pencil_candidate(int N, int pass, int variant) {
   if (pass < 0 || pass > 3 || variant < 0 || variant >= kPencilCands) return 0;
   switch (N) {
-    case 16: return fp::cand<16>(pass, variant);
-    case 32: return fp::cand<32>(pass, variant);
-    case 48: return fp::cand<48>(pass, variant);
     case 64: return fp::cand<64>(pass, variant);
     case 96: return fp::cand<96>(pass, variant);
     case 128: return fp::cand<128>(pass, variant);
@@ -841,9 +835,6 @@ bool launch_pencil_pass(const SpecGeom& g, int pass, int variant, const double* 
   cplx* T1 = spec;
   cplx* T2 = spec + 9 * g.S1;
   switch (g.N) {
-    case 16: fp::launch_pass<16>(g, pass, variant, F, K4, T1, T2, tw, s); return true;
-    case 32: fp::launch_pass<32>(g, pass, variant, F, K4, T1, T2, tw, s); return true;
-    case 48: fp::launch_pass<48>(g, pass, variant, F, K4, T1, T2, tw, s); return true;
     case 64: fp::launch_pass<64>(g, pass, variant, F, K4, T1, T2, tw, s); return true;
     case 96: fp::launch_pass<96>(g, pass, variant, F, K4, T1, T2, tw, s); return true;
     case 128: fp::launch_pass<128>(g, pass, variant, F, K4, T1, T2, tw, s); return true;
@@ -854,9 +845,6 @@ bool launch_pencil_pass(const SpecGeom& g, int pass, int variant, const double* 
 
 int gkdf_dot_parts(int N) {
   switch (N) {
-    case 16: return fp::dot_parts<16>();
-    case 32: return fp::dot_parts<32>();
-    case 48: return fp::dot_parts<48>();
     case 64: return fp::dot_parts<64>();
     case 96: return fp::dot_parts<96>();
     case 128: return fp::dot_parts<128>();

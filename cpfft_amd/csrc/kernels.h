@@ -12,10 +12,11 @@
 
 namespace cpfft {
 
-// Launch shapes of the compile-time-planned FFT path chosen by the
-// autotuner, as candidate indices (0 = the default shape): a, a0 pass A
-// with / without K4, b the y passes, c pass C.  All candidates compute
-// bit-identical results.
+// Launch shapes chosen by the autotuner, as candidate indices (0 = the
+// default shape).  fft_pencil.hip: a, a0 pass A with / without K4, b the y
+// passes, c pass C.  fft_grid.hip (16, 32, 48): a, a0 k_fwd with / without
+// K4, b k_inv (where they form no CG sum), c k_mid.  All
+// candidates compute bit-identical results.
 struct PencilTune {
   int a = 0, a0 = 0, b = 0, c = 0;
 };
@@ -25,20 +26,14 @@ struct SpecGeom {
   int N, Nz;        // grid edge, number of z frequencies kept (N/2+1)
   long V;           // N^3
   long S1;          // complex entries per spectral component: N*N*Nz
-  FftPlan plan;     // radix plan for length N
   int gamma_mode;   // 0 reference operator, 1 textbook projection
-  int ty;           // kz columns per block in the y pass
-  int tz;           // kz columns per block in the x pass
-  const int* skip;  // if non-null and *skip != 0, every block returns at once
-  PencilTune tune;  // launch shapes of the planned path
+  const int* skip;  // fft_pencil.hip: if non-null and *skip != 0, every block returns at once
+  PencilTune tune;  // launch shapes
 };
 
-// Geometry of the operator for edge N and Gamma variant gamma_mode: the
-// spectrum sizes, the radix plan and the generic path's tiles, sized for
-// min(lds, 64 KiB) bytes of shared memory per block (the same tiles on
-// every device, so results do not depend on the device).  Returns nullptr,
-// or why N cannot be served.
-const char* make_spec_geom(int N, int gamma_mode, int lds, SpecGeom& g);
+// Geometry of the operator for edge N and Gamma variant gamma_mode.  Returns
+// nullptr, or why N cannot be served.
+const char* make_spec_geom(int N, int gamma_mode, SpecGeom& g);
 
 // Displacement reconstruction (f2disp.hip): the cosine table (of
 // f2disp_cos_doubles(N) doubles) once, then u (device, [3 (N+1)^3]
@@ -51,9 +46,9 @@ void launch_f2disp(int N, const double* F, const double len[3], const double* C,
                    double* u, hipStream_t s);
 
 // Gamma:(K4:F) or Gamma:F (K4 == nullptr).  spec: 2*9*S1 complex scratch.
-// tw: the N twiddles exp(-2 pi i k/N).  Uses the compile-time-planned path
-// of fft_pencil.hip where it exists for N, else the generic runtime plan.
-// CG work fused into the operator's passes (compile-time-planned path only):
+// tw: the N twiddles exp(-2 pi i k/N).  fft_pencil.hip for N = 64, 96, 128,
+// 256, fft_grid.hip for every other edge.
+// CG work fused into the operator's passes (fft_pencil.hip):
 // dir_p != nullptr: pass A first sets dir_p = dir_r + cs->beta * dir_p (the
 //   CG direction, F must be dir_p) and transforms the new direction;
 // dot_p != nullptr: pass D writes per-block partial sums of dot_p . out
@@ -88,6 +83,53 @@ struct CGFuse {
 
 void launch_gkdf(const SpecGeom& g, const double* F, const double* K4, double* out, cplx* spec,
                  const cplx* tw, hipStream_t s);
+// ---- fft_grid.hip
+// whether edge N is served there; whether by the slab kernels, which serve
+// launch_cg_grid with q and launch_homo_rhs_grid for N = 64 and 96 too
+bool gkdf_grid_edge(int N);
+bool gkdf_slab_edge(int N);
+void launch_gkdf_grid(const SpecGeom& g, const double* F, const double* K4, double* out,
+                      cplx* spec, const cplx* tw, hipStream_t s);
+// One CG iteration of nrhs systems (at most nine) that share K4.
+// part 0: the forward pass (with chk first the convergence test of the
+//   previous iteration, as launch_cg_check does it; p_new = r + beta p_old;
+//   K4:p_new and its product with p_new) and the passes up to the projected
+//   spectrum, alpha among them;
+// part 1: the inverse pass: r -= alpha q, where x[i] != nullptr also
+//   x += alpha p_new, and the r.r partial sums.
+// out[0] != nullptr instead (the reference's operator): part 0 forms no
+//   alpha; part 1 stores q in out, takes p.q from it and updates r and x.
+// cs_old is the state before the iteration, cs_new the one after chk; they
+// may be the same array when !chk.  p_old and p_new are different fields.
+struct GridCG {
+  int nrhs;
+  double *p_old[9], *p_new[9], *r[9], *x[9], *out[9];
+  const double* q[9];  // q[0] != nullptr: K4:p_new, formed by the caller (part 0 then neither
+  int npq;             // tests nor forms the direction) with npq values of pq per system
+  const double* K4;
+  cplx* spec;  // nrhs * grid_spec_len entries
+  const cplx* tw;
+  CGScalars *cs_old, *cs_new;
+  int chk;
+  double *pq, *rr;  // partial sums: nrhs * grid_parts(N), nrhs * grid_rr_parts(N, out[0] == nullptr)
+  double *dc, *m;   // as launch_cg_check, nine values per system (or nullptr)
+  double scale;
+};
+void launch_cg_grid(const SpecGeom& g, const GridCG& c, int part, hipStream_t s);
+// r[i] = -G(K4:E_i) for the unit tensors E_i, i0 <= i < i0 + n, with the r.r
+// partial sums in rr (tangent_homo's right-hand sides)
+void launch_homo_rhs_grid(const SpecGeom& g, const double* K4, int i0, int n, double* const* r,
+                          cplx* spec, const cplx* tw, double* rr, hipStream_t s);
+int grid_parts(int N);
+int grid_rr_parts(int N, bool projection);
+bool grid_fused_check(int N);  // whether chk may be used at this edge
+long grid_spec_len(const SpecGeom& g);
+// autotuner support for N = 16, 32, 48 (see pencil_candidate)
+int grid_candidate(int N, int pass, int v);
+void launch_grid_pass(const SpecGeom& g, int pass, int v, const double* F, const double* K4,
+                      cplx* spec, const cplx* tw, hipStream_t s);
+
+// ---- fft_pencil.hip
 bool gkdf_pencil_supported(int N);
 // returns false (and launches nothing) when N has no compile-time plan
 bool launch_gkdf_pencil(const SpecGeom& g, const double* F, const double* K4, double* out,
@@ -120,13 +162,20 @@ void launch_cg_update_check(long n, CGScalars* cs, const double* p, const double
                             const double* dc = nullptr, double* m = nullptr,
                             double scale = 0.0);
 
-// One CG iteration after q = A p: alpha = rr / (p.q); x += alpha p;
-// r -= alpha q; convergence test on |r|; p = r + beta p.  All scalars stay
-// in *cs; nothing happens once cs->done is set.
-void launch_cg_tail(long n, CGScalars* cs, const double* p, const double* q, double* x,
-                    double* r, double* partials, hipStream_t s);
-// p = r + beta p with beta from *cs (skipped once cs->done is set)
-void launch_cg_dir_dev(long n, const CGScalars* cs, const double* r, double* p, hipStream_t s);
+// x = 0, r = b, with p != nullptr also p = b, and the partial sums of b.b
+// (start of a CG solve); then launch_cg_init with np = cg_start_parts()
+void launch_cg_start(long n, const double* b, double* x, double* r, double* p, double* partials,
+                     hipStream_t s);
+int cg_start_parts();
+// state of nsys solves about to start, from the partial sums of b.b (np per
+// system): done = zero_code where |b| vanishes (FFT_nr3.f:254-262); with
+// m != nullptr its nine values per system are cleared
+void launch_cg_init(const double* part, int np, double tol, int maxit, int zero_code,
+                    CGScalars* cs, double* m, int nsys, hipStream_t s);
+// out[9 j + i] = mean of row 9 j + i of K4 + m[9 i + j] (tangent_homo's end:
+// the mean of K4:(E_i + x_i))
+void launch_mean81(const double* K4, long V, const double* m, double* partials, double* out,
+                   hipStream_t s);
 
 // up to nine field pointers (multi-RHS solves)
 struct Ptr9 {
@@ -139,7 +188,7 @@ struct Ptr9r {
   const double* r[9];
 };
 // pqpart != nullptr: also p_i . (K4:p_i) of each running right-hand side,
-// per block, at pqpart[i * k4_contract_multi_blocks(V) + block]
+// per block, at pqpart[i * k4_contract_multi_blocks(V) + block].
 void launch_k4_contract_multi(long V, const double* K4, const Ptr9& pp, const CGScalars* cs,
                               int nrhs, hipStream_t s, const Ptr9r* rr = nullptr,
                               double* pqpart = nullptr);
@@ -159,17 +208,8 @@ void launch_fill_f32(long n, float v, float* x, hipStream_t s);
 // initial material state [W][V] (mm10_init_cc_hist0, mm10_a.f:473-573, with
 // mm10_init_voche, :2042-2055): zero, except Rp = I and tau_tilde = tt0
 void launch_state_init(long V, int W, double tt0, double* state, hipStream_t s);
-void launch_add_identity_comp(long V, int comp, double* x, hipStream_t s);
-// CG vector update: x += a p; r -= a q; partial r.r into partials
-void launch_cg_update(long n, double a, const double* p, const double* q, double* x, double* r,
-                      double* partials, double* d_out, hipStream_t s);
-// p = r + b p
-void launch_cg_dir(long n, double b, const double* r, double* p, hipStream_t s);
 // C[j] = K4[(9 j + i) rows] copy (tangent_homo column i)
 void launch_gather_k4_col(long V, int i, const double* K4, double* C, hipStream_t s);
-// out[j] = sum_e sum_m K4[9j+m][e] * C[m][e] for j=0..8 (tangent_homo.f:62-66)
-void launch_k4_dot9(long V, const double* K4, const double* C, double* partials, double* d_out,
-                    hipStream_t s);
 
 // per-voxel update: stress update (state n+1, P, material tangent into
 // tan6 [36][V]) followed by its pull-back to K4 = dP/dF

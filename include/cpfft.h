@@ -210,10 +210,10 @@ int cpfft_set_graphs(cpfft_ctx* ctx, int on);
  * (FFT_nr3.f:335-339).  -1 for a limit below 1.                           */
 int cpfft_set_cg_maxit(cpfft_ctx* ctx, int maxit);
 
-/* Autotuner of the compile-time-planned FFT path (N in 16, 32, 48, 64, 96,
- * 128, 256): times the candidate launch shapes of each of pass A with K4,
- * pass A without K4, the y passes and pass C on this context's buffers
- * (reps launches each) and keeps the fastest.  The choice is cached per
+/* Autotuner of the compile-time-planned FFT paths (N in 16, 32, 48, 64, 96,
+ * 128, 256): times the candidate launch shapes of each of the forward pass
+ * with K4, without K4, the y passes (N <= 48: the inverse pass) and the x
+ * pass on this context's buffers (reps launches each) and keeps the fastest.  The choice is cached per
  * device and N for every context of the process (force != 0 measures
  * again).  Only shapes that compute bit-identical results are candidates
  * (which block transforms which lines; never the radix order or a
@@ -224,7 +224,10 @@ int cpfft_autotune(cpfft_ctx* ctx, int reps, int force);
  * without K4, out[2] lines per block of the y passes, out[3] component
  * lines per block of pass C: 24, 12 or 6 (one tensor row of 8, 4 or 2 y
  * lines, transforms in registers) for N = 64, 128, 256, else 18 or 9 (all
- * nine components of 2 or 1 y lines); 0 where N has no planned path      */
+ * nine components of 2 or 1 y lines).  N = 16, 32, 48: wavefronts per block
+ * of the forward pass with K4, without K4, the inverse pass and the x pass
+ * (the first and third of plain G_K_dF applications; solves take the
+ * default there).  0 where N has no planned path                          */
 int cpfft_get_tune(cpfft_ctx* ctx, int out[4]);
 /* set them (each must be one of the candidates; -1 otherwise)             */
 int cpfft_set_tune(cpfft_ctx* ctx, const int in[4]);
@@ -237,7 +240,7 @@ int cpfft_set_tune(cpfft_ctx* ctx, const int in[4]);
 int cpfft_counters(cpfft_ctx* ctx, long long out[8]);
 /* device-time measurement with HIP events recorded on the context's stream
  * (no host synchronisation while recording).  out[0..3]: average ms per
- * launch group since cpfft_set_timing of [0] G_K_dF with K4 (five kernels),
+ * launch group since cpfft_set_timing of [0] G_K_dF with K4,
  * [1] drive_eps_sig, [2] CG vector update, [3] G_K_dF without K4;
  * out[4..7]: number of launch groups measured.
  * cpfft_set_timing(ctx, k): 0 off; k > 0 records every k-th launch group
