@@ -5,6 +5,8 @@
 //    block reductions (fixed order, no floating-point atomics).
 //  * drive_eps_sig (src/drive_eps_sig.f:16-339): one thread per voxel,
 //    body in mm10_core.h.
+#include <type_traits>
+
 #include "../../include/cpfft.h"
 #include "green.h"
 #include "kernels.h"
@@ -443,11 +445,21 @@ void launch_k4_contract_multi(long V, const double* K4, const Ptr9& pp, const CG
 }
 
 // ------------------------------------------------------- stress update
-template <int NS>
-__global__ __launch_bounds__(64) void k_drive_eps_sig(long V, MatParams P,
+// One thread per voxel, one wave per block.  Bound by FP64 issue and the
+// latency of a single wave per SIMD: the Newton iteration's 7x7 system and
+// the slip sums take 512 registers a lane (two waves would spill more than a
+// kilobyte a lane and run 1.7 times as long).  So what is not needed is left
+// out of each instantiation: EXPL the explicit update of iteration 0, WARM
+// the warm-start candidates, MatParamsInt the calls to pow; scratch falls from 640
+// to 148 bytes a lane.  At 128^3, about five local iterations a voxel: 3.31 ms
+// for fcc (61% of the cycles issue) against 5.83 with the stages of the local
+// solve, their line searches and the general parameters inlined one after
+// another and slip systems taken one at a time (45%).
+template <int NS, bool EXPL, bool WARM, class MP>
+__global__ __launch_bounds__(64) void k_drive_eps_sig(long V, MP P,
                                                       const Orient<NS>* __restrict__ orients,
                                                       const int32_t* __restrict__ oid, int step,
-                                                      int iter, const double* __restrict__ Fn,
+                                                      const double* __restrict__ Fn,
                                                       const double* __restrict__ Fn1,
                                                       const double* __restrict__ sn,
                                                       double* __restrict__ snp1,
@@ -463,13 +475,13 @@ __global__ __launch_bounds__(64) void k_drive_eps_sig(long V, MatParams P,
     // this step's previous global iterate (stress, slip resistance), read
     // before the update overwrites it
     double xp[7];
-    if (warm_prev) {
+    if (WARM && warm_prev) {
 #pragma unroll
       for (int k = 0; k < 6; ++k) xp[k] = snp1[k * V + e];
       xp[6] = snp1[15 * V + e];
     }
-    voxel_update<NS>(
-        P, o, step, iter,
+    voxel_update<NS, EXPL, WARM>(
+        P, o, step,
         [&](int which, int c) { return which ? Fn1[c * V + e] : Fn[c * V + e]; },
         [&](int w) { return sn[w * V + e]; },
         [&](int w, double v) { snp1[w * V + e] = v; },
@@ -516,8 +528,22 @@ void launch_drive_eps_sig(long V, const MatParams& P, const Orient<NS>* orients,
                           long long* counters, hipStream_t s) {
   const int bs = 64;
   unsigned g = (unsigned)((V + bs - 1) / bs);
-  k_drive_eps_sig<NS><<<g, bs, 0, s>>>(V, P, orients, orient_id, step, iter, Fn, Fn1, sn, snp1,
-                                       Pn1, tan6, ws, warm_prev, counters);
+  auto update = [&](auto expl, auto warm, auto params) {
+    k_drive_eps_sig<NS, decltype(expl)::value, decltype(warm)::value><<<g, bs, 0, s>>>(
+        V, params, orients, orient_id, step, Fn, Fn1, sn, snp1, Pn1, tan6, ws, warm_prev, counters);
+  };
+  const std::true_type yes;
+  const std::false_type no;
+  // the narrowest instantiation that covers the call
+  const bool simple = P.int_rate && P.m_is_one, warm = ws || warm_prev;
+  if (iter == 0)
+    update(yes, no, P);
+  else if (simple && !warm)
+    update(no, no, MatParamsInt{P});
+  else if (simple)
+    update(no, yes, MatParamsInt{P});
+  else
+    update(no, yes, P);
   k_cep2A<<<g, bs, 0, s>>>(V, Fn, Fn1, snp1, tan6, K4);
 }
 

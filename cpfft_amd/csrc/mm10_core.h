@@ -37,11 +37,21 @@ struct MatParams {
   int m_is_one;                                // voche_m == 1
 };
 
+// Parameters with an integral rate exponent and voche_m == 1 known at compile
+// time, as most materials have: without the calls to pow on the other
+// branches the update needs fewer registers and half the code.
+struct MatParamsInt : MatParams {};
+CPFFT_HD inline bool rate_is_int(const MatParams& p) { return p.int_rate != 0; }
+CPFFT_HD inline constexpr bool rate_is_int(const MatParamsInt&) { return true; }
+CPFFT_HD inline bool m_is_one(const MatParams& p) { return p.m_is_one != 0; }
+CPFFT_HD inline constexpr bool m_is_one(const MatParamsInt&) { return true; }
+
 // per-orientation invariants (setup_mm10_rknstr, drive_eps_sig.f:537-1002):
 // rotated stiffness C (row-major 6x6), ms (Voigt 6, eng. shear), qs (skew 3)
 template <int NS>
 struct Orient {
   double C[36];
+  double S[36];  // C^-1
   double ms[NS][6];
   double qs[NS][3];
 };
@@ -69,13 +79,24 @@ CPFFT_HD inline double pw_nm2(const MatParams& p, double au) {
   return p.int_rate ? ipow(au, (int)p.rate_n - 2) : pow(au, p.rate_n - 2.0);
 }
 
+// whether c holds in any active lane of the wavefront (host build: in this one)
+CPFFT_HD inline bool any_lane(bool c) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  return __any(c);
+#else
+  return c;
+#endif
+}
+
 // Gaussian elimination with partial pivoting on [A | B] followed by back
 // substitution, N <= 7, row-major A (destroyed).  Every index is static
 // once the loops are unrolled (the row exchange of each step is done with
-// selects), so A and B stay in registers.  The arithmetic is that of an LU
-// factorisation followed by forward and back substitution.
+// selects, and skipped where no lane of the wavefront exchanges), so A and B
+// stay in registers.  The arithmetic is that of an LU factorisation followed
+// by forward and back substitution, the pivots' reciprocals kept.
 template <int N, int NR>
 CPFFT_HD inline void lu_solve(double (&A)[N][N], double (&B)[N][NR]) {
+  double rp[N];
 #pragma unroll
   for (int j = 0; j < N; ++j) {
     int p = j;
@@ -85,26 +106,28 @@ CPFFT_HD inline void lu_solve(double (&A)[N][N], double (&B)[N][NR]) {
       const double v = fabs(A[i][j]);
       if (v > amax) { amax = v; p = i; }
     }
+    if (any_lane(p != j)) {
 #pragma unroll
-    for (int i = j + 1; i < N; ++i) {
-      const bool sw = (p == i);
+      for (int i = j + 1; i < N; ++i) {
+        const bool sw = (p == i);
 #pragma unroll
-      for (int k = j; k < N; ++k) {
-        const double a = A[j][k], b = A[i][k];
-        A[j][k] = sw ? b : a;
-        A[i][k] = sw ? a : b;
-      }
+        for (int k = j; k < N; ++k) {
+          const double a = A[j][k], b = A[i][k];
+          A[j][k] = sw ? b : a;
+          A[i][k] = sw ? a : b;
+        }
 #pragma unroll
-      for (int r = 0; r < NR; ++r) {
-        const double a = B[j][r], b = B[i][r];
-        B[j][r] = sw ? b : a;
-        B[i][r] = sw ? a : b;
+        for (int r = 0; r < NR; ++r) {
+          const double a = B[j][r], b = B[i][r];
+          B[j][r] = sw ? b : a;
+          B[i][r] = sw ? a : b;
+        }
       }
     }
-    const double rp = 1.0 / A[j][j];
+    rp[j] = 1.0 / A[j][j];
 #pragma unroll
     for (int i = j + 1; i < N; ++i) {
-      const double l = A[i][j] * rp;
+      const double l = A[i][j] * rp[j];
 #pragma unroll
       for (int k = j + 1; k < N; ++k) A[i][k] -= l * A[j][k];
 #pragma unroll
@@ -118,7 +141,7 @@ CPFFT_HD inline void lu_solve(double (&A)[N][N], double (&B)[N][NR]) {
       double s = B[i][r];
 #pragma unroll
       for (int k = i + 1; k < N; ++k) s -= A[i][k] * B[k][r];
-      B[i][r] = s / A[i][i];
+      B[i][r] = s * rp[i];
     }
   }
 }
@@ -333,20 +356,63 @@ CPFFT_HD inline void Cv6(const double* __restrict__ C, const double v[6], double
 struct Slip {
   double u, au, p, g;
 };
-CPFFT_HD inline Slip slip_of(const MatParams& P, double dg, double rs, double tt) {
-  Slip r;
-  r.u = rs / tt;
-  r.au = fabs(r.u);
-  r.p = pw_nm2(P, r.au);
-  r.g = dg * (r.p * r.au) * r.u;
-  return r;
+
+// Slip systems taken at a time by the sums below: their loads, divisions and
+// powers are independent chains that overlap (one at a time, a chain of a
+// load, a dot product, a division and five dependent squarings is waited for
+// at each system: there is one wave per SIMD to fill it).  Divides 12, 24, 48;
+// six are no faster and need more registers.
+constexpr int kSysBatch = 4;
+
+// the slip increments of the kSysBatch systems from i0 on (sE = E^T s)
+template <int NS, class MP>
+CPFFT_HD inline void slip_batch(const MP& P, const Orient<NS>& o, double dg, int i0,
+                                const double sE[6], double tt, double (&m)[kSysBatch][6],
+                                double (&q)[kSysBatch][3], Slip (&sl)[kSysBatch]) {
+  static_assert(NS % kSysBatch == 0, "slip systems per batch");
+  const double itt = 1.0 / tt;
+#pragma unroll
+  for (int j = 0; j < kSysBatch; ++j) {
+#pragma unroll
+    for (int k = 0; k < 6; ++k) m[j][k] = o.ms[i0 + j][k];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) q[j][k] = o.qs[i0 + j][k];
+  }
+#pragma unroll
+  for (int j = 0; j < kSysBatch; ++j) {
+    const double rs = sE[0] * m[j][0] + sE[1] * m[j][1] + sE[2] * m[j][2] + sE[3] * m[j][3] +
+                      sE[4] * m[j][4] + sE[5] * m[j][5];
+    sl[j].u = rs * itt;
+    sl[j].au = fabs(sl[j].u);
+  }
+  if (rate_is_int(P)) {  // ipow of each
+    double b[kSysBatch];
+#pragma unroll
+    for (int j = 0; j < kSysBatch; ++j) {
+      sl[j].p = 1.0;
+      b[j] = sl[j].au;
+    }
+    for (int n = (int)P.rate_n - 2; n > 0; n >>= 1) {
+      if (n & 1) {
+#pragma unroll
+        for (int j = 0; j < kSysBatch; ++j) sl[j].p *= b[j];
+      }
+#pragma unroll
+      for (int j = 0; j < kSysBatch; ++j) b[j] *= b[j];
+    }
+  } else {
+#pragma unroll
+    for (int j = 0; j < kSysBatch; ++j) sl[j].p = pow(sl[j].au, P.rate_n - 2.0);
+  }
+#pragma unroll
+  for (int j = 0; j < kSysBatch; ++j) sl[j].g = dg * (sl[j].p * sl[j].au) * sl[j].u;
 }
 
 // Sums over slip systems at stress s and resistance tt, in the lattice
 // frame: mb = sum_s slip_s m_s, qb = sum_s slip_s q_s, sabs = sum |slip_s|.
 // The resolved shear is rs_s = s . (E m_s) = (E^T s) . m_s.
-template <int NS>
-CPFFT_HD inline void slip_sums(const MatParams& P, const Orient<NS>& o, const Point& pt,
+template <int NS, class MP>
+CPFFT_HD inline void slip_sums(const MP& P, const Orient<NS>& o, const Point& pt,
                                const double s[6], double tt, double mb[6], double qb[3],
                                double* sabs) {
   double sE[6];
@@ -355,26 +421,27 @@ CPFFT_HD inline void slip_sums(const MatParams& P, const Orient<NS>& o, const Po
 #pragma unroll
   for (int k = 0; k < 6; ++k) mb[k] = 0.0;
   qb[0] = qb[1] = qb[2] = 0.0;
-#pragma unroll 2
-  for (int i = 0; i < NS; ++i) {
-    const double* __restrict__ m = o.ms[i];
-    const double* __restrict__ q = o.qs[i];
-    const double rs = sE[0] * m[0] + sE[1] * m[1] + sE[2] * m[2] + sE[3] * m[3] + sE[4] * m[4] +
-                      sE[5] * m[5];
-    const Slip sl = slip_of(P, pt.dg, rs, tt);
+#pragma unroll 1
+  for (int i = 0; i < NS; i += kSysBatch) {
+    double m[kSysBatch][6], q[kSysBatch][3];
+    Slip sl[kSysBatch];
+    slip_batch<NS>(P, o, pt.dg, i, sE, tt, m, q, sl);
 #pragma unroll
-    for (int k = 0; k < 6; ++k) mb[k] += sl.g * m[k];
+    for (int j = 0; j < kSysBatch; ++j) {
 #pragma unroll
-    for (int k = 0; k < 3; ++k) qb[k] += sl.g * q[k];
-    sa += fabs(sl.g);
+      for (int k = 0; k < 6; ++k) mb[k] += sl[j].g * m[j][k];
+#pragma unroll
+      for (int k = 0; k < 3; ++k) qb[k] += sl[j].g * q[j][k];
+      sa += fabs(sl[j].g);
+    }
   }
   *sabs = sa;
 }
 
 // R1 (mm10_formR1, mm10_b.f:1065-1113): s - s_n - C (D - dbar) + 2 sym(s W)
 // with dbar = E mb, wp = W qb
-template <int NS>
-CPFFT_HD inline void form_R1(const MatParams& P, const Orient<NS>& o, const Point& pt,
+template <int NS, class MP>
+CPFFT_HD inline void form_R1(const MP& P, const Orient<NS>& o, const Point& pt,
                              const StateN& n, const double s[6], double tt, double R1[6],
                              double* sabs) {
   double mb[6], qb[3];
@@ -391,15 +458,16 @@ CPFFT_HD inline void form_R1(const MatParams& P, const Orient<NS>& o, const Poin
 }
 
 // tt from the Voce law (mm10_h_voche, mm10_b.f:1888-1916), tau_l = 0
-CPFFT_HD inline double voce_h(const MatParams& P, const StateN& n, double tt, double sabs) {
+template <class MP>
+CPFFT_HD inline double voce_h(const MP& P, const StateN& n, double tt, double sabs) {
   double h_term = 1.0 - (tt - P.tau_y) / P.tau_v;
-  double f = P.m_is_one ? h_term : pow(fabs(h_term), P.voche_m) * sgn1(h_term);
+  double f = m_is_one(P) ? h_term : pow(fabs(h_term), P.voche_m) * sgn1(h_term);
   return n.tt + P.theta_0 * (f * sabs);
 }
 
 // full residual R (mm10_formR, mm10_b.f:1029-1063); returns |R|^2 and tt_rate
-template <int NS>
-CPFFT_HD inline double form_R(const MatParams& P, const Orient<NS>& o, const Point& pt,
+template <int NS, class MP>
+CPFFT_HD inline double form_R(const MP& P, const Orient<NS>& o, const Point& pt,
                               const StateN& n, const double x[7], double R[7], double* tt_rate) {
   double sabs;
   form_R1<NS>(P, o, pt, n, x, x[6], R, &sabs);
@@ -413,22 +481,21 @@ CPFFT_HD inline double form_R(const MatParams& P, const Orient<NS>& o, const Poi
 }
 
 // Jacobian (mm10_formJ11/J12/J21/J22, mm10_b.f:177-481, 1918-1983).
-// NJ = 6: stress block only (predictor); NJ = 7: full system.
 // J11 = I + IW(wp) + sum_s dgdt_s (C E m_s + 2 sym(s, W q_s)) (E m_s)^T
 //     = I + IW(wp) + (C E M + 2 [sym(s, (W Q)_c)]_c) E^T
 // with M = sum_s dgdt_s m_s m_s^T (upper triangle kept) and
 // Q = sum_s dgdt_s q_s m_s^T.
-template <int NS, int NJ>
-CPFFT_HD inline void form_J(const MatParams& P, const Orient<NS>& o, const Point& pt,
-                            const double s[6], double tt, double (&J)[NJ][NJ]) {
+template <int NS, class MP>
+CPFFT_HD inline void form_J(const MP& P, const Orient<NS>& o, const Point& pt,
+                            const double s[6], double tt, double (&J)[7][7]) {
   const double n_ = P.rate_n;
   const double h_term = 1.0 - (tt - P.tau_y) / P.tau_v;
-  const double fh = P.m_is_one ? h_term : pow(fabs(h_term), P.voche_m) * sgn1(h_term);
-  const double absh_m = P.m_is_one ? fabs(h_term) : pow(fabs(h_term), P.voche_m);
+  const double fh = m_is_one(P) ? h_term : pow(fabs(h_term), P.voche_m) * sgn1(h_term);
+  const double absh_m = m_is_one(P) ? fabs(h_term) : pow(fabs(h_term), P.voche_m);
   double sE[6];
   rotET(pt.tn, s, sE);
   double M[6][6], Q[3][6], mb[6], qb[3], mf[6];
-  double etau = 0.0;
+  double sas = 0.0, sgas = 0.0;
 #pragma unroll
   for (int a = 0; a < 6; ++a) {
 #pragma unroll
@@ -442,38 +509,35 @@ CPFFT_HD inline void form_J(const MatParams& P, const Orient<NS>& o, const Point
 #pragma unroll
     for (int b = 0; b < 6; ++b) Q[k][b] = 0.0;
   }
-#pragma unroll 2
-  for (int i = 0; i < NS; ++i) {
-    const double* __restrict__ m = o.ms[i];
-    const double* __restrict__ q = o.qs[i];
-    const double rs = sE[0] * m[0] + sE[1] * m[1] + sE[2] * m[2] + sE[3] * m[3] + sE[4] * m[4] +
-                      sE[5] * m[5];
-    const Slip sl = slip_of(P, pt.dg, rs, tt);
-    const double dgdt = pt.dg * n_ / tt * (sl.p * sl.au);  // d slip / d rs
-    double dm[6];
+#pragma unroll 1
+  for (int i = 0; i < NS; i += kSysBatch) {
+    double m[kSysBatch][6], q[kSysBatch][3];
+    Slip sl[kSysBatch];
+    slip_batch<NS>(P, o, pt.dg, i, sE, tt, m, q, sl);
 #pragma unroll
-    for (int a = 0; a < 6; ++a) dm[a] = dgdt * m[a];
+    for (int j = 0; j < kSysBatch; ++j) {
+      const double dgdt = pt.dg * n_ / tt * (sl[j].p * sl[j].au);  // d slip / d rs
+      double dm[6];
 #pragma unroll
-    for (int a = 0; a < 6; ++a)
+      for (int a = 0; a < 6; ++a) dm[a] = dgdt * m[j][a];
 #pragma unroll
-      for (int b = a; b < 6; ++b) M[a][b] += dm[a] * m[b];
+      for (int a = 0; a < 6; ++a)
 #pragma unroll
-    for (int k = 0; k < 3; ++k)
+        for (int b = a; b < 6; ++b) M[a][b] += dm[a] * m[j][b];
 #pragma unroll
-      for (int b = 0; b < 6; ++b) Q[k][b] += q[k] * dm[b];
+      for (int k = 0; k < 3; ++k)
 #pragma unroll
-    for (int k = 0; k < 6; ++k) mb[k] += sl.g * m[k];
+        for (int b = 0; b < 6; ++b) Q[k][b] += q[j][k] * dm[b];
 #pragma unroll
-    for (int k = 0; k < 3; ++k) qb[k] += sl.g * q[k];
-    if (NJ == 7) {
-      const double f21 = fh * sl.p * sl.u;  // |h|^m sgn(h) |u|^(n-2) u
+      for (int k = 0; k < 6; ++k) mb[k] += sl[j].g * m[j][k];
 #pragma unroll
-      for (int k = 0; k < 6; ++k) mf[k] += f21 * m[k];
-      const double as = fabs(sl.g);
-      const double sgs = P.jac_exact ? 1.0 : sgn1(sl.g);
-      etau += (P.voche_m * (-1.0 / P.tau_v) * as / fabs(h_term) -
-               as * n_ / tt * sgn1(h_term) * sgs) *
-              absh_m;
+      for (int k = 0; k < 3; ++k) qb[k] += sl[j].g * q[j][k];
+      const double f21 = fh * sl[j].p * sl[j].u;  // |h|^m sgn(h) |u|^(n-2) u
+#pragma unroll
+      for (int k = 0; k < 6; ++k) mf[k] += f21 * m[j][k];
+      const double as = fabs(sl[j].g);
+      sas += as;
+      sgas += P.jac_exact ? as : sl[j].g;  // as * sgn(slip)
     }
   }
   // T[:, c] = C E M[:, c] + 2 sym(s, W Q[:, c]); row a of J11 is E T[a, :]^T
@@ -502,21 +566,24 @@ CPFFT_HD inline void form_J(const MatParams& P, const Orient<NS>& o, const Point
   }
   double wp[3];
   mv3(pt.W, qb, wp);
-  if (NJ == 7) {
+  {
     // J12 = -n/tt sum_s slip_s (C E m_s + 2 sym(s, W q_s)) = -n/tt (C E mb + 2 sym(s, wp))
     double emb[6], cm[6], sw[6];
     rotE(pt.tn, mb, emb);
     Cv6(o.C, emb, cm);
     symsw(s, wp, sw);
 #pragma unroll
-    for (int a = 0; a < 6; ++a) J[a][NJ - 1] = (cm[a] + 2.0 * sw[a]) * (-n_ / tt);
+    for (int a = 0; a < 6; ++a) J[a][6] = (cm[a] + 2.0 * sw[a]) * (-n_ / tt);
     // J21 = -theta_0 dg n/tt E mf, J22 = 1 - theta_0 etau
     double emf[6];
     rotE(pt.tn, mf, emf);
     const double fac = P.theta_0 * pt.dg * n_ / tt;
 #pragma unroll
-    for (int b = 0; b < 6; ++b) J[NJ - 1][b] = -emf[b] * fac;
-    J[NJ - 1][NJ - 1] = 1.0 - P.theta_0 * etau;
+    for (int b = 0; b < 6; ++b) J[6][b] = -emf[b] * fac;
+    const double etau = (P.voche_m * (-1.0 / P.tau_v) / fabs(h_term) * sas -
+                         n_ / tt * sgn1(h_term) * sgas) *
+                        absh_m;
+    J[6][6] = 1.0 - P.theta_0 * etau;
   }
   // IW(wp) (mm10_iw, mm10_b.f:1605-1634) and identity
   J[0][3] += 2.0 * wp[2];
@@ -567,17 +634,22 @@ CPFFT_HD inline void setup_point(const MatParams& P, const double R[3][3], const
 // which the last full Jacobian was formed. Returns fail.
 // x0w: optional starting point [stress, tt] (the warm start); without it
 // the predictor starts from x with tt extrapolated (mm10_a.f:2993-3023).
-template <int NS>
-CPFFT_HD inline int local_solve(const MatParams& P, const Orient<NS>& o, const Point& pt,
+// One loop for both stages of the reference: the predictor (a 6x6 Newton on
+// R1 at the extrapolated tt, mm10_a.f:2975-3156) and the full Newton on
+// [R1; R2] (mm10_a.f:3162-3293), start points and line searches included.  A
+// trip evaluates the residual at xn, decides, and unless the point is
+// rejected or final forms the Jacobian and the next step; the predictor's
+// system is the full one with tt held (unit last row and column).  So lanes
+// of a wave in different stages share trips, and the residual, the Jacobian
+// and the factorisation are in the code (and its registers) once.
+template <int NS, class MP>
+CPFFT_HD inline int local_solve(const MP& P, const Orient<NS>& o, const Point& pt,
                                 const StateN& n, double dtinc, double x[7], double xprev[7],
                                 double* tt_rate, Counters& cnt, const double* x0w = nullptr,
                                 double x0w_res = 0.0) {
   const double cls = 1.0e-4, red = 0.5;
   const int mls = 10;
-  int fail = 0;
-  bool warm = false;
-  double inR1;
-  // ---- predictor: 6x6 Newton on R1 at extrapolated tt (mm10_a.f:2975-3156)
+  double xn[7];  // the point to evaluate
   {
     double d1[6], d2[6];
 #pragma unroll
@@ -600,290 +672,263 @@ CPFFT_HD inline int local_solve(const MatParams& P, const Orient<NS>& o, const P
 #pragma unroll
     for (int k = 0; k < 6; ++k) cosang += d1[k] * d2[k];
     cosang = fmax(cosang, 0.0);
-    double x2 = x[6] + cosang * n.tt_rate * dtinc;
-    double x1[6], R1[6], sabs;
 #pragma unroll
-    for (int k = 0; k < 6; ++k) x1[k] = x[k];
-    form_R1<NS>(P, o, pt, n, x1, x2, R1, &sabs);
-    double dot = 0.0;
+    for (int k = 0; k < 6; ++k) xn[k] = x[k];
+    xn[6] = x[6] + cosang * n.tt_rate * dtinc;
+  }
+  enum { kStart, kWarm, kSearch };
+  int at = kStart;     // what xn is
+  bool full = false;   // stage: predictor or full Newton
+  int it = 0, ls = 0;  // iterations of the stage, cuts of the line search
+  double inR1 = 0.0, inR = 0.0, ls1 = 0.0, ls2 = 0.0, alpha = 1.0;
+  double R[7], dx[7];
+  for (;;) {
+    const double dot7 = form_R<NS>(P, o, pt, n, xn, R, tt_rate);
+    double dot = full ? dot7 : 0.0;
+    if (!full) {
 #pragma unroll
-    for (int k = 0; k < 6; ++k) dot += R1[k] * R1[k];
-    double nR1 = sqrt(dot);
-    inR1 = nR1;
-    if (x0w && x0w_res < nR1) {
-      // warm start: the full state x0w (stress and slip resistance) has a
-      // full residual below the plain start's predictor residual, so the
-      // predictor is skipped and the full Newton starts there
-#pragma unroll
-      for (int k = 0; k < 7; ++k) x[k] = x0w[k];
-      warm = true;
+      for (int k = 0; k < 6; ++k) dot += R[k] * R[k];
     }
-    int it = 0, pfail = 0;
-    while (!warm && nR1 > P.atol1 && nR1 / inR1 > P.rtol1) {
-      double A[6][6], dx[6][1], gJ[6];
-      form_J<NS, 6>(P, o, pt, x1, x2, A);
-      // line-search slope J^T R before A is factorised
-#pragma unroll
-      for (int b = 0; b < 6; ++b) {
-        double wv = 0.0;
-#pragma unroll
-        for (int a = 0; a < 6; ++a) wv += A[a][b] * R1[a];
-        gJ[b] = wv;
-      }
-#pragma unroll
-      for (int a = 0; a < 6; ++a) {
-        dx[a][0] = R1[a];
-#pragma unroll
-        for (int b = 0; b < 6; ++b) A[a][b] = -A[a][b];
-      }
-      lu_solve<6, 1>(A, dx);
-      double ls1 = 0.5 * dot, ls2 = 0.0;
-#pragma unroll
-      for (int b = 0; b < 6; ++b) ls2 += dx[b][0] * gJ[b];
-      ls2 *= cls;
-      double alpha = 1.0;
-      for (int ls = 0;; ++ls) {
-        double nlsx = ls1 + ls2 * alpha, xn[6];
-#pragma unroll
-        for (int k = 0; k < 6; ++k) xn[k] = x1[k] + alpha * dx[k][0];
-        form_R1<NS>(P, o, pt, n, xn, x2, R1, &sabs);
-        cnt.ls_evals++;
-        dot = 0.0;
-#pragma unroll
-        for (int k = 0; k < 6; ++k) dot += R1[k] * R1[k];
-        nR1 = sqrt(dot);
-        if (0.5 * dot <= nlsx || ls > mls) {
-#pragma unroll
-          for (int k = 0; k < 6; ++k) x1[k] = xn[k];
-          break;
-        }
+    double nR = sqrt(dot);
+    if (at == kSearch) {
+      cnt.ls_evals++;
+      if (!(0.5 * dot <= ls1 + ls2 * alpha || ls > mls)) {
+        ++ls;
         alpha *= red;
+#pragma unroll
+        for (int k = 0; k < 7; ++k) xn[k] = x[k] + alpha * dx[k];
+        continue;
       }
       ++it;
       bool nan = false;
 #pragma unroll
-      for (int k = 0; k < 6; ++k) nan |= (x1[k] != x1[k]);
-      if (it > P.miter || nan) { pfail = 1; break; }
-    }
-    cnt.pred_it += it;
-    if (pfail) {
-      fail = 1;
-    } else if (!warm) {
+      for (int k = 0; k < 7; ++k) nan |= (xn[k] != xn[k]);
+      if (it > P.miter || nan) {
+        if (full) cnt.upd_it += it; else cnt.pred_it += it;
+        return 1;
+      }
+    } else if (at == kStart) {
+      inR1 = inR = nR;
+      if (x0w && x0w_res < nR) {
+        // warm start: the full state x0w (stress and slip resistance) has a
+        // full residual below the plain start's predictor residual, so the
+        // predictor is skipped and the full Newton starts there
 #pragma unroll
-      for (int k = 0; k < 6; ++k) x[k] = x1[k];
-      x[6] = x2;
+        for (int k = 0; k < 7; ++k) xn[k] = x0w[k];
+        at = kWarm;
+        full = true;
+        continue;
+      }
+    } else {  // kWarm
+      inR = nR == 0.0 ? inR1 : nR;
     }
-  }
-  // ---- full Newton on [R1; R2] (mm10_a.f:3162-3293)
-  {
-    double R[7];
-    double dot = form_R<NS>(P, o, pt, n, x, R, tt_rate);
-    double nR = sqrt(dot), inR = nR;
-    if (inR == 0.0) inR = inR1;
-    int it = 0;
 #pragma unroll
-    for (int k = 0; k < 7; ++k) xprev[k] = x[k];
-    while ((nR > P.atol && nR / inR > P.rtol) || it < 1) {
-      double A[7][7], dx[7][1], gJ[7];
-      form_J<NS, 7>(P, o, pt, x, x[6], A);
+    for (int k = 0; k < 7; ++k) x[k] = xn[k];
+    if (!full && !(nR > P.atol1 && nR / inR > P.rtol1)) {
+      // predictor done: the full Newton starts here
+      cnt.pred_it += it;
+      it = 0;
+      full = true;
+      dot = dot7;
+      nR = sqrt(dot);
+      inR = nR == 0.0 ? inR1 : nR;
+    }
+    if (full && !((nR > P.atol && nR / inR > P.rtol) || it < 1)) break;
+    double A[7][7], rhs[7][1];
+    form_J<NS>(P, o, pt, x, x[6], A);
+    if (full) {
 #pragma unroll
       for (int k = 0; k < 7; ++k) xprev[k] = x[k];
+    } else {
 #pragma unroll
-      for (int b = 0; b < 7; ++b) {
-        double wv = 0.0;
-#pragma unroll
-        for (int a = 0; a < 7; ++a) wv += A[a][b] * R[a];
-        gJ[b] = wv;
-      }
-#pragma unroll
-      for (int a = 0; a < 7; ++a) {
-        dx[a][0] = R[a];
-#pragma unroll
-        for (int b = 0; b < 7; ++b) A[a][b] = -A[a][b];
-      }
-      lu_solve<7, 1>(A, dx);
-      double ls1 = 0.5 * dot, ls2 = 0.0;
-#pragma unroll
-      for (int b = 0; b < 7; ++b) ls2 += dx[b][0] * gJ[b];
-      ls2 *= cls;
-      double alpha = 1.0;
-      for (int ls = 0;; ++ls) {
-        double nlsx = ls1 + ls2 * alpha, xn[7];
-#pragma unroll
-        for (int k = 0; k < 7; ++k) xn[k] = x[k] + alpha * dx[k][0];
-        dot = form_R<NS>(P, o, pt, n, xn, R, tt_rate);
-        cnt.ls_evals++;
-        nR = sqrt(dot);
-        if (0.5 * dot <= nlsx || ls > mls) {
-#pragma unroll
-          for (int k = 0; k < 7; ++k) x[k] = xn[k];
-          break;
-        }
-        alpha *= red;
-      }
-      ++it;
-      bool nan = false;
-#pragma unroll
-      for (int k = 0; k < 7; ++k) nan |= (x[k] != x[k]);
-      if (it > P.miter || nan) { fail = 1; break; }
+      for (int k = 0; k < 6; ++k) A[k][6] = A[6][k] = 0.0;
+      A[6][6] = 1.0;
+      R[6] = 0.0;
     }
-    cnt.upd_it += it;
+    // line-search slope J^T R before A is factorised
+    double gJ[7];
+#pragma unroll
+    for (int b = 0; b < 7; ++b) {
+      double wv = 0.0;
+#pragma unroll
+      for (int a = 0; a < 7; ++a) wv += A[a][b] * R[a];
+      gJ[b] = wv;
+    }
+#pragma unroll
+    for (int a = 0; a < 7; ++a) {
+      rhs[a][0] = R[a];
+#pragma unroll
+      for (int b = 0; b < 7; ++b) A[a][b] = -A[a][b];
+    }
+    lu_solve<7, 1>(A, rhs);
+    ls1 = 0.5 * dot;
+    ls2 = 0.0;
+#pragma unroll
+    for (int b = 0; b < 7; ++b) {
+      dx[b] = rhs[b][0];
+      ls2 += dx[b] * gJ[b];
+    }
+    ls2 *= cls;
+    alpha = 1.0;
+    ls = 0;
+    at = kSearch;
+#pragma unroll
+    for (int k = 0; k < 7; ++k) xn[k] = x[k] + dx[k];
   }
-  return fail;
+  cnt.upd_it += it;
+  return 0;
 }
 
 // ------------------------------------------------------- exact dP/dF
 // cep2A_a (cep2A.f:86-284) for one voxel; C = consistent tangent (row-major
 // 6x6), t = unrotated Cauchy stress (Voigt), K written column (k,l) at a time.
+// The derivatives of the two polar rotations and of the velocity gradient
+// with respect to F_kl are sums of outer products of column k of one matrix
+// with row l of another (dR = dY1 (RYR_.k Y_l. - RY_.l RY_k.) with
+// Y = tr(U) I - U, and so on), so every product with them is one too, and
+// its factors are 3x3 products formed once: about 190 multiply-adds a column
+// instead of 570 with the derivatives multiplied out.  Bound by the 81 stores
+// and the two polar decompositions: 0.53 ms at 128^3 (4.2 TB/s of its 1080
+// bytes a voxel) against 1.40 ms, one wave per SIMD either way (with two,
+// the compiler keeps a kilobyte a lane in scratch memory: 1.79 ms).
 template <class Store>
 CPFFT_HD inline void dPdF(const double Fn[3][3], const double Fn1[3][3], const double t6[6],
                           const double C[6][6], const double Rh[3][3], const double fnhinv[3][3],
                           const double R[3][3], const double finv[3][3], double J,
                           Store&& store) {
-  double t[3][3] = {{t6[0], t6[3], t6[5]}, {t6[3], t6[1], t6[4]}, {t6[5], t6[4], t6[2]}};
-  auto mm = [](const double A[3][3], const double B[3][3], double Cc[3][3]) {
+  const double t[3][3] = {{t6[0], t6[3], t6[5]}, {t6[3], t6[1], t6[4]}, {t6[5], t6[4], t6[2]}};
+  // A B, A B^T, A^T B
+  auto mm = [](const double A[3][3], const double B[3][3], double o[3][3]) {
+#pragma unroll
     for (int i = 0; i < 3; ++i)
-      for (int j = 0; j < 3; ++j) Cc[i][j] = A[i][0] * B[0][j] + A[i][1] * B[1][j] + A[i][2] * B[2][j];
+#pragma unroll
+      for (int j = 0; j < 3; ++j) o[i][j] = A[i][0] * B[0][j] + A[i][1] * B[1][j] + A[i][2] * B[2][j];
+  };
+  auto mmt = [](const double A[3][3], const double B[3][3], double o[3][3]) {
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+#pragma unroll
+      for (int j = 0; j < 3; ++j) o[i][j] = A[i][0] * B[j][0] + A[i][1] * B[j][1] + A[i][2] * B[j][2];
+  };
+  auto mtm = [](const double A[3][3], const double B[3][3], double o[3][3]) {
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+#pragma unroll
+      for (int j = 0; j < 3; ++j) o[i][j] = A[0][i] * B[0][j] + A[1][i] * B[1][j] + A[2][i] * B[2][j];
+  };
+  auto scale = [](double A[3][3], double f) {
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+#pragma unroll
+      for (int j = 0; j < 3; ++j) A[i][j] *= f;
   };
   auto det = [](const double A[3][3]) {
     return A[0][0] * A[1][1] * A[2][2] + A[0][1] * A[1][2] * A[2][0] + A[0][2] * A[1][0] * A[2][1] -
            A[0][0] * A[1][2] * A[2][1] - A[0][1] * A[1][0] * A[2][2] - A[0][2] * A[1][1] * A[2][0];
   };
-  double Rt[3][3], U[3][3], Y[3][3], sigma[3][3], Uinv[3][3], tUi[3][3], RT_[3][3];
-  double RY[3][3], RYR[3][3], RtRF[3][3];
-  for (int i = 0; i < 3; ++i)
-    for (int j = 0; j < 3; ++j) Rt[i][j] = R[j][i];
-  mm(Rt, Fn1, U);
-  double trU = U[0][0] + U[1][1] + U[2][2];
-  for (int i = 0; i < 3; ++i)
-    for (int j = 0; j < 3; ++j) Y[i][j] = (i == j ? trU : 0.0) - U[i][j];
-  mm(R, t, RT_);
-  mm(RT_, Rt, sigma);
-  mm(finv, R, Uinv);
-  mm(t, Uinv, tUi);
-  mm(R, Y, RY);
-  mm(RY, Rt, RYR);
-  double dY1 = 1.0 / det(Y);
-  mm(RT_, Uinv, RtRF);
-  double Rht[3][3], Fnh[3][3], dFn[3][3], Uh[3][3], Yh[3][3], RYRh[3][3], RYh[3][3], FpF[3][3];
-  double L[3][3], D2[3][3];
-  for (int i = 0; i < 3; ++i)
-    for (int j = 0; j < 3; ++j) {
-      Rht[i][j] = Rh[j][i];
-      Fnh[i][j] = 0.5 * (Fn1[i][j] + Fn[i][j]);
-      dFn[i][j] = Fn1[i][j] - Fn[i][j];
-      FpF[i][j] = 0.5 * fnhinv[i][j];
-    }
-  mm(Rht, Fnh, Uh);
-  double trUh = Uh[0][0] + Uh[1][1] + Uh[2][2];
-  for (int i = 0; i < 3; ++i)
-    for (int j = 0; j < 3; ++j) Yh[i][j] = (i == j ? trUh : 0.0) - Uh[i][j];
-  mm(Rh, Yh, RYh);
-  mm(RYh, Rht, RYRh);
-  double dYh1 = 0.5 / det(Yh);
-  mm(dFn, FpF, L);
-  for (int i = 0; i < 3; ++i)
-    for (int j = 0; j < 3; ++j) D2[i][j] = L[i][j] + L[j][i];
-  const int vg[3][3] = {{0, 3, 5}, {3, 1, 4}, {5, 4, 2}};
-  // row l / column k of a 3x3 matrix for a run-time k, l (selects keep the
-  // matrices in registers)
-  auto colk = [](const double A[3][3], int k, double o[3]) {
+  // tr(U) I - U of U = R^T F
+  auto trace_minus = [&](const double Rr[3][3], const double Ff[3][3], double Y[3][3]) {
+    double U[3][3];
+    mtm(Rr, Ff, U);
+    const double tr = U[0][0] + U[1][1] + U[2][2];
 #pragma unroll
-    for (int i = 0; i < 3; ++i) o[i] = k == 0 ? A[i][0] : (k == 1 ? A[i][1] : A[i][2]);
+    for (int i = 0; i < 3; ++i)
+#pragma unroll
+      for (int j = 0; j < 3; ++j) Y[i][j] = (i == j ? tr : 0.0) - U[i][j];
   };
-  auto rowl = [](const double A[3][3], int l, double o[3]) {
-#pragma unroll
-    for (int i = 0; i < 3; ++i) o[i] = l == 0 ? A[0][i] : (l == 1 ? A[1][i] : A[2][i]);
-  };
-  // D2 Rh does not depend on (k, l)
-  double A1[3][3];
-  mm(D2, Rh, A1);
-#pragma unroll 1
-  for (int kl = 0; kl < 9; ++kl) {
-    const int k = kl / 3, l = kl - 3 * k;
-    double RYRk[3], Yl[3], RYl[3], RYk[3], RYRhk[3], Yhl[3], RYhl[3], RYhk[3], FpFl[3], Lk[3];
-    double fk[3], fl[3];
-    colk(RYR, k, RYRk);
-    rowl(Y, l, Yl);
-    colk(RY, l, RYl);
-    rowl(RY, k, RYk);
-    colk(RYRh, k, RYRhk);
-    rowl(Yh, l, Yhl);
-    colk(RYh, l, RYhl);
-    rowl(RYh, k, RYhk);
-    rowl(FpF, l, FpFl);
-    colk(L, k, Lk);
-    colk(finv, k, fk);  // finv[.][k]
-    rowl(finv, l, fl);  // finv[l][.]
-    const double flk = fk[0] * (l == 0) + fk[1] * (l == 1) + fk[2] * (l == 2);
-    // dR(i,m)/dF(k,l), dRh(i,m)/dF(k,l), dL(i,m)/dF(k,l)
-    double dR[3][3], dRh[3][3], dL[3][3];
-#pragma unroll
-    for (int i = 0; i < 3; ++i)
-#pragma unroll
-      for (int m = 0; m < 3; ++m) {
-        dR[i][m] = dY1 * (RYRk[i] * Yl[m] - RYl[i] * RYk[m]);
-        dRh[i][m] = dYh1 * (RYRhk[i] * Yhl[m] - RYhl[i] * RYhk[m]);
-        dL[i][m] = ((i == k) ? FpFl[m] : 0.0) - Lk[i] * FpFl[m];
-      }
-    // dt(i,j)/dF(k,l): dRh^T D2 Rh + Rh^T (dL + dL^T) Rh + Rh^T D2 dRh
-    double S[3][3], A2[3][3], dd[3][3];
-#pragma unroll
-    for (int i = 0; i < 3; ++i)
-#pragma unroll
-      for (int j = 0; j < 3; ++j) S[i][j] = dL[i][j] + dL[j][i];
-    mm(S, Rh, A2);  // S Rh
+  // strain part: d(uddt)(k,l) = sym2(Yh_l. x Ek - RYh_k. x Gl + Bk x Hl), sym2(X) = X + X^T
+  double Yh[3][3], RYh[3][3], E[3][3], G[3][3], B[3][3], H[3][3];
+  {
+    double Fnh[3][3], L[3][3], FpF[3][3], D2[3][3], A1[3][3], RYRh[3][3], T[3][3];
 #pragma unroll
     for (int i = 0; i < 3; ++i)
 #pragma unroll
       for (int j = 0; j < 3; ++j) {
-        double v = 0.0;
-#pragma unroll
-        for (int m = 0; m < 3; ++m) v += dRh[m][i] * A1[m][j] + Rh[m][i] * A2[m][j];
-        double w = 0.0;
-#pragma unroll
-        for (int m = 0; m < 3; ++m) {
-          double dm = 0.0;
-#pragma unroll
-          for (int q = 0; q < 3; ++q) dm += D2[m][q] * dRh[q][j];
-          w += Rh[m][i] * dm;
-        }
-        dd[i][j] = v + w;
+        Fnh[i][j] = 0.5 * (Fn1[i][j] + Fn[i][j]);
+        T[i][j] = Fn1[i][j] - Fn[i][j];
+        FpF[i][j] = 0.5 * fnhinv[i][j];
       }
-    // tangent contraction dt'(i,j) = sum_ab cep99(ij,ab) dd(b,a)
-    double dt[3][3];
+    trace_minus(Rh, Fnh, Yh);
+    const double dYh1 = 0.5 / det(Yh);
+    mm(Rh, Yh, RYh);
+    mmt(RYh, Rh, RYRh);
+    mm(T, FpF, L);  // dF F_{n+1/2}^-1 / 2
 #pragma unroll
     for (int i = 0; i < 3; ++i)
 #pragma unroll
-      for (int j = 0; j < 3; ++j) {
-        double v = 0.0;
-#pragma unroll
-        for (int a = 0; a < 3; ++a)
-#pragma unroll
-          for (int b = 0; b < 3; ++b) v += C[vg[a][b]][vg[i][j]] * dd[b][a];
-        dt[i][j] = v;
-      }
-    // dP(i,j)/dF(k,l)
-    double Rdt[3][3], RdtU[3][3];
-    mm(R, dt, Rdt);
-    mm(Rdt, Uinv, RdtU);
+      for (int j = 0; j < 3; ++j) D2[i][j] = L[i][j] + L[j][i];
+    mm(D2, Rh, A1);
+    mtm(RYRh, A1, E);  // row k
+    mtm(RYh, A1, G);   // row l
+    scale(E, dYh1);
+    scale(G, dYh1);
 #pragma unroll
     for (int i = 0; i < 3; ++i)
 #pragma unroll
-      for (int j = 0; j < 3; ++j) {
-        double v = RtRF[i][j] * (J * flk) + J * RdtU[i][j];
-#pragma unroll
-        for (int m = 0; m < 3; ++m) {
-          v -= J * sigma[i][m] * fk[j] * fl[m];
-          v += J * dR[i][m] * tUi[m][j];
-          double s4 = 0.0;
-#pragma unroll
-          for (int q = 0; q < 3; ++q) s4 += dR[q][m] * finv[j][q];
-          v += J * RT_[i][m] * s4;
-        }
-        store(i * 27 + j * 9 + kl, v);
-      }
+      for (int j = 0; j < 3; ++j) T[i][j] = (i == j ? 1.0 : 0.0) - L[i][j];
+    mtm(T, Rh, B);  // row k: Rh^T (e_k - L_.k)
+    mm(FpF, Rh, H);  // row l
   }
+  // stress part
+  double RT[3][3], Ui[3][3], W[3][3], Sg[3][3], RY[3][3], RYR[3][3], YT[3][3], RYT[3][3];
+  double P1[3][3], P2[3][3], Q1[3][3], Q2[3][3], JR[3][3];
+  {
+    double Y[3][3], tUi[3][3], sigma[3][3];
+    trace_minus(R, Fn1, Y);
+    const double f = J / det(Y);
+    mm(R, t, RT);
+    mmt(RT, R, sigma);
+    mm(finv, R, Ui);
+    mm(t, Ui, tUi);
+    mm(RT, Ui, W);
+    scale(W, J);
+    mmt(sigma, finv, Sg);  // column l
+    scale(Sg, J);
+    mm(R, Y, RY);
+    mmt(RY, R, RYR);
+    mm(Y, tUi, YT);    // row l
+    mm(RY, tUi, RYT);  // row k
+    mmt(RT, Y, P1);    // column l
+    mm(finv, RYR, Q1);  // column k
+    mmt(RT, RY, P2);    // column k
+    mm(finv, RY, Q2);   // column l
+    scale(YT, f);
+    scale(RYT, f);
+    scale(P1, f);
+    scale(P2, f);
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+#pragma unroll
+      for (int j = 0; j < 3; ++j) JR[i][j] = J * R[i][j];
+  }
+#pragma unroll
+  for (int k = 0; k < 3; ++k)
+#pragma unroll
+    for (int l = 0; l < 3; ++l) {
+      auto dd = [&](int i, int j) {
+        return (Yh[l][i] * E[k][j] + Yh[l][j] * E[k][i]) - (RYh[k][i] * G[l][j] + RYh[k][j] * G[l][i]) +
+               (B[k][i] * H[l][j] + B[k][j] * H[l][i]);
+      };
+      // engineering strains of the increment, C column by column as cep99
+      const double e[6] = {dd(0, 0), dd(1, 1), dd(2, 2), 2.0 * dd(0, 1), 2.0 * dd(1, 2), 2.0 * dd(0, 2)};
+      double d6[6];
+#pragma unroll
+      for (int v = 0; v < 6; ++v)
+        d6[v] = (C[0][v] * e[0] + C[1][v] * e[1] + C[2][v] * e[2]) +
+                (C[3][v] * e[3] + C[4][v] * e[4] + C[5][v] * e[5]);
+      const double dt[3][3] = {{d6[0], d6[3], d6[5]}, {d6[3], d6[1], d6[4]}, {d6[5], d6[4], d6[2]}};
+      double Rdt[3][3], X[3][3];
+      mm(JR, dt, Rdt);
+      mm(Rdt, Ui, X);
+#pragma unroll
+      for (int i = 0; i < 3; ++i)
+#pragma unroll
+        for (int j = 0; j < 3; ++j)
+          store(i * 27 + j * 9 + 3 * k + l,
+                X[i][j] + ((W[i][j] * finv[l][k] - Sg[i][l] * finv[j][k]) +
+                           ((RYR[i][k] * YT[l][j] - RY[i][l] * RYT[k][j]) +
+                            (P1[i][l] * Q1[j][k] - P2[i][k] * Q2[j][l]))));
+    }
 }
 
 // ------------------------------------------------------- voxel update
@@ -1208,9 +1253,11 @@ CPFFT_HD inline void voxel_features(const MatParams& P, const Orient<NS>& o, int
 // handed to local_solve, which starts its full Newton there when that
 // residual is below the plain start's predictor residual; a warm solve that
 // fails is redone from the plain start.
-template <int NS, class LoadF, class LoadS, class StoreS, class StoreP, class StoreT>
-CPFFT_HD inline void voxel_update(const MatParams& P, const Orient<NS>& o, int step, int iter,
-                                  LoadF&& ldF, LoadS&& ldn, StoreS&& stn1, StoreP&& stP,
+// EXPL: the explicit elastic predictor (iter 0), else a Newton iteration.
+// WARM: whether ws or xprev_it may be given.
+template <int NS, bool EXPL, bool WARM, class MP, class LoadF, class LoadS, class StoreS, class StoreP,
+          class StoreT>
+CPFFT_HD inline void voxel_update(const MP& P, const Orient<NS>& o, int step, LoadF&& ldF, LoadS&& ldn, StoreS&& stn1, StoreP&& stP,
                                   StoreT&& stT, Counters& cnt, const float* ws = nullptr,
                                   long wstride = 0, const double* xprev_it = nullptr) {
   double uddt[6], rn1[3][3];
@@ -1269,7 +1316,7 @@ CPFFT_HD inline void voxel_update(const MatParams& P, const Orient<NS>& o, int s
 #pragma unroll
   for (int k = 0; k < 6; ++k) { temp1 += uddt[k] * uddt[k]; temp2 += n.stress[k] * n.stress[k]; }
   const bool no_load = (temp2 == 0.0) && (temp1 == 0.0);
-  if (iter == 0 || no_load) {
+  if (EXPL || no_load) {
     // explicit update with the elastic tangent (mm10_a.f:2735-2753)
 #pragma unroll
     for (int a = 0; a < 6; ++a)
@@ -1277,14 +1324,16 @@ CPFFT_HD inline void voxel_update(const MatParams& P, const Orient<NS>& o, int s
       for (int b = 0; b < 6; ++b) tangent[a][b] = C[a * 6 + b];
 #pragma unroll
     for (int k = 0; k < 6; ++k) s1[k] = n.stress[k];
-    if (!no_load) {
-      double R1[6], sabs;
-      form_R1<NS>(P, o, pt, n, n.stress, n.tt, R1, &sabs);
+    if constexpr (EXPL) {
+      if (!no_load) {
+        double R1[6], sabs;
+        form_R1<NS>(P, o, pt, n, n.stress, n.tt, R1, &sabs);
 #pragma unroll
-      for (int k = 0; k < 6; ++k) s1[k] = n.stress[k] - R1[k];
+        for (int k = 0; k < 6; ++k) s1[k] = n.stress[k] - R1[k];
+      }
     }
     tt1 = n.tt;
-  } else {
+  } else if constexpr (!EXPL) {
     // adaptive sub-stepping (mm10_a.f:2759-2843).  A successful pass ends
     // with frac + stp == 1 exactly (dyadic fractions), so pt then holds the
     // full-step point again.
@@ -1293,34 +1342,27 @@ CPFFT_HD inline void voxel_update(const MatParams& P, const Orient<NS>& o, int s
     for (int k = 0; k < 6; ++k) { x[k] = n.stress[k]; ost[k] = x[k]; }
     double frac = 0.0, stp = 1.0;
     int cuts = 0, fail = 0;
-    if (ws || xprev_it) {
-      double x0[7], xc[7], R[7], tr, best = 1.0e300;
-      auto consider = [&](const double* c) {
-        const double d = sqrt(form_R<NS>(P, o, pt, n, c, R, &tr));
+    // warm-start candidates: the first pass below tries the better one
+    double x0[7], best = 1.0e300;
+    bool warm = WARM && (ws || xprev_it);
+    if constexpr (WARM) {
+#pragma unroll 1
+      for (int c = 0; c < 2; ++c) {
+        double xc[7], R[7], tr;
+        if (c == 0) {
+          if (!ws) continue;
+          warm_x0<NS>(P, o, pt, n, ws, wstride, xc);
+        } else {
+          if (!xprev_it) continue;
+#pragma unroll
+          for (int k = 0; k < 7; ++k) xc[k] = xprev_it[k];
+        }
+        const double d = sqrt(form_R<NS>(P, o, pt, n, xc, R, &tr));
         if (d < best) {  // false for NaN
           best = d;
 #pragma unroll
-          for (int k = 0; k < 7; ++k) x0[k] = c[k];
+          for (int k = 0; k < 7; ++k) x0[k] = xc[k];
         }
-      };
-      if (ws) {
-        warm_x0<NS>(P, o, pt, n, ws, wstride, xc);
-        consider(xc);
-      }
-      if (xprev_it) consider(xprev_it);
-      x[6] = n.tt;
-      fail = local_solve<NS>(P, o, pt, n, P.dt, x, xprev, &ttrate1, cnt,
-                             best < 1.0e300 ? x0 : nullptr, best);
-      bool ok = !fail && (x[6] == x[6]);
-#pragma unroll
-      for (int k = 0; k < 6; ++k) ok &= (x[k] == x[k]);
-      if (ok) {
-        frac = 1.0;
-      } else {
-        cnt.ws_fallback++;
-        fail = 0;
-#pragma unroll
-        for (int k = 0; k < 6; ++k) x[k] = ost[k];
       }
     }
     while (frac < 1.0) {
@@ -1331,7 +1373,21 @@ CPFFT_HD inline void voxel_update(const MatParams& P, const Orient<NS>& o, int s
         setup_point(P, rn1, n, Dw, P.dt * (stp + frac), pt);
       }
       x[6] = n.tt;
-      fail = local_solve<NS>(P, o, pt, n, P.dt * stp, x, xprev, &ttrate1, cnt);
+      fail = local_solve<NS>(P, o, pt, n, P.dt * stp, x, xprev, &ttrate1, cnt,
+                             warm && best < 1.0e300 ? x0 : nullptr, best);
+      if (WARM && warm) {
+        // a warm solve that fails is redone from the plain start
+        warm = false;
+        bool ok = !fail && (x[6] == x[6]);
+#pragma unroll
+        for (int k = 0; k < 6; ++k) ok &= (x[k] == x[k]);
+        if (ok) break;
+        cnt.ws_fallback++;
+        fail = 0;
+#pragma unroll
+        for (int k = 0; k < 6; ++k) x[k] = ost[k];
+        continue;
+      }
       if (fail) {
 #pragma unroll
         for (int k = 0; k < 6; ++k) x[k] = ost[k];
@@ -1377,7 +1433,7 @@ CPFFT_HD inline void voxel_update(const MatParams& P, const Orient<NS>& o, int s
       // symmetrised (mm10_a.f:1134-1142)
       {
         double J[7][7];
-        form_J<NS, 7>(P, o, pt, xprev, xprev[6], J);
+        form_J<NS>(P, o, pt, xprev, xprev[6], J);
         double JJ[6][6], B[6][6];
         const double j22 = J[6][6];
 #pragma unroll
@@ -1394,9 +1450,32 @@ CPFFT_HD inline void voxel_update(const MatParams& P, const Orient<NS>& o, int s
 #pragma unroll
           for (int b = 0; b < 6; ++b) tangent[a][b] = 0.5 * (B[a][b] + B[b][a]);
       }
-      // slip sums at the converged state
-      double mb[6], qb[3], sabs;
-      slip_sums<NS>(P, o, pt, s1, tt1, mb, qb, &sabs);
+      // slip sums at the converged state, the increments (and cumulative
+      // slips) stored as they are formed
+      double mb[6], qb[3];
+      {
+        double sE[6];
+        rotET(pt.tn, s1, sE);
+#pragma unroll
+        for (int k = 0; k < 6; ++k) mb[k] = 0.0;
+        qb[0] = qb[1] = qb[2] = 0.0;
+#pragma unroll 1
+        for (int i = 0; i < NS; i += kSysBatch) {
+          double m[kSysBatch][6], q[kSysBatch][3];
+          Slip sl[kSysBatch];
+          slip_batch<NS>(P, o, pt.dg, i, sE, tt1, m, q, sl);
+#pragma unroll
+          for (int j = 0; j < kSysBatch; ++j) {
+            const double g = sl[j].g;
+#pragma unroll
+            for (int k = 0; k < 6; ++k) mb[k] += g * m[j][k];
+#pragma unroll
+            for (int k = 0; k < 3; ++k) qb[k] += g * q[j][k];
+            stn1(23 + i + j, g);
+            stn1(23 + NS + i + j, (step == 1 ? 0.0 : ldn(23 + NS + i + j)) + g);
+          }
+        }
+      }
       // plastic rotation (mm10_update_rotation): Rp = expm(W(wbarp)) Rp_n
       {
         double RW[3][3], tn[3][3], wb[3];
@@ -1434,18 +1513,9 @@ CPFFT_HD inline void voxel_update(const MatParams& P, const Orient<NS>& o, int s
              s1[4] * uddt[4] + s1[5] * uddt[5];
       double ee[6];
       {
-        double S[6][6], b[6][1];
-#pragma unroll
-        for (int a = 0; a < 6; ++a) {
-          b[a][0] = s1[a];
-#pragma unroll
-          for (int c = 0; c < 6; ++c) S[a][c] = C[a * 6 + c];
-        }
-        lu_solve<6, 1>(S, b);  // C^-1 sigma (SPD solve, mm10_a.f:3537)
         double er[6][6], bv[6];
+        Cv6(o.S, s1, bv);  // C^-1 sigma (mm10_a.f:3537)
         rt2rve(rn1, er);
-#pragma unroll
-        for (int c = 0; c < 6; ++c) bv[c] = b[c][0];
         mv6(er, bv, ee);
       }
       double dbar[6], wp[3], ewwe[6], ep[6];
@@ -1474,21 +1544,11 @@ CPFFT_HD inline void voxel_update(const MatParams& P, const Orient<NS>& o, int s
   stn1(16, ttrate1);
 #pragma unroll
   for (int k = 0; k < 6; ++k) stn1(17 + k, uddt[k]);
-  {
-    // slip increments and cumulative slip (zero outside a converged plastic update)
-    double sE[6];
-    rotET(pt.tn, s1, sE);
+  if (!plastic) {  // no slip outside a converged plastic update
 #pragma unroll 2
     for (int i = 0; i < NS; ++i) {
-      double g = 0.0;
-      if (plastic) {
-        const double* __restrict__ m = o.ms[i];
-        const double rs = sE[0] * m[0] + sE[1] * m[1] + sE[2] * m[2] + sE[3] * m[3] +
-                          sE[4] * m[4] + sE[5] * m[5];
-        g = slip_of(P, pt.dg, rs, tt1).g;
-      }
-      stn1(23 + i, g);
-      stn1(23 + NS + i, (step == 1 ? 0.0 : ldn(23 + NS + i)) + g);
+      stn1(23 + i, 0.0);
+      stn1(23 + NS + i, step == 1 ? 0.0 : ldn(23 + NS + i));
     }
   }
   const double w0 = step == 1 ? 0.0 : ldn(23 + 2 * NS + 0);
@@ -1528,6 +1588,17 @@ CPFFT_HD inline void voxel_update(const MatParams& P, const Orient<NS>& o, int s
     for (int j = 0; j < 3; ++j)
       stP(3 * i + j,
           detF * (cs[i][0] * fn1inv[j][0] + cs[i][1] * fn1inv[j][1] + cs[i][2] * fn1inv[j][2]));
+}
+
+template <int NS, class LoadF, class LoadS, class StoreS, class StoreP, class StoreT>
+CPFFT_HD inline void voxel_update(const MatParams& P, const Orient<NS>& o, int step, int iter,
+                                  LoadF&& ldF, LoadS&& ldn, StoreS&& stn1, StoreP&& stP,
+                                  StoreT&& stT, Counters& cnt, const float* ws = nullptr,
+                                  long wstride = 0, const double* xprev_it = nullptr) {
+  if (iter == 0)
+    voxel_update<NS, true, false>(P, o, step, ldF, ldn, stn1, stP, stT, cnt, ws, wstride, xprev_it);
+  else
+    voxel_update<NS, false, true>(P, o, step, ldF, ldn, stn1, stP, stT, cnt, ws, wstride, xprev_it);
 }
 
 // K4 = dP/dF (cep2A, cep2A.f:86-284) of one voxel from F_n, F_{n+1}, the

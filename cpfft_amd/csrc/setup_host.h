@@ -164,6 +164,24 @@ inline void build_orient(const double stiff[6][6], const double b[kMaxSlip][3], 
       for (int k = 0; k < 6; ++k) v += Rs[i][k] * tmp[k][j];
       o.C[i * 6 + j] = v;
     }
+  // S = C^-1 (C is positive definite: no pivoting)
+  long double A[6][12];
+  for (int i = 0; i < 6; ++i)
+    for (int j = 0; j < 6; ++j) {
+      A[i][j] = o.C[i * 6 + j];
+      A[i][6 + j] = i == j;
+    }
+  for (int p = 0; p < 6; ++p) {
+    const long double r = 1.0L / A[p][p];
+    for (int j = 0; j < 12; ++j) A[p][j] *= r;
+    for (int i = 0; i < 6; ++i) {
+      if (i == p) continue;
+      const long double f = A[i][p];
+      for (int j = 0; j < 12; ++j) A[i][j] -= f * A[p][j];
+    }
+  }
+  for (int i = 0; i < 6; ++i)
+    for (int j = 0; j < 6; ++j) o.S[i * 6 + j] = (double)A[i][6 + j];
 }
 
 // cubic elasticity through the compliance (mod_crystals.f:1833-1879)
