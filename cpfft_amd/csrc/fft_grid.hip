@@ -51,6 +51,12 @@ constexpr int kMaxE = 8;    // elements per thread of a transform, at most
 constexpr int kSlabN = 126; // largest edge of the slab kernels: N (N/2 + 1) <= kMaxE * 1024
 constexpr int kML = 8;      // x lines per component and block of k_mid (128-byte runs)
 constexpr int kMaxSt = 8;
+// Kernels' NC: the edge, or a plan read at run time.  Radices 11 and 13 take
+// more registers than 1024 threads have (24 to 96 bytes a lane go to scratch),
+// so the edges without these factors have instantiations without them: no
+// scratch, a solve at 45^3 3.21 ms instead of 3.35.
+constexpr int kAnyRadix = 0, kSmooth = -1;
+inline bool smooth(int N) { return N <= kSlabN && N % 11 != 0 && N % 13 != 0; }
 
 struct Grid {
   int N, NZ, nzk, NN;  // edge, N/2+1, planes kept, lines N*N
@@ -304,9 +310,14 @@ __device__ __forceinline__ void fft(cplx* buf, const cplx* tw, const Grid& g, in
     break;
       switch (r) {
         CPFFT_STAGE(2) CPFFT_STAGE(3) CPFFT_STAGE(4) CPFFT_STAGE(5) CPFFT_STAGE(6)
-        CPFFT_STAGE(7) CPFFT_STAGE(8) CPFFT_STAGE(9) CPFFT_STAGE(10) CPFFT_STAGE(11)
-        CPFFT_STAGE(13)
+        CPFFT_STAGE(7) CPFFT_STAGE(8) CPFFT_STAGE(9) CPFFT_STAGE(10)
         default: break;
+      }
+      if constexpr (NC == kAnyRadix) {
+        switch (r) {
+          CPFFT_STAGE(11) CPFFT_STAGE(13)
+          default: break;
+        }
       }
 #undef CPFFT_STAGE
       Ns *= r;
@@ -432,33 +443,62 @@ __device__ __forceinline__ bool cg_begin(const FwdArgs& a, int rhs, bool first, 
   return s_done != 0;
 }
 
-// (K4:F)_c of components c0 .. c0 + CPB at voxel e (or F_c without K4); DIR:
-// F is the new direction, its components stored, fc its value there
+// What components c0 .. c0 + CPB of K4:F (or of F, !HASK) at a voxel are formed
+// from; DIR: F is the last direction.  Fetched apart from their use: the first
+// point's travel while the kernel still reads the state of the iteration.
 template <bool HASK, bool DIR, int CPB>
-__device__ __forceinline__ void load_point(const FwdArgs& a, int rhs, int c0, long e, long V,
-                                           double beta, double (&v)[CPB], double (&fc)[CPB]) {
+struct Point {
+  double k[HASK ? CPB : 1][9], f[9], r[9];
+};
+template <bool HASK, bool DIR, int CPB>
+__device__ __forceinline__ void fetch_point(const FwdArgs& a, int rhs, int c0, long e, long V,
+                                            Point<HASK, DIR, CPB>& p) {
   const double* F = a.F.p[rhs];
   if constexpr (HASK) {
-    double k[CPB][9], f[9];
+    // uniform bases and one 32-bit offset (8 V < 2^32 at these edges): 27
+    // loads without 27 addresses in vector registers
+    const unsigned o = 8u * (unsigned)e;
+    auto ld = [&](const double* base) {
+      return *reinterpret_cast<const double*>(reinterpret_cast<const char*>(base) + o);
+    };
 #pragma unroll
     for (int j = 0; j < CPB; ++j)
 #pragma unroll
-      for (int d = 0; d < 9; ++d) k[j][d] = a.K4[(9 * (c0 + j) + d) * V + e];
+      for (int d = 0; d < 9; ++d) p.k[j][d] = ld(a.K4 + (9 * (c0 + j) + d) * V);
     if constexpr (DIR) {
       const double* R = a.r.p[rhs];
 #pragma unroll
-      for (int d = 0; d < 9; ++d) f[d] = R[d * V + e];
+      for (int d = 0; d < 9; ++d) p.r[d] = ld(R + d * V);
+    }
+#pragma unroll
+    for (int d = 0; d < 9; ++d) p.f[d] = ld(F + d * V);
+  } else {
+#pragma unroll
+    for (int j = 0; j < CPB; ++j) p.f[j] = F[(c0 + j) * a.fs + e];
+  }
+}
+// (K4:F)_c of components c0 .. c0 + CPB at voxel e (or F_c without K4); DIR:
+// F is the new direction r + beta F, its components stored, fc its value there
+template <bool HASK, bool DIR, int CPB>
+__device__ __forceinline__ void use_point(const FwdArgs& a, int rhs, int c0, long e, long V,
+                                          double beta, const Point<HASK, DIR, CPB>& p,
+                                          double (&v)[CPB], double (&fc)[CPB]) {
+  if constexpr (HASK) {
+    double f[9];
+    if constexpr (DIR) {
+#pragma unroll
+      for (int d = 0; d < 9; ++d) f[d] = p.r[d];
       if (beta != 0.0) {
 #pragma unroll
-        for (int d = 0; d < 9; ++d) f[d] = f[d] + beta * F[d * V + e];
+        for (int d = 0; d < 9; ++d) f[d] = f[d] + beta * p.f[d];
       }
     } else {
 #pragma unroll
-      for (int d = 0; d < 9; ++d) f[d] = F[d * V + e];
+      for (int d = 0; d < 9; ++d) f[d] = p.f[d];
     }
 #pragma unroll
     for (int j = 0; j < CPB; ++j) {
-      v[j] = ddot42n_row(k[j], f);
+      v[j] = ddot42n_row(p.k[j], f);
       if constexpr (DIR) {
 #pragma unroll
         for (int d = 0; d < 9; ++d) fc[j] = (d == c0 + j) ? f[d] : fc[j];
@@ -467,17 +507,18 @@ __device__ __forceinline__ void load_point(const FwdArgs& a, int rhs, int c0, lo
     }
   } else {
 #pragma unroll
-    for (int j = 0; j < CPB; ++j) v[j] = F[(c0 + j) * a.fs + e];
+    for (int j = 0; j < CPB; ++j) v[j] = p.f[j];
   }
 }
 
 // The points e0 + p, p < npts, of a run (line p / N, z = p mod N) into the
 // line pairs of buf; DIR: the sums of v fc to pq[j * pqs] (each thread its
-// points in turn, then the block).  Ends synchronised.
-template <int NC, bool HASK, bool DIR, int CPB>
+// points in turn, then the block).  pt: with AHEAD the operands of point tid,
+// already fetched.  Ends synchronised.
+template <int NC, bool HASK, bool DIR, int CPB, bool AHEAD>
 __device__ __forceinline__ void load_lines(const Grid& g, const FwdArgs& a, int rhs, int c0,
                                            long e0, int npts, int nl, double beta, cplx* buf,
-                                           double* pq, long pqs) {
+                                           double* pq, long pqs, Point<HASK, DIR, CPB>& pt) {
   __shared__ double wsum[CPB][16];
   const int N = edge<NC>(g), LS = N | 1, LP = (nl + 1) >> 1, T = blockDim.x, tid = threadIdx.x;
   const Div dN = divN<NC>(g);
@@ -487,7 +528,9 @@ __device__ __forceinline__ void load_lines(const Grid& g, const FwdArgs& a, int 
   for (int j = 0; j < CPB; ++j) acc[j] = 0.0;
   for (int p = tid; p < npts; p += T) {
     double v[CPB], fc[CPB];
-    load_point<HASK, DIR, CPB>(a, rhs, c0, e0 + p, g.V, beta, v, fc);
+    if (!AHEAD) fetch_point<HASK, DIR, CPB>(a, rhs, c0, e0 + p, g.V, pt);
+    use_point<HASK, DIR, CPB>(a, rhs, c0, e0 + p, g.V, beta, pt, v, fc);
+    if (AHEAD && p + T < npts) fetch_point<HASK, DIR, CPB>(a, rhs, c0, e0 + p + T, g.V, pt);
     const int l = dN(p), z = p - l * N;
 #pragma unroll
     for (int j = 0; j < CPB; ++j) {
@@ -648,23 +691,27 @@ __device__ __forceinline__ void form_alpha(const MidArgs& a, int rhs) {
 // contraction in it the kernel is slower than fft_pencil.hip's pass A from
 // 64^3 on (56 against 41 us), where the F of the slabs in flight outgrows an
 // XCD's L2.
-template <int NC, int ME, bool HASK, bool DIR>
+template <int NC, int ME, bool HASK, bool DIR, bool AHEAD>
 __global__ __launch_bounds__(1024) void k_fwd(Grid g, FwdArgs a) {
   extern __shared__ cplx lds[];
   const Where w = where<1>(a.nrhs);
   const int N = edge<NC>(g), LS = N | 1, NN = N * N, T = blockDim.x, tid = threadIdx.x;
   if (w.tile >= N) return;
-  if (!DIR && a.old && a.old[w.rhs].done) return;
   const int x = w.tile, nzk = g.nzk, LP = (N + 1) >> 1;
   cplx* tw = lds;
   cplx* buf = lds + N;
+  Point<HASK, DIR, 1> pt;
+  if (AHEAD && tid < NN) fetch_point<HASK, DIR, 1>(a, w.rhs, w.c0, (long)x * NN + tid, g.V, pt);
   load_tw<NC>(tw, a.tw, N);
   double beta = 0.0;
   if constexpr (DIR) {
     if (cg_begin(a, w.rhs, x == 0 && w.c0 == 0, beta)) return;
+  } else {
+    if (a.old && a.old[w.rhs].done) return;
   }
-  load_lines<NC, HASK, DIR, 1>(g, a, w.rhs, w.c0, (long)x * NN, NN, N, beta, buf,
-                               DIR && a.pqp ? a.pqp + ((long)w.rhs * 9 + w.c0) * N + x : nullptr, N);
+  load_lines<NC, HASK, DIR, 1, AHEAD>(g, a, w.rhs, w.c0, (long)x * NN, NN, N, beta, buf,
+                               DIR && a.pqp ? a.pqp + ((long)w.rhs * 9 + w.c0) * N + x : nullptr, N,
+                               pt);
   auto lb = [&](int l) { return l * LS; };
   fft<NC, true, ME>(buf, tw, g, LP, lb, 1);
   {
@@ -888,15 +935,17 @@ __global__ __launch_bounds__(256) void k_zf(Grid g, FwdArgs a) {
   const int L0 = w.tile * g.TL, nl = min(g.TL, g.NN - L0), LP = (nl + 1) >> 1;
   cplx* tw = lds;
   cplx* buf = lds + N;
-  load_tw<0>(tw, a.tw, N);
+  Point<HASK, DIR, CPB> pt;
+  load_tw<kAnyRadix>(tw, a.tw, N);
   double beta = 0.0;
   if constexpr (DIR) {
     if (cg_begin(a, w.rhs, w.tile == 0 && w.c0 == 0, beta)) return;
   }
-  load_lines<0, HASK, DIR, CPB>(
+  load_lines<kAnyRadix, HASK, DIR, CPB, false>(
       g, a, w.rhs, w.c0, (long)L0 * N, nl * N, nl, beta, buf,
-      DIR && a.pqp ? a.pqp + ((long)w.rhs * 9 + w.c0) * g.nzb + w.tile : nullptr, g.nzb);
-  fft<0, true, kMaxE>(buf, tw, g, CPB * LP, [&](int l) { return l * LS; }, 1);
+      DIR && a.pqp ? a.pqp + ((long)w.rhs * 9 + w.c0) * g.nzb + w.tile : nullptr, g.nzb,
+      pt);
+  fft<kAnyRadix, true, kMaxE>(buf, tw, g, CPB * LP, [&](int l) { return l * LS; }, 1);
   const Div dLP(LP);
 #pragma unroll
   for (int j = 0; j < CPB; ++j) {
@@ -924,7 +973,7 @@ __global__ __launch_bounds__(256) void k_y(Grid g, MidArgs a) {
   const int N = g.N, LS = N | 1, x0 = blockIdx.x * kTX, nx = min(kTX, N - x0);
   cplx* tw = lds;
   cplx* buf = lds + N;
-  load_tw<0>(tw, a.tw, N);
+  load_tw<kAnyRadix>(tw, a.tw, N);
   const long plane = rhs * a.ts + ((long)c * g.NZ + kz) * g.NN;
   const Div dnx(nx);
   if constexpr (FWD) {
@@ -939,7 +988,7 @@ __global__ __launch_bounds__(256) void k_y(Grid g, MidArgs a) {
     }
   }
   __syncthreads();
-  fft<0, FWD, kMaxE>(buf, tw, g, nx, [&](int l) { return l * LS; }, 1);
+  fft<kAnyRadix, FWD, kMaxE>(buf, tw, g, nx, [&](int l) { return l * LS; }, 1);
   if constexpr (FWD) {
     for (int i = threadIdx.x; i < nx * N; i += 256) {
       const int y = dnx(i), t = i - y * nx;
@@ -968,7 +1017,7 @@ __global__ __launch_bounds__(256) void k_x(Grid g, MidArgs a) {
   const int N = g.N, LS = N | 1, YB = x_lines(N), y0 = blockIdx.x * YB, ny = min(YB, N - y0);
   cplx* tw = lds;
   cplx* buf = lds + N;
-  load_tw<0>(tw, a.tw, N);
+  load_tw<kAnyRadix>(tw, a.tw, N);
   const long cst = (long)g.NZ * g.NN;
   cplx* T2 = a.T2 + rhs * a.ts + ((long)(3 * row) * g.NZ + kz) * g.NN + (long)y0 * N;
 #pragma unroll
@@ -979,7 +1028,7 @@ __global__ __launch_bounds__(256) void k_x(Grid g, MidArgs a) {
     }
   __syncthreads();
   auto lb = [&](int l) { return l * LS; };
-  fft<0, true, kMaxE>(buf, tw, g, 3 * ny, lb, 1);
+  fft<kAnyRadix, true, kMaxE>(buf, tw, g, 3 * ny, lb, 1);
   if (a.dc && kz == 0 && y0 == 0) {
     if (threadIdx.x < 3) a.dc[9 * rhs + 3 * row + threadIdx.x] = buf[threadIdx.x * ny * LS].re;
     __syncthreads();
@@ -995,7 +1044,7 @@ __global__ __launch_bounds__(256) void k_x(Grid g, MidArgs a) {
     b[2 * ny * LS] = o[2];
   }
   __syncthreads();
-  fft<0, false, kMaxE>(buf, tw, g, 3 * ny, lb, 1);
+  fft<kAnyRadix, false, kMaxE>(buf, tw, g, 3 * ny, lb, 1);
 #pragma unroll
   for (int c = 0; c < 3; ++c)
     for (int i = threadIdx.x; i < ny * N; i += 256) {
@@ -1015,7 +1064,7 @@ __global__ __launch_bounds__(256) void k_zi(Grid g, InvArgs a) {
   const long e0 = (long)L0 * N + c * g.V;
   cplx* tw = lds;
   cplx* buf = lds + N;
-  load_tw<0>(tw, a.tw, N);
+  load_tw<kAnyRadix>(tw, a.tw, N);
   const cplx* T1 = a.T1 + rhs * a.ts + (long)c * g.NZ * g.NN + L0;
   const Div dLP(LP);
   for (int q = tid; q < LP * g.nzk; q += 256) {
@@ -1029,8 +1078,8 @@ __global__ __launch_bounds__(256) void k_zi(Grid g, InvArgs a) {
 #pragma unroll
   for (int j = 0; j < 2; ++j) fetch<MODE>(a, rhs, e0 + tid + j * 256, tid + j * 256 < npts, j, f);
   __syncthreads();
-  fft<0, false, 4>(buf, tw, g, LP, [&](int l) { return l * LS; }, 1);
-  store_lines<0, MODE>(g, a, rhs, e0, npts, buf, f,
+  fft<kAnyRadix, false, 4>(buf, tw, g, LP, [&](int l) { return l * LS; }, 1);
+  store_lines<kAnyRadix, MODE>(g, a, rhs, e0, npts, buf, f,
                        a.part + ((long)rhs * 9 + c) * g.nzb + tile);
 }
 
@@ -1083,9 +1132,17 @@ static Grid make_grid(const SpecGeom& s) {
 }
 
 static int up64(int n) { return (n + 63) / 64 * 64; }
+// Threads of the slab kernels.  The transforms need a quarter of the half
+// spectrum's elements (candidate kFew); a lone system's blocks do not fill
+// the chip, and each thread waits for its voxels one after the other, so up
+// to 512 threads take one each (solve 32^3 1.33 -> 1.20 ms, 45^3 3.21 -> 3.14;
+// 768 are slower: one block a CU).  Several systems with the contraction in
+// the kernel keep the few: their blocks fill the chip and 384 or 512 threads
+// are fewer waves (nine at 32^3: 3.3 ms with 192 threads, 3.9 with 512).
+constexpr int kFew = -1;
 static int slab_threads(int N, int i) {
   const int t = std::min(1024, up64((N * (N / 2 + 1) + 3) / 4));
-  return i == 1 ? std::min(1024, 2 * t) : t;
+  return i == kFew ? t : i == 1 ? std::min(1024, 2 * t) : std::max(t, std::min(512, up64(N * N)));
 }
 static int mid_threads(int N, int i) { return up64(3 * kML * N / (N < 32 || i == 1 ? 2 : 4)) * (N < 32 && i == 1 ? 2 : 1); }
 // elements per thread the runtime plans allow for: four up to edge 88
@@ -1103,9 +1160,16 @@ static size_t lds_lines(int N, int lines) {
   return ((size_t)N + (size_t)lines * (N | 1)) * sizeof(cplx);
 }
 
+// The first point's operands ahead of the rest need some 40 registers more:
+// for a lone system, where a block's own latency counts (16^3 0.75 -> 0.69 ms);
+// several systems' blocks do better with more waves a SIMD (nine at 32^3 3.28
+// against 3.38), and radices 11 and 13 leave no registers for it.
 template <int NC, int ME, bool HASK, bool DIR>
 static void fwd_slab(const Grid& g, const FwdArgs& a, int threads, hipStream_t s) {
-  auto k = k_fwd<NC, ME, HASK, DIR>;
+  auto k = k_fwd<NC, ME, HASK, DIR, false>;
+  if constexpr (HASK && NC != kAnyRadix) {
+    if (a.nrhs == 1) k = k_fwd<NC, ME, HASK, DIR, true>;
+  }
   const size_t lds = lds_slab(g.N);
   allow_lds(k, lds);
   k<<<8 * ((g.N + 7) / 8) * 9 * a.nrhs, threads, lds, s>>>(g, a);
@@ -1114,11 +1178,11 @@ static void fwd_slab(const Grid& g, const FwdArgs& a, int threads, hipStream_t s
 template <int NC, bool HASK, bool DIR>
 static void forward(const Grid& g, const FwdArgs& a, int cand, hipStream_t s) {
   const int t = slab_threads(g.N, cand);
-  if (NC == 0 && g.N > kSlabN) {
+  if (NC == kAnyRadix && g.N > kSlabN) {
     k_zf<HASK, DIR><<<8 * ((g.nzb + 7) / 8) * 3 * a.nrhs, 256,
                       lds_lines(g.N, 3 * (g.TL / 2)), s>>>(g, a);
-  } else if (NC == 0 && g.N > kE4N) {
-    fwd_slab<0, kMaxE, HASK, DIR>(g, a, t, s);
+  } else if (NC <= 0 && g.N > kE4N) {
+    fwd_slab<NC, kMaxE, HASK, DIR>(g, a, t, s);
   } else {
     fwd_slab<NC, NC == 96 ? 5 : 4, HASK, DIR>(g, a, t, s);
   }
@@ -1126,11 +1190,11 @@ static void forward(const Grid& g, const FwdArgs& a, int cand, hipStream_t s) {
 
 template <int NC>
 static void middle(const Grid& g, const MidArgs& a, int nrhs, int cand, hipStream_t s) {
-  if (NC > 0 || g.N <= kSlabN) {
+  if (NC != kAnyRadix || g.N <= kSlabN) {
     const int tiles = (g.nzk * g.N + kML - 1) / kML;
     k_mid<NC><<<dim3(tiles + (a.pqp ? 1 : 0), 3, nrhs), mid_threads(g.N, cand),
                 lds_lines(g.N, 3 * kML), s>>>(g, a);
-  } else if constexpr (NC == 0) {
+  } else if constexpr (NC == kAnyRadix) {
     const int yb = x_lines(g.N);
     if (a.pqp) launch_cg_alpha(a.pqp, a.npq, a.cs, s, nrhs, a.npq);
     const dim3 gy((g.N + kTX - 1) / kTX, g.nzk, 9 * nrhs);
@@ -1150,10 +1214,10 @@ static void inv_slab(const Grid& g, const InvArgs& a, int nrhs, int threads, hip
 template <int NC, int MODE>
 static void inverse(const Grid& g, const InvArgs& a, int nrhs, int cand, hipStream_t s) {
   const int t = slab_threads(g.N, cand);
-  if (NC == 0 && g.N > kSlabN)
+  if (NC == kAnyRadix && g.N > kSlabN)
     k_zi<MODE><<<dim3(g.nzb, 9, nrhs), 256, lds_lines(g.N, g.TL / 2), s>>>(g, a);
-  else if (NC == 0 && g.N > kE4N)
-    inv_slab<0, kMaxE, MODE>(g, a, nrhs, t, s);
+  else if (NC <= 0 && g.N > kE4N)
+    inv_slab<NC, kMaxE, MODE>(g, a, nrhs, t, s);
   else
     inv_slab<NC, NC == 96 ? 5 : 4, MODE>(g, a, nrhs, t, s);
 }
@@ -1198,6 +1262,7 @@ static void run_cg(const SpecGeom& sg, const GridCG& c, int part, hipStream_t s)
   const Grid g = make_grid(sg);
   const int np = 9 * g.nzb;
   const bool plain = c.out[0] != nullptr;  // p.q from the inverse pass
+  const int ct = c.nrhs > 1 && !c.q[0] ? kFew : 0;
   Args a(g, c.K4, c.spec, c.tw, c.nrhs);
   for (int k = 0; k < c.nrhs; ++k) {
     a.f.F.p[k] = c.p_old[k];
@@ -1224,11 +1289,11 @@ static void run_cg(const SpecGeom& sg, const GridCG& c, int part, hipStream_t s)
       for (int k = 0; k < c.nrhs; ++k) a.f.F.p[k] = const_cast<double*>(c.q[k]);
       forward<NC, false, false>(g, a.f, sg.tune.a0, s);
     } else {
-      forward<NC, true, true>(g, a.f, 0, s);
+      forward<NC, true, true>(g, a.f, ct, s);
     }
     middle<NC>(g, a.m, c.nrhs, sg.tune.c, s);
   } else if (plain) {
-    inverse<NC, 1>(g, a.i, c.nrhs, 0, s);
+    inverse<NC, 1>(g, a.i, c.nrhs, ct, s);
     StepArgs t{};
     t.p = a.i.pd;
     t.q = a.i.out;
@@ -1240,7 +1305,7 @@ static void run_cg(const SpecGeom& sg, const GridCG& c, int part, hipStream_t s)
     t.rrp = c.rr;
     k_step<<<dim3(a.f.nrr, c.nrhs), 256, 0, s>>>(9 * g.V, t);
   } else {
-    inverse<NC, 2>(g, a.i, c.nrhs, 0, s);
+    inverse<NC, 2>(g, a.i, c.nrhs, ct, s);
   }
 }
 
@@ -1289,7 +1354,12 @@ bool gkdf_grid_edge(int N) { return !(N == 64 || N == 96 || N == 128 || N == 256
     case 48: gp::call<48> CPFFT_ARGS; break; \
     case 64: gp::call<64> CPFFT_ARGS; break; \
     case 96: gp::call<96> CPFFT_ARGS; break; \
-    default: gp::call<0> CPFFT_ARGS; break;  \
+    default:                        \
+      if (gp::smooth(g.N))          \
+        gp::call<gp::kSmooth> CPFFT_ARGS; \
+      else                          \
+        gp::call<gp::kAnyRadix> CPFFT_ARGS; \
+      break;                        \
   }
 
 void launch_gkdf_grid(const SpecGeom& g, const double* F, const double* K4, double* out,
