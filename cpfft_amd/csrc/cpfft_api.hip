@@ -10,6 +10,7 @@
 #include <mutex>
 #include <random>
 #include <string>
+#include <thread>
 #include <tuple>
 #include <vector>
 
@@ -72,6 +73,12 @@ struct cpfft_ctx {
   double* hm = nullptr;
   double* hpq = nullptr;  // p_i . (K4:p_i) block sums of the K4 pass [9][blocks]
   double* f2d_cos = nullptr;  // cosine table of cpfft_f2disp
+  // pinned staging of copy_out: kStages pieces of kStageBytes, allocated at
+  // its first use, and an event for each
+  static constexpr int kStages = 4;
+  static constexpr size_t kStageBytes = size_t(1) << 20;
+  char* stage = nullptr;
+  hipEvent_t stage_ev[kStages] = {};
   CGScalars* hcg9 = nullptr;
   // learned warm start
   MlpBuffers mlp;
@@ -165,6 +172,9 @@ extern "C" int cpfft_destroy(cpfft_ctx* c) {
   if (c->hm) (void)hipFree(c->hm);
   if (c->hpq) (void)hipFree(c->hpq);
   if (c->f2d_cos) (void)hipFree(c->f2d_cos);
+  if (c->stage) (void)hipHostFree(c->stage);
+  for (hipEvent_t e : c->stage_ev)
+    if (e) (void)hipEventDestroy(e);
   {
     MlpBuffers& b = c->mlp;
     void* mb[] = {b.params, b.pbf, b.grads, b.m, b.v, b.norm, b.logX, b.logT, b.Xf, b.Tb, b.Y,
@@ -489,6 +499,73 @@ extern "C" int cpfft_mean9(cpfft_ctx* c, const double* x, double out[9]) {
   return 0;
 }
 
+// Device memory to the caller's pageable memory on the context's stream,
+// through pinned pieces that kStages threads copy on while the next arrive.
+// cpfft_f2disp as a whole takes 0.39 ms at 64^3 (6.6 MB) and 3.2 at 128^3
+// (52 MB); with one thread 0.42 and 5.3, with the runtime's own copy to
+// pageable memory 0.56 and 6.1.  Up to a quarter of a piece that copy is as fast.
+static int copy_out(cpfft_ctx* c, void* dst, const void* src, size_t bytes) {
+  constexpr int S = cpfft_ctx::kStages;
+  constexpr size_t B = cpfft_ctx::kStageBytes;
+  bool staged = bytes > B / 4;
+  if (staged && !c->stage && hipHostMalloc(&c->stage, S * B, hipHostMallocDefault) != hipSuccess) {
+    c->stage = nullptr;
+    staged = false;
+    (void)hipGetLastError();
+  }
+  for (int i = 0; staged && i < S; ++i)
+    if (!c->stage_ev[i] &&
+        hipEventCreateWithFlags(&c->stage_ev[i], hipEventDisableTiming) != hipSuccess) {
+      c->stage_ev[i] = nullptr;
+      staged = false;
+      (void)hipGetLastError();
+    }
+  if (!staged) {
+    HIP_OK(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, c->stream));
+    HIP_OK(hipStreamSynchronize(c->stream));
+    return 0;
+  }
+  const long n = (long)((bytes + B - 1) / B);
+  auto size = [&](long k) { return std::min(B, bytes - (size_t)k * B); };
+  auto ask = [&](long k) {
+    hipError_t e = hipMemcpyAsync(c->stage + (k % S) * B, (const char*)src + (size_t)k * B, size(k),
+                                  hipMemcpyDeviceToHost, c->stream);
+    return e == hipSuccess ? hipEventRecord(c->stage_ev[k % S], c->stream) : e;
+  };
+  for (long k = 0; k < std::min<long>(S, n); ++k) HIP_OK(ask(k));
+  // worker w: the pieces w, w + S, ... through stage w
+  int dev = 0;
+  HIP_OK(hipGetDevice(&dev));
+  std::array<hipError_t, S> err;
+  err.fill(hipSuccess);
+  auto work = [&](int w) {
+    hipError_t e = hipSetDevice(dev);
+    for (long k = w; e == hipSuccess && k < n; k += S) {
+      if ((e = hipEventSynchronize(c->stage_ev[w])) != hipSuccess) break;
+      memcpy((char*)dst + (size_t)k * B, c->stage + w * B, size(k));
+      if (k + S < n) e = ask(k + S);
+    }
+    err[w] = e;
+  };
+  const int nw = (int)std::min<long>(S, n);
+  std::array<std::thread, S> th;
+  for (int w = 1; w < nw; ++w) {
+    try {
+      th[w] = std::thread(work, w);
+    } catch (...) {  // no thread to be had: done below
+    }
+  }
+  work(0);
+  for (int w = 1; w < nw; ++w) {
+    if (th[w].joinable())
+      th[w].join();
+    else
+      work(w);
+  }
+  for (hipError_t e : err) HIP_OK(e);
+  return 0;
+}
+
 // f2disp (f2disp.f:16-175): the spectrum buffers (2 * 9 * S1 complex) hold
 // the right-hand side, the transforms and u before the copy to the host
 extern "C" int cpfft_f2disp(cpfft_ctx* c, const double* F, const double lengths[3], double* u) {
@@ -506,14 +583,12 @@ extern "C" int cpfft_f2disp(cpfft_ctx* c, const double* F, const double lengths[
     launch_f2disp_cos(N, c->f2d_cos, c->stream);
   }
   double* work = reinterpret_cast<double*>(c->spec);
-  // the last transform leaves x in the first half of the scratch, so u
-  // goes to the second
-  double* ud = work + 3 * P3;
+  // the last transform leaves x in the second half of the scratch, so u
+  // goes to the first
+  double* ud = work;
   launch_f2disp(N, F, lengths, c->f2d_cos, work, ud, c->stream);
   HIP_OK(hipGetLastError());
-  HIP_OK(hipMemcpyAsync(u, ud, 3 * P3 * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-  HIP_OK(hipStreamSynchronize(c->stream));
-  return 0;
+  return copy_out(c, u, ud, 3 * P3 * sizeof(double));
 }
 
 // CG iterations enqueued per host round trip
