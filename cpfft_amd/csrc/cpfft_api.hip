@@ -1039,7 +1039,7 @@ static void enqueue_homo_slab(cpfft_ctx* c) {
     rr.r[i] = c->th[1][i];
   }
   for (int j = 0; j < kChunk; ++j) {
-    launch_k4_contract_multi(V, c->fields[CPFFT_K4], pp, c->dcg9, 9, c->stream, &rr,
+    launch_k4_contract_multi(V, c->fields[CPFFT_K4], pp, c->dcg9, 9, c->stream, rr,
                              pr ? c->hpq : nullptr);
     for (int i0 = 0; i0 < 9; i0 += c->homo_group) {
       GridCG k{};
@@ -1127,7 +1127,7 @@ static void enqueue_homo_chunk(cpfft_ctx* c) {
   const int nb = k4_contract_multi_blocks(V);
   const double sc = 1.0 / (double)V;
   for (int j = 0; j < kChunk; ++j) {
-    launch_k4_contract_multi(V, K4, pp, c->dcg9, 9, c->stream, &rr, apq ? c->hpq : nullptr);
+    launch_k4_contract_multi(V, K4, pp, c->dcg9, 9, c->stream, rr, apq ? c->hpq : nullptr);
     // the nine alphas in one launch (one block per right-hand side)
     if (apq) launch_cg_alpha(c->hpq, nb, c->dcg9, c->stream, 9, nb);
     for (int i = 0; i < 9; ++i) {

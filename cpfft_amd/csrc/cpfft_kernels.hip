@@ -364,7 +364,7 @@ void launch_cg_check(const double* part, int np, CGScalars* cs, hipStream_t s, c
 // ------------------------------------------ multi-RHS K4 contraction
 // q_i = K4 : p_i for the right-hand sides i < nrhs whose solve is still
 // running (tangent_homo's nine solves share K4, which is read once).
-template <bool DIR>
+// First p_i = r_i + beta p_i.
 __global__ __launch_bounds__(kBlock) void k_k4_contract_multi(long V, const double* __restrict__ K4,
                                                               Ptr9 pp, const CGScalars* __restrict__ cs,
                                                               int nrhs, Ptr9r rr,
@@ -385,7 +385,7 @@ __global__ __launch_bounds__(kBlock) void k_k4_contract_multi(long V, const doub
   auto load = [&](int i, double (&r9)[9], double (&p9)[9]) {
 #pragma unroll
     for (int c = 0; c < 9; ++c) {
-      if (DIR) r9[c] = valid ? __builtin_nontemporal_load(rr.r[i] + c * V + e) : 0.0;
+      r9[c] = valid ? __builtin_nontemporal_load(rr.r[i] + c * V + e) : 0.0;
       p9[c] = valid ? __builtin_nontemporal_load(pp.p[i] + c * V + e) : 0.0;
     }
   };
@@ -398,18 +398,13 @@ __global__ __launch_bounds__(kBlock) void k_k4_contract_multi(long V, const doub
     if (i + 1 < 9 && running(i + 1)) load(i + 1, rb[(i + 1) & 1], pb[(i + 1) & 1]);
     if (!running(i)) continue;
     double f[9];
-    if (DIR) {
-      const double beta = cs[i].beta;
-      double* pw = const_cast<double*>(pp.p[i]);
+    const double beta = cs[i].beta;
+    double* pw = const_cast<double*>(pp.p[i]);
 #pragma unroll
-      for (int c = 0; c < 9; ++c) {
-        // (the first direction is r, whatever p holds)
-        f[c] = beta == 0.0 ? rb[i & 1][c] : rb[i & 1][c] + beta * pb[i & 1][c];
-        if (valid) __builtin_nontemporal_store(f[c], pw + c * V + e);
-      }
-    } else {
-#pragma unroll
-      for (int c = 0; c < 9; ++c) f[c] = pb[i & 1][c];
+    for (int c = 0; c < 9; ++c) {
+      // (the first direction is r, whatever p holds)
+      f[c] = beta == 0.0 ? rb[i & 1][c] : rb[i & 1][c] + beta * pb[i & 1][c];
+      if (valid) __builtin_nontemporal_store(f[c], pw + c * V + e);
     }
     double pq = 0.0;
 #pragma unroll
@@ -436,12 +431,9 @@ __global__ __launch_bounds__(kBlock) void k_k4_contract_multi(long V, const doub
 int k4_contract_multi_blocks(long V) { return (int)((V + kBlock - 1) / kBlock); }
 
 void launch_k4_contract_multi(long V, const double* K4, const Ptr9& pp, const CGScalars* cs,
-                              int nrhs, hipStream_t s, const Ptr9r* rr, double* pqpart) {
-  const unsigned g = (unsigned)k4_contract_multi_blocks(V);
-  if (rr)
-    k_k4_contract_multi<true><<<g, kBlock, 0, s>>>(V, K4, pp, cs, nrhs, *rr, pqpart);
-  else
-    k_k4_contract_multi<false><<<g, kBlock, 0, s>>>(V, K4, pp, cs, nrhs, Ptr9r{}, pqpart);
+                              int nrhs, hipStream_t s, const Ptr9r& rr, double* pqpart) {
+  k_k4_contract_multi<<<(unsigned)k4_contract_multi_blocks(V), kBlock, 0, s>>>(V, K4, pp, cs, nrhs,
+                                                                              rr, pqpart);
 }
 
 // ------------------------------------------------------- stress update

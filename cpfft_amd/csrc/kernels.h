@@ -182,15 +182,15 @@ struct Ptr9 {
   const double* p[9];
   double* q[9];
 };
-// q_i = K4 : p_i (ddot42n) for every i < nrhs with cs[i].done == 0; with
-// r != nullptr the direction is first updated, p_i = r_i + cs[i].beta p_i
+// for every i < nrhs with cs[i].done == 0: the direction p_i = r_i +
+// cs[i].beta p_i, then q_i = K4 : p_i (ddot42n)
 struct Ptr9r {
   const double* r[9];
 };
 // pqpart != nullptr: also p_i . (K4:p_i) of each running right-hand side,
 // per block, at pqpart[i * k4_contract_multi_blocks(V) + block].
 void launch_k4_contract_multi(long V, const double* K4, const Ptr9& pp, const CGScalars* cs,
-                              int nrhs, hipStream_t s, const Ptr9r* rr = nullptr,
+                              int nrhs, hipStream_t s, const Ptr9r& rr,
                               double* pqpart = nullptr);
 int k4_contract_multi_blocks(long V);
 
