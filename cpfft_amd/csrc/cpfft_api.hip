@@ -915,12 +915,17 @@ extern "C" int cpfft_pcg(cpfft_ctx* c, const double* b, double* x, double tol, i
     }
   }
   int launched = 0;
+  // the events of this solve follow the first ev0[f] of family f
+  int ev0[cpfft_ctx::kFam];
+  std::copy(c->ev_n, c->ev_n + cpfft_ctx::kFam, ev0);
   for (;;) {
     if (graph) {
       HIP_OK(hipGraphLaunch(ge, c->stream));
     } else {
-      if (c->timing && (c->ev_n[0] + kChunk > cpfft_ctx::kRing || c->ev_n[2] + kChunk > cpfft_ctx::kRing))
+      if (c->timing && (c->ev_n[0] + kChunk > cpfft_ctx::kRing || c->ev_n[2] + kChunk > cpfft_ctx::kRing)) {
         flush_events(c);
+        std::fill(ev0, ev0 + cpfft_ctx::kFam, 0);
+      }
       enqueue_pcg_chunk(c, x, launched);
     }
     launched += kChunk;
@@ -930,16 +935,10 @@ extern "C" int cpfft_pcg(cpfft_ctx* c, const double* b, double* x, double tol, i
     if (c->hcg->done) break;
   }
   const int k = c->hcg->k;
-  if (c->hcg->done == 3) {  // zero right-hand side
-    if (c->timing)
-      for (int f : {0, 2}) {
-        while (c->ev_n[f] > 0 && c->ev_it[f][c->ev_n[f] - 1] >= 0) c->ev_n[f]--;
-      }
-    return 1;
-  }
   if (c->timing)  // drop the events of the no-op iterations at the end
     for (int f : {0, 2})
-      while (c->ev_n[f] > 0 && c->ev_it[f][c->ev_n[f] - 1] >= k) c->ev_n[f]--;
+      while (c->ev_n[f] > ev0[f] && c->ev_it[f][c->ev_n[f] - 1] >= k) c->ev_n[f]--;
+  if (c->hcg->done == 3) return 1;  // zero right-hand side
   c->cg_iters += k;
   c->gkdf_calls += k;
   if (iters) *iters = k;

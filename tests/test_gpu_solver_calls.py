@@ -1,0 +1,40 @@
+"""GPU tests of what the solver's calls leave behind beside their results: the
+recorded kernel times, the time of a solve with nothing to do, the device
+memory a context holds, and the launch shapes it reports."""
+import numpy as np
+import pytest
+
+import cpfft_amd as C
+from cpfft_amd.microstructure import polycrystal
+
+pytestmark = pytest.mark.gpu
+
+
+def _solver(N, mode=1):
+    _, ang = polycrystal(N, 4, 5 * N)
+    return C.Solver(N, ang, C.Material(), dt=0.25, gamma_mode=mode)
+
+
+def _rhs(s, seed):
+    """tangent of the explicit update in K4, a right-hand side in B"""
+    s.drive_eps_sig(1, 0)
+    rng = np.random.default_rng(seed)
+    s.upload(C.DFM, 1e-3 * rng.standard_normal((9, s.V)))
+    s.gkdf(C.DFM, C.B, 1)
+    s.dscal(-1.0, C.B)
+
+
+@pytest.mark.parametrize("N,mode", [(16, 1), (9, 0), (64, 1)])
+def test_zero_right_hand_side_keeps_recorded_times(N, mode):
+    """a solve with nothing to do records nothing and drops nothing"""
+    s = _solver(N, mode)
+    _rhs(s, N)
+    s.set_timing(1)
+    rc, it, _ = s.pcg(C.B, C.WORK, 1e-8)
+    assert rc == 0 and it > 0
+    s.fill9(C.B, np.zeros(9))
+    assert s.pcg(C.B, C.WORK, 1e-8) == (1, 0, 0.0)
+    assert not s.download(C.WORK).any()
+    _, cnt = s.kernel_times()
+    assert cnt[0] == it and cnt[2] == it
+    s.close()
