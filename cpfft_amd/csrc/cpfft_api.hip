@@ -6,6 +6,7 @@
 
 #include <algorithm>
 #include <array>
+#include <chrono>
 #include <map>
 #include <mutex>
 #include <random>
@@ -62,6 +63,9 @@ struct cpfft_ctx {
   double* hres = nullptr;  // pinned host mirror
   CGScalars* dcg = nullptr;  // device scalars of the running CG solve (two, see enqueue_pcg_grid)
   CGScalars* hcg = nullptr;  // pinned host mirror
+  // what launch_cg_init of the solve number cg_seq says of its right-hand side (zero_rhs)
+  long long* hzero = nullptr;
+  long long cg_seq = 0;
   // tangent_homo's nine simultaneous solves: x, r, p, q per right-hand side
   double* th[4][9] = {};
   CGScalars* dcg9 = nullptr;
@@ -161,6 +165,7 @@ extern "C" int cpfft_destroy(cpfft_ctx* c) {
     if (b) (void)hipFree(b);
   if (c->hres) (void)hipHostFree(c->hres);
   if (c->hcg) (void)hipHostFree(c->hcg);
+  if (c->hzero) (void)hipHostFree(c->hzero);
   if (c->hcg9) (void)hipHostFree(c->hcg9);
   if (c->hcnt) (void)hipHostFree(c->hcnt);
   if (c->hhm) (void)hipHostFree(c->hhm);
@@ -282,6 +287,8 @@ extern "C" int cpfft_create(int N, const cpfft_material* m, const double* angles
   HIP_OK(hipHostMalloc(&c->hres, 16 * sizeof(double), hipHostMallocDefault));
   HIP_OK(hipMalloc(&c->dcg, 2 * sizeof(CGScalars)));
   HIP_OK(hipHostMalloc(&c->hcg, sizeof(CGScalars), hipHostMallocDefault));
+  HIP_OK(hipHostMalloc(&c->hzero, sizeof(long long), hipHostMallocCoherent));
+  *c->hzero = 0;
   for (int a = 0; a < 4; ++a)
     for (int i = 0; i < 9; ++i) HIP_OK(hipMalloc(&c->th[a][i], 9 * V * sizeof(double)));
   HIP_OK(hipMalloc(&c->dcg9, 18 * sizeof(CGScalars)));
@@ -600,6 +607,26 @@ static constexpr int kChunk = 8;
 // reference's example deck, the two differ in the iterations they spend there.)
 static bool projection(const cpfft_ctx* c) { return c->geom.gamma_mode == 1; }
 
+// Whether the running solve's right-hand side vanishes, which k_cg_init tells
+// the host.  Not known in 10 ms (the stream has earlier work to do): no.  With
+// all of a chunk's kernels enqueued, such a solve took 75 (a graph) or 107 to
+// 129 us at 16^3 and 330 at 130^3; asked here, 27 to 30 and 122.
+static bool zero_rhs(const cpfft_ctx* c) {
+  const auto t0 = std::chrono::steady_clock::now();
+  for (;;) {
+    const long long v = __atomic_load_n(c->hzero, __ATOMIC_RELAXED);
+    if (v >> 1 == c->cg_seq) return v & 1;
+    if (std::chrono::steady_clock::now() - t0 > std::chrono::milliseconds(10)) return false;
+    std::this_thread::yield();
+  }
+}
+
+// The iteration before which a solve asks: up to 60^3 the second, so that the
+// device has the first one to do while the host waits; above, where the few
+// microseconds it idles are below 0.2% of a solve, the first, which spares the
+// empty kernels of an iteration (64^3: 66 us with them).
+static int zero_at(const cpfft_ctx* c) { return c->N <= 60 ? 1 : 0; }
+
 // kChunk CG iterations on fft_grid.hip's edges.  The convergence test of an
 // iteration is part of the next one's first kernel where grid_fused_check
 // says so; blocks then read the old state while one of them writes the new,
@@ -607,8 +634,9 @@ static bool projection(const cpfft_ctx* c) { return c->geom.gamma_mode == 1; }
 // holds it between chunks) and the chunk ends with a test of its own.  The
 // direction alternates between two fields for the same reason: blocks read
 // all of the old one to form their component of the new.
+// watch: as enqueue_pcg_chunk
 static_assert(kChunk % 2 == 0, "the state ends a chunk where it began");
-static void enqueue_pcg_grid(cpfft_ctx* c, double* x, int base) {
+static void enqueue_pcg_grid(cpfft_ctx* c, double* x, int base, bool watch) {
   const bool pr = projection(c), fchk = grid_fused_check(c->N);
   const int np = grid_rr_parts(c->N, pr);
   double* pd[2] = {c->p, pr ? c->q : c->tmp9};
@@ -624,6 +652,7 @@ static void enqueue_pcg_grid(cpfft_ctx* c, double* x, int base) {
   k.pq = c->dpart;
   k.rr = c->rpart;
   for (int j = 0; j < kChunk; ++j) {
+    if (watch && j == zero_at(c) && zero_rhs(c)) break;
     k.p_old[0] = pd[j & 1];
     k.p_new[0] = pd[(j & 1) ^ 1];
     k.cs_old = cs[j & 1];
@@ -647,9 +676,9 @@ static void enqueue_pcg_grid(cpfft_ctx* c, double* x, int base) {
 // once after convergence, so the chunk has no host-side control flow and can
 // be replayed from a graph.
 // base: the solve's iteration number of the chunk's first iteration (only
-// labels timing events)
-static void enqueue_pcg_chunk(cpfft_ctx* c, double* x, int base = 0) {
-  if (gkdf_grid_edge(c->N)) return enqueue_pcg_grid(c, x, base);
+// labels timing events); watch: stop early if the right-hand side vanishes
+static void enqueue_pcg_chunk(cpfft_ctx* c, double* x, int base = 0, bool watch = false) {
+  if (gkdf_grid_edge(c->N)) return enqueue_pcg_grid(c, x, base, watch);
   const long n = 9 * c->V;
   SpecGeom g = c->geom;
   g.skip = &c->dcg->done;
@@ -671,6 +700,7 @@ static void enqueue_pcg_chunk(cpfft_ctx* c, double* x, int base = 0) {
     fz.rr_part = c->rpart;
   }
   for (int j = 0; j < kChunk; ++j) {
+    if (watch && j == zero_at(c) && zero_rhs(c)) break;
     c->ev_cur = base + j;
     tstart(c, 0);
     launch_gkdf_pencil(g, c->p, c->fields[CPFFT_K4], c->q, c->spec, c->tw, c->stream, &fz);
@@ -903,7 +933,9 @@ extern "C" int cpfft_pcg(cpfft_ctx* c, const double* b, double* x, double tol, i
   // enqueues them in chunks and reads the state once per chunk.  Kernels of
   // iterations enqueued after convergence return at once.
   launch_cg_start(n, b, x, c->r, gkdf_grid_edge(c->N) ? nullptr : c->p, c->partials, c->stream);
-  launch_cg_init(c->partials, cg_start_parts(), tol, c->cg_maxit, 3, c->dcg, nullptr, 1, c->stream);
+  c->cg_seq++;
+  launch_cg_init(c->partials, cg_start_parts(), tol, c->cg_maxit, 3, c->dcg, nullptr, 1, c->stream,
+                 c->hzero, c->cg_seq);
   const bool graph = c->use_graphs && !c->timing;
   hipGraphExec_t ge = nullptr;
   if (graph) {
@@ -914,19 +946,20 @@ extern "C" int cpfft_pcg(cpfft_ctx* c, const double* b, double* x, double tol, i
       c->pcg_graphs.emplace_back(x, ge);
     }
   }
+  // (The first chunk is launched kernel by kernel also with graphs: zero_rhs.)
   int launched = 0;
   // the events of this solve follow the first ev0[f] of family f
   int ev0[cpfft_ctx::kFam];
   std::copy(c->ev_n, c->ev_n + cpfft_ctx::kFam, ev0);
   for (;;) {
-    if (graph) {
+    if (graph && launched > 0) {
       HIP_OK(hipGraphLaunch(ge, c->stream));
     } else {
       if (c->timing && (c->ev_n[0] + kChunk > cpfft_ctx::kRing || c->ev_n[2] + kChunk > cpfft_ctx::kRing)) {
         flush_events(c);
         std::fill(ev0, ev0 + cpfft_ctx::kFam, 0);
       }
-      enqueue_pcg_chunk(c, x, launched);
+      enqueue_pcg_chunk(c, x, launched, launched == 0);
     }
     launched += kChunk;
     HIP_OK(hipGetLastError());

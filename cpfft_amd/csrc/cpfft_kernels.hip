@@ -234,11 +234,13 @@ __global__ __launch_bounds__(kBlock) void k_cg_start(long n, const double* __res
   const double s = block_sum(acc, sh);
   if (threadIdx.x == 0) part[blockIdx.x] = s;
 }
-// block b: system b
+// block b: system b; told: with one system, host memory that receives
+// 2 seq + (whether the right-hand side vanishes)
 __global__ __launch_bounds__(kBlock) void k_cg_init(const double* __restrict__ part, int np,
                                                     double tol, int maxit, int zero_code,
                                                     CGScalars* __restrict__ cs,
-                                                    double* __restrict__ m) {
+                                                    double* __restrict__ m, long long* told,
+                                                    long long seq) {
   __shared__ double sh[kBlock];
   const double bb = ordered_sum<kBlock>(part + (long)blockIdx.x * np, np, sh);
   if (m && threadIdx.x < 9) m[9 * blockIdx.x + threadIdx.x] = 0.0;
@@ -252,6 +254,8 @@ __global__ __launch_bounds__(kBlock) void k_cg_init(const double* __restrict__ p
     c.maxit = maxit;
     c.done = c.n2b <= 2.220446049250313e-16 ? zero_code : 0;
     cs[blockIdx.x] = c;
+    if (told)
+      __hip_atomic_store(told, 2 * seq + (c.done != 0), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
   }
 }
 void launch_cg_start(long n, const double* b, double* x, double* r, double* p, double* partials,
@@ -263,8 +267,9 @@ void launch_cg_start(long n, const double* b, double* x, double* r, double* p, d
 }
 int cg_start_parts() { return kRedBlocks; }
 void launch_cg_init(const double* part, int np, double tol, int maxit, int zero_code,
-                    CGScalars* cs, double* m, int nsys, hipStream_t s) {
-  k_cg_init<<<nsys, kBlock, 0, s>>>(part, np, tol, maxit, zero_code, cs, m);
+                    CGScalars* cs, double* m, int nsys, hipStream_t s, long long* told,
+                    long long seq) {
+  k_cg_init<<<nsys, kBlock, 0, s>>>(part, np, tol, maxit, zero_code, cs, m, told, seq);
 }
 // alpha = rr / (p.q) from the partial sums (same order as k_sum_parts)
 // block b serves system b: partial sums part + b pstride, scalars cs + b

@@ -169,9 +169,11 @@ void launch_cg_start(long n, const double* b, double* x, double* r, double* p, d
 int cg_start_parts();
 // state of nsys solves about to start, from the partial sums of b.b (np per
 // system): done = zero_code where |b| vanishes (FFT_nr3.f:254-262); with
-// m != nullptr its nine values per system are cleared
+// m != nullptr its nine values per system are cleared; with told != nullptr
+// (pinned host memory, one system) *told = 2 seq + (whether |b| vanishes)
 void launch_cg_init(const double* part, int np, double tol, int maxit, int zero_code,
-                    CGScalars* cs, double* m, int nsys, hipStream_t s);
+                    CGScalars* cs, double* m, int nsys, hipStream_t s, long long* told = nullptr,
+                    long long seq = 0);
 // out[9 j + i] = mean of row 9 j + i of K4 + m[9 i + j] (tangent_homo's end:
 // the mean of K4:(E_i + x_i))
 void launch_mean81(const double* K4, long V, const double* m, double* partials, double* out,

@@ -1,6 +1,8 @@
 """GPU tests of what the solver's calls leave behind beside their results: the
 recorded kernel times, the time of a solve with nothing to do, the device
 memory a context holds, and the launch shapes it reports."""
+import time
+
 import numpy as np
 import pytest
 
@@ -37,4 +39,42 @@ def test_zero_right_hand_side_keeps_recorded_times(N, mode):
     assert not s.download(C.WORK).any()
     _, cnt = s.kernel_times()
     assert cnt[0] == it and cnt[2] == it
+    s.close()
+
+
+@pytest.mark.parametrize("graphs", [False, True])
+@pytest.mark.parametrize("mode", [0, 1])
+def test_zero_right_hand_side_returns_early(mode, graphs):
+    """Nothing but the norm of b is formed for it: under 0.4 of the time of a
+    solve stopped after the eight iterations of a host round trip (a solve whose
+    iterations are all enqueued and return one by one takes 0.45 to 0.7)."""
+    s = _solver(16, mode)
+    _rhs(s, 16)
+    s.set_graphs(graphs)
+    s.set_cg_maxit(8)
+    s.fill9(C.DFM, np.zeros(9))
+
+    def median(f):
+        for _ in range(5):
+            f()
+        v = []
+        for _ in range(41):
+            t0 = time.perf_counter()
+            f()
+            s.sync()
+            v.append(time.perf_counter() - t0)
+        return np.median(v)
+
+    def solve():
+        with pytest.raises(C.CpfftError):
+            s.pcg(C.B, C.WORK, 1e-12)
+
+    def zero():
+        assert s.pcg(C.DFM, C.WORK, 1e-12) == (1, 0, 0.0)
+
+    a = median(zero)
+    assert not s.download(C.WORK).any()
+    b = median(solve)
+    print(f"\n[zero] mode {mode} graphs {graphs}: {a * 1e6:.0f} of {b * 1e6:.0f} us", flush=True)
+    assert a < 0.4 * b
     s.close()
