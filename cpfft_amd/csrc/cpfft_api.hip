@@ -69,7 +69,10 @@ struct cpfft_ctx {
   // tangent_homo's nine simultaneous solves: x, r, p, q per right-hand side
   double* th[4][9] = {};
   CGScalars* dcg9 = nullptr;
-  int homo_group = 1;  // systems per launch of tangent_homo on fft_grid.hip's edges
+  // systems per launch of tangent_homo on fft_grid.hip's edges (0: not chosen
+  // yet, see homo_prepare) and their spectra (nullptr: spec holds them)
+  int homo_group = 0;
+  cplx* hspec = nullptr;
   // tangent_homo keeps no x: per right-hand side i,
   // hdc[9i..9i+9) receives the voxel sums of K4:p_i from pass C and
   // hm[9i..9i+9) the running sum of alpha * mean(K4:p_i) = mean(K4:x_i)
@@ -136,18 +139,34 @@ static int upload_orients(cpfft_ctx* c, const std::vector<std::array<double, 3>>
   return 0;
 }
 
-// Right-hand sides of tangent_homo per launch on fft_grid.hip's kernels: as
-// many as 700 MB of spectra hold, so all nine up to 96^3.  (That the spectra
-// outgrow the 256 MB memory-side cache costs less than the launches: at 96^3
-// one, three and nine a launch took 85.0, 73.3 and 69.4 ms a call.)
-static int homo_group(const SpecGeom& g) {
-  const long one = 9 * g.S1 * (long)sizeof(cplx);
-  return (int)std::max(1L, std::min(9L, (700L << 20) / one));
-}
 // whether tangent_homo runs on fft_grid.hip's kernels
 static bool homo_grid(const SpecGeom& g) {
   return gkdf_grid_edge(g.N) || (gkdf_slab_edge(g.N) && g.gamma_mode == 1);
 }
+
+// Chooses the systems per launch of tangent_homo on fft_grid.hip's kernels and
+// allocates their spectra, once, before the first solve or graph needs them: a
+// context that only solves does not hold them (585 MB at 96^3).  As many
+// systems as 700 MB hold, so all nine up to 96^3 (1.4 GB above 126^3, where a
+// transposed copy follows each), evenly over the launches; fewer if the device
+// has less.  (That the spectra outgrow the 256 MB memory-side cache costs less
+// than the launches: at 96^3 one, three and nine a launch took 85.0, 73.3 and
+// 69.4 ms a call; at 130^3 two and three 233 and 223.)
+static void homo_prepare(cpfft_ctx* c) {
+  if (c->homo_group > 0 || !homo_grid(c->geom)) return;
+  const long one = grid_spec_len(c->geom);  // entries per system
+  const int fit = (int)(18 * c->geom.S1 / one);  // systems spec holds
+  const long budget = (700L << 20) / (9 * c->geom.S1 * (long)sizeof(cplx));
+  auto even = [](int n) { return (9 + (9 + n - 1) / n - 1) / ((9 + n - 1) / n); };
+  int n = even((int)std::max(1L, std::min(9L, budget)));
+  for (; n > fit; n = even(n / 2)) {
+    if (hipMalloc(&c->hspec, n * one * sizeof(cplx)) == hipSuccess) break;
+    (void)hipGetLastError();
+    c->hspec = nullptr;
+  }
+  c->homo_group = c->hspec ? n : std::min(even(fit), 9);
+}
+static cplx* homo_spec(const cpfft_ctx* c) { return c->hspec ? c->hspec : c->spec; }
 
 static void drop_graphs(cpfft_ctx* c);
 static void enqueue_homo_chunk(cpfft_ctx* c);
@@ -160,7 +179,7 @@ extern "C" int cpfft_destroy(cpfft_ctx* c) {
   if (c->stream) (void)hipStreamSynchronize(c->stream);
   for (int f = 0; f < CPFFT_NFIELDS; ++f)
     if (c->fields[f]) (void)hipFree(c->fields[f]);
-  void* bufs[] = {c->spec, c->tw, c->r, c->p, c->q, c->tmp9, c->tan6, c->partials, c->dpart, c->rpart, c->dres, c->orients, c->oid, c->dcnt, c->dcg};
+  void* bufs[] = {c->spec, c->hspec, c->tw, c->r, c->p, c->q, c->tmp9, c->tan6, c->partials, c->dpart, c->rpart, c->dres, c->orients, c->oid, c->dcnt, c->dcg};
   for (void* b : bufs)
     if (b) (void)hipFree(b);
   if (c->hres) (void)hipHostFree(c->hres);
@@ -264,12 +283,8 @@ extern "C" int cpfft_create(int N, const cpfft_material* m, const double* angles
     c->field_len[f] = lens[f];
     HIP_OK(hipMalloc(&c->fields[f], lens[f] * sizeof(double)));
   }
-  c->homo_group = homo_group(c->geom);
   const bool grid = gkdf_grid_edge(N);
-  const long nspec = homo_grid(c->geom)
-                         ? std::max(18 * c->geom.S1, c->homo_group * grid_spec_len(c->geom))
-                         : 18 * c->geom.S1;
-  HIP_OK(hipMalloc(&c->spec, nspec * sizeof(cplx)));
+  HIP_OK(hipMalloc(&c->spec, 2 * 9 * c->geom.S1 * sizeof(cplx)));
   HIP_OK(hipMalloc(&c->r, 9 * V * sizeof(double)));
   HIP_OK(hipMalloc(&c->p, 9 * V * sizeof(double)));
   HIP_OK(hipMalloc(&c->q, 9 * V * sizeof(double)));
@@ -726,12 +741,12 @@ static void enqueue_pcg_chunk(cpfft_ctx* c, double* x, int base = 0, bool watch 
 //   capture);
 // - capture in thread-local mode; the graph must consist of kernel nodes
 //   only, as many as the first capture of the same chunk (kind, edge,
-//   operator and launch shapes) held, so that a capture that took in a
+//   operator, launch shapes and systems per launch) held, so that a capture that took in a
 //   foreign launch or lost one of its own is an error, not a wrong result;
 // - instantiation, then the upload of the executable graph (its kernel
 //   arguments included) completed by a stream synchronisation.
 static std::mutex g_capture_mu;
-static std::map<std::array<int, 7>, size_t> g_chunk_nodes;
+static std::map<std::array<int, 8>, size_t> g_chunk_nodes;
 
 template <class F>
 static int capture_chunk(cpfft_ctx* c, int kind, F&& enqueue, hipGraphExec_t* out) {
@@ -760,7 +775,7 @@ static int capture_chunk(cpfft_ctx* c, int kind, F&& enqueue, hipGraphExec_t* ou
     kernels_only = hipGraphNodeGetType(nodes[i], &t) == hipSuccess && t == hipGraphNodeTypeKernel;
   }
   const PencilTune& tu = c->geom.tune;
-  const std::array<int, 7> key{kind, c->N, c->geom.gamma_mode, tu.a, tu.a0, tu.b, tu.c};
+  const std::array<int, 8> key{kind, c->N, c->geom.gamma_mode, tu.a, tu.a0, tu.b, tu.c, c->homo_group};
   auto it = g_chunk_nodes.find(key);
   const bool count_ok = it == g_chunk_nodes.end() || it->second == nn;
   if (!kernels_only || !count_ok || nn == 0) {
@@ -897,6 +912,7 @@ static int prepare_graphs(cpfft_ctx* c) {
     if ((rc = capture_chunk(c, 0, [&] { enqueue_pcg_chunk(c, x); }, &ge))) return rc;
     c->pcg_graphs.emplace_back(x, ge);
   }
+  homo_prepare(c);
   if (!c->homo_graph &&
       (rc = capture_chunk(c, 1, [&] { enqueue_homo_chunk(c); }, &c->homo_graph)))
     return rc;
@@ -1083,7 +1099,7 @@ static void enqueue_homo_slab(cpfft_ctx* c) {
         k.out[i] = pr ? nullptr : c->th[3][i0 + i];
       }
       k.npq = nb;
-      k.spec = c->spec;
+      k.spec = homo_spec(c);
       k.tw = c->tw;
       k.cs_old = k.cs_new = c->dcg9 + i0;
       k.pq = pq + (long)i0 * npq;
@@ -1117,7 +1133,7 @@ static void enqueue_homo_grid(cpfft_ctx* c) {
         k.out[i] = pr ? nullptr : Q[i0 + i];
       }
       k.K4 = c->fields[CPFFT_K4];
-      k.spec = c->spec;
+      k.spec = homo_spec(c);
       k.tw = c->tw;
       k.cs_old = cs[j & 1] + i0;
       k.cs_new = cs[(j & 1) ^ 1] + i0;
@@ -1197,13 +1213,15 @@ extern "C" int cpfft_tangent_homo(cpfft_ctx* c, double tol, double C_homo[81]) {
   double* const* Q = c->th[3];
   const double* K4 = c->fields[CPFFT_K4];
   int rc;
+  homo_prepare(c);
   // right-hand sides b_i = -G(K4 : E_i) in R[i]; a zero one needs no
   // iterations (dF_i = 0)
   if (homo_grid(c->geom)) {
     const int np = grid_parts(c->N);
     for (int i0 = 0; i0 < 9; i0 += c->homo_group) {
       tstart(c, 3);
-      launch_homo_rhs_grid(c->geom, K4, i0, std::min(c->homo_group, 9 - i0), R + i0, c->spec, c->tw,
+      launch_homo_rhs_grid(c->geom, K4, i0, std::min(c->homo_group, 9 - i0), R + i0,
+                           homo_spec(c), c->tw,
                            c->rpart + (long)i0 * np, c->stream);
       tstop(c, 3);
     }

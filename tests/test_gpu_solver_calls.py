@@ -5,6 +5,7 @@ import time
 
 import numpy as np
 import pytest
+import torch
 
 import cpfft_amd as C
 from cpfft_amd.microstructure import polycrystal
@@ -77,4 +78,60 @@ def test_zero_right_hand_side_returns_early(mode, graphs):
     b = median(solve)
     print(f"\n[zero] mode {mode} graphs {graphs}: {a * 1e6:.0f} of {b * 1e6:.0f} us", flush=True)
     assert a < 0.4 * b
+    s.close()
+
+
+@pytest.mark.parametrize("N,systems", [(96, 9), (126, 5), (130, 3)])
+def test_tangent_spectra_are_allocated_at_first_use(N, systems):
+    """The spectra of tangent_homo's systems, 700 MB at most (twice that above
+    126), are not part of what a context that only solves holds.  (The device
+    hands out 2 MiB pages, so the free memory tells the size to that much at
+    either end.)"""
+    free = lambda: torch.cuda.mem_get_info()[0]  # noqa: E731
+
+    def one():
+        s = _solver(N)
+        s.drive_eps_sig(1, 0)
+        s.set_cg_maxit(1)
+        s.sync()
+        a = free()
+        with pytest.raises(C.CpfftError):
+            s.tangent_homo(1e-8)
+        b = free()
+        with pytest.raises(C.CpfftError):
+            s.tangent_homo(1e-8)
+        assert free() == b
+        s.close()
+        return a - b
+
+    one()  # loads the kernels
+    grown = one()
+    want = systems * (9 if N <= 126 else 18) * N * N * (N // 2 + 1) * 16
+    assert abs(grown - want) <= 4 << 20
+    assert want <= (700 if N <= 126 else 1400) << 20
+
+
+@pytest.mark.parametrize("N,mode,graphs", [(96, 1, True), (126, 1, False), (130, 1, True),
+                                           (135, 0, False)])
+def test_tangent_homo_in_groups(N, mode, graphs):
+    """tangent_homo where nine systems share a launch with more than 64 KiB of
+    LDS a block (96), where five and four do (126) and where fewer share the
+    five kernels above 126: two columns, of the first and the last group,
+    against a cpfft_pcg solve each (1e-9, as test_tangent_homo_edges)."""
+    s = _solver(N, mode)
+    s.drive_eps_sig(1, 0)
+    s.set_graphs(graphs)
+    got = s.tangent_homo(1e-8).reshape(9, 9)  # [j][i]
+    K = s.download(C.K4)
+    for i in (1, 8):
+        E = np.zeros(9)
+        E[i] = 1.0
+        s.fill9(C.DFM, E)
+        s.gkdf(C.DFM, C.B, 1)
+        s.dscal(-1.0, C.B)
+        assert s.pcg(C.B, C.WORK, 1e-8)[0] == 0
+        x = s.download(C.WORK)
+        x[i] += 1.0
+        want = np.array([np.einsum("cv,cv->", K[9 * j:9 * j + 9], x) for j in range(9)]) / s.V
+        assert abs(got[:, i] - want).max() <= 1e-9 * abs(want).max()
     s.close()
