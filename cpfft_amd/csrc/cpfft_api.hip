@@ -122,6 +122,7 @@ struct cpfft_ctx {
   int ev_cur = -1;
   std::vector<hipEvent_t> ev[kFam][2];
   std::vector<int> ev_it[kFam];
+  std::vector<int> ev_w[kFam];
   int ev_n[kFam] = {0, 0, 0, 0};
   double t_ms[kFam] = {0, 0, 0, 0};
   long t_n[kFam] = {0, 0, 0, 0};
@@ -403,13 +404,14 @@ static void flush_events(cpfft_ctx* c) {
       float ms = 0.f;
       if (hipEventElapsedTime(&ms, c->ev[f][0][k], c->ev[f][1][k]) == hipSuccess) {
         c->t_ms[f] += ms;
-        c->t_n[f] += 1;
+        c->t_n[f] += c->ev_w[f][k];
       }
     }
     c->ev_n[f] = 0;
   }
 }
-static void tstart(cpfft_ctx* c, int fam) {
+// w: operator applications (or updates) of the group
+static void tstart(cpfft_ctx* c, int fam, int w = 1) {
   if (!c->timing) return;
   if (c->ev_seq[fam]++ % c->timing != 0) return;  // not sampled: tstop does nothing
   if (c->ev_n[fam] == cpfft_ctx::kRing) flush_events(c);
@@ -420,9 +422,11 @@ static void tstart(cpfft_ctx* c, int fam) {
     c->ev[fam][0].push_back(a);
     c->ev[fam][1].push_back(b);
     c->ev_it[fam].push_back(-1);
+    c->ev_w[fam].push_back(1);
   }
   (void)hipEventRecord(c->ev[fam][0][k], c->stream);
   c->ev_it[fam][k] = c->ev_cur;
+  c->ev_w[fam][k] = w;
   c->open_fam = fam;
 }
 static void tstop(cpfft_ctx* c, int fam) {
@@ -445,8 +449,8 @@ extern "C" int cpfft_set_timing(cpfft_ctx* c, int on) {
   return 0;
 }
 
-// average device time (ms) per launch group of each family since
-// cpfft_set_timing, followed by the counts in out[4..7]
+// average device time (ms) per application or update of each family since
+// cpfft_set_timing, followed by their numbers in out[4..7]
 extern "C" int cpfft_kernel_times(cpfft_ctx* c, double out[8]) {
   flush_events(c);
   for (int i = 0; i < cpfft_ctx::kFam; ++i) {
@@ -685,9 +689,10 @@ static void enqueue_pcg_grid(cpfft_ctx* c, double* x, int base, bool watch) {
     c->ev_cur = base + j;
     tstart(c, 0);
     launch_cg_grid(c->geom, k, 0, c->stream);
+    launch_cg_grid(c->geom, k, 1, c->stream);
     tstop(c, 0);
     tstart(c, 2);
-    launch_cg_grid(c->geom, k, 1, c->stream);
+    launch_cg_grid(c->geom, k, 2, c->stream);
     if (!fchk || j == kChunk - 1) launch_cg_check(c->rpart, np, c->dcg, c->stream);
     tstop(c, 2);
   }
@@ -1114,8 +1119,7 @@ static void enqueue_homo_slab(cpfft_ctx* c) {
       k.pq = pq + (long)i0 * npq;
       k.rr = c->rpart + (long)i0 * np;
       k.dc = c->hdc + 9 * i0;
-      launch_cg_grid(c->geom, k, 0, c->stream);
-      launch_cg_grid(c->geom, k, 1, c->stream);
+      for (int part = 0; part < 3; ++part) launch_cg_grid(c->geom, k, part, c->stream);
     }
     launch_cg_check(c->rpart, np, c->dcg9, c->stream, c->hdc, c->hm, 1.0 / (double)V, 9, np);
   }
@@ -1152,8 +1156,7 @@ static void enqueue_homo_grid(cpfft_ctx* c) {
       k.dc = c->hdc + 9 * i0;
       k.m = c->hm + 9 * i0;
       k.scale = sc;
-      launch_cg_grid(c->geom, k, 0, c->stream);
-      launch_cg_grid(c->geom, k, 1, c->stream);
+      for (int part = 0; part < 3; ++part) launch_cg_grid(c->geom, k, part, c->stream);
     }
     if (!fchk || j == kChunk - 1)
       launch_cg_check(c->rpart, np, c->dcg9, c->stream, c->hdc, c->hm, sc, 9, np);
@@ -1228,9 +1231,9 @@ extern "C" int cpfft_tangent_homo(cpfft_ctx* c, double tol, double C_homo[81]) {
   if (homo_grid(c->geom)) {
     const int np = grid_parts(c->N);
     for (int i0 = 0; i0 < 9; i0 += c->homo_group) {
-      tstart(c, 3);
-      launch_homo_rhs_grid(c->geom, K4, i0, std::min(c->homo_group, 9 - i0), R + i0,
-                           homo_spec(c), c->tw,
+      const int nsys = std::min(c->homo_group, 9 - i0);
+      tstart(c, 3, nsys);
+      launch_homo_rhs_grid(c->geom, K4, i0, nsys, R + i0, homo_spec(c), c->tw,
                            c->rpart + (long)i0 * np, c->stream);
       tstop(c, 3);
     }

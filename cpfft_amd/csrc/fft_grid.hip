@@ -1364,8 +1364,12 @@ static void run_cg(const SpecGeom& sg, const GridCG& c, int part, hipStream_t s)
       forward<NC, true, true>(g, a.f, ct, s);
     }
     middle<NC>(g, a.m, c.nrhs, sg.tune.c, s);
+  } else if (part == 1) {
+    if (plain)
+      inverse<NC, 1>(g, a.i, c.nrhs, ct, s);
+    else
+      inverse<NC, 2>(g, a.i, c.nrhs, ct, s);
   } else if (plain) {
-    inverse<NC, 1>(g, a.i, c.nrhs, ct, s);
     StepArgs t{};
     t.p = a.i.pd;
     t.q = a.i.out;
@@ -1376,8 +1380,6 @@ static void run_cg(const SpecGeom& sg, const GridCG& c, int part, hipStream_t s)
     t.cs = c.cs_new;
     t.rrp = c.rr;
     k_step<<<dim3(a.f.nrr, c.nrhs), 256, 0, s>>>(9 * g.V, t);
-  } else {
-    inverse<NC, 2>(g, a.i, c.nrhs, ct, s);
   }
 }
 

@@ -96,9 +96,11 @@ void launch_gkdf_grid(const SpecGeom& g, const double* F, const double* K4, doub
 //   K4:p_new and its product with p_new) and the passes up to the projected
 //   spectrum, alpha among them;
 // part 1: the inverse pass: r -= alpha q, where x[i] != nullptr also
-//   x += alpha p_new, and the r.r partial sums.
+//   x += alpha p_new, and the r.r partial sums;
+// part 2: nothing.
 // out[0] != nullptr instead (the reference's operator): part 0 forms no
-//   alpha; part 1 stores q in out, takes p.q from it and updates r and x.
+//   alpha; part 1 stores q in out with the p.q partial sums; part 2 forms alpha
+//   and updates r and x.
 // cs_old is the state before the iteration, cs_new the one after chk; they
 // may be the same array when !chk.  p_old and p_new are different fields.
 struct GridCG {

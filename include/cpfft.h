@@ -239,10 +239,12 @@ int cpfft_set_tune(cpfft_ctx* ctx, const int in[4]);
  * evaluations in line searches                                            */
 int cpfft_counters(cpfft_ctx* ctx, long long out[8]);
 /* device-time measurement with HIP events recorded on the context's stream
- * (no host synchronisation while recording).  out[0..3]: average ms per
- * launch group since cpfft_set_timing of [0] G_K_dF with K4,
- * [1] drive_eps_sig, [2] CG vector update, [3] G_K_dF without K4;
- * out[4..7]: number of launch groups measured.
+ * (no host synchronisation while recording).  out[0..3]: average ms since
+ * cpfft_set_timing of [0] G_K_dF with K4 (in a solve with what of the vector
+ * update its kernels take over), [1] drive_eps_sig, [2] the rest of the CG
+ * vector update and its test, [3] G_K_dF without K4 (per application, also
+ * where tangent_homo launches several together); out[4..7]: how many of each
+ * were measured.
  * cpfft_set_timing(ctx, k): 0 off; k > 0 records every k-th launch group
  * of each family.  Each recorded pair costs the stream about 10 us of idle
  * time around it, so a long run is timed with a sampling stride (bench.py

@@ -172,3 +172,52 @@ def test_displacements_into_any_memory(N):
     if N == 96:
         assert b < 0.9 * a
     s.close()
+
+
+@pytest.mark.parametrize("N,mode", [(90, 1), (45, 0)])
+def test_times_of_a_solve_are_the_operators(N, mode):
+    """The operator's time within a solve is that of all its kernels: at least
+    0.9 of an application's own (it also forms the direction), and with the
+    textbook operator, whose inverse pass updates the vectors too, what is left
+    for the update is under a fifth of it."""
+    s = _solver(N, mode)
+    _rhs(s, N)
+    s.set_timing(1)
+    for _ in range(20):
+        s.gkdf(C.DFM, C.WORK, 1)
+    gk, n = s.kernel_times()
+    assert n[0] == 20
+    s.set_timing(1)
+    assert s.pcg(C.B, C.WORK, 1e-8)[0] == 0
+    cg, _ = s.kernel_times()
+    print(f"\n[times] {N}: G_K_dF {gk[0] * 1e3:.1f}, in a solve {cg[0] * 1e3:.1f} + {cg[2] * 1e3:.1f} us",
+          flush=True)
+    assert cg[0] >= 0.9 * gk[0]
+    if mode == 1:
+        assert cg[2] < 0.2 * cg[0]
+    s.close()
+
+
+@pytest.mark.parametrize("N,mode", [(16, 1), (45, 0), (96, 1), (126, 1), (128, 1)])
+def test_times_count_applications(N, mode):
+    """tangent_homo's right-hand sides are nine applications, however many share
+    a launch; the average is an application's (launched together they take less
+    than alone)."""
+    s = _solver(N, mode)
+    s.drive_eps_sig(1, 0)
+    s.set_timing(1)
+    s.gkdf(C.DFM, C.B, 0)
+    for _ in range(20):
+        s.gkdf(C.DFM, C.B, 0)
+    one, _ = s.kernel_times()
+    s.set_cg_maxit(1)
+    with pytest.raises(C.CpfftError):
+        s.tangent_homo(1e-8)
+    s.set_timing(1)
+    with pytest.raises(C.CpfftError):
+        s.tangent_homo(1e-8)
+    avg, cnt = s.kernel_times()
+    print(f"\n[times] {N}: alone {one[3] * 1e3:.1f}, in tangent_homo {avg[3] * 1e3:.1f} us", flush=True)
+    assert cnt[3] == 9
+    assert 0.0 < avg[3] < 1.5 * one[3]
+    s.close()
