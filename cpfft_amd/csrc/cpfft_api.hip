@@ -813,13 +813,14 @@ static void drop_graphs(cpfft_ctx* c) {
 }
 
 // ---------------------------------------------------------- autotuner
-// Shapes chosen per (device, N), shared by every context of the process.
+// Shapes chosen per (device, N, operator), shared by every context of the
+// process (fft_pencil.hip's kernels are the same for both operators).
 static std::mutex g_tune_mu;
-static std::map<std::pair<int, int>, PencilTune> g_tune;
+static std::map<std::array<int, 3>, PencilTune> g_tune;
 
 // value of candidate v of pass p, 0 if there is none
-static int tune_value(int N, int p, int v) {
-  return gkdf_grid_edge(N) ? grid_candidate(N, p, v) : pencil_candidate(N, p, v);
+static int tune_value(const SpecGeom& g, int p, int v) {
+  return gkdf_grid_edge(g.N) ? grid_candidate(g.N, g.gamma_mode, p, v) : pencil_candidate(g.N, p, v);
 }
 
 static void apply_tune(cpfft_ctx* c, const PencilTune& t) {
@@ -834,9 +835,9 @@ static void apply_tune(cpfft_ctx* c, const PencilTune& t) {
 
 extern "C" int cpfft_autotune(cpfft_ctx* c, int reps, int force) {
   if (!c) return fail(-1, "cpfft_autotune: null context");
-  if (!tune_value(c->N, 0, 0)) return 1;
+  if (!tune_value(c->geom, 0, 0)) return 1;
   if (reps < 1) reps = 10;
-  const std::pair<int, int> key(c->dev, c->N);
+  const std::array<int, 3> key{c->dev, c->N, gkdf_grid_edge(c->N) ? c->geom.gamma_mode : 1};
   if (!force) {
     std::lock_guard<std::mutex> lk(g_tune_mu);
     auto it = g_tune.find(key);
@@ -858,7 +859,7 @@ extern "C" int cpfft_autotune(cpfft_ctx* c, int reps, int force) {
     float best = 0.f;
     int bi = 0;
     for (int v = 0; v < kPencilCands; ++v) {
-      if (!tune_value(c->N, pass, v)) continue;
+      if (!tune_value(c->geom, pass, v)) continue;
       auto one = [&] {
         if (gkdf_grid_edge(c->N))
           launch_grid_pass(c->geom, pass, v, F, K4, c->spec, c->tw, c->stream);
@@ -892,19 +893,19 @@ extern "C" int cpfft_get_tune(cpfft_ctx* c, int out[4]) {
   if (!c) return fail(-1, "cpfft_get_tune: null context");
   const PencilTune& t = c->geom.tune;
   const int idx[4] = {t.a, t.a0, t.b, t.c};
-  for (int p = 0; p < 4; ++p) out[p] = tune_value(c->N, p, idx[p]);
+  for (int p = 0; p < 4; ++p) out[p] = tune_value(c->geom, p, idx[p]);
   return 0;
 }
 
 extern "C" int cpfft_set_tune(cpfft_ctx* c, const int in[4]) {
   if (!c) return fail(-1, "cpfft_set_tune: null context");
-  if (!tune_value(c->N, 0, 0)) return fail(-1, "cpfft_set_tune: no tunable shapes for this N");
+  if (!tune_value(c->geom, 0, 0)) return fail(-1, "cpfft_set_tune: no tunable shapes for this N");
   PencilTune t;
   int* knob[4] = {&t.a, &t.a0, &t.b, &t.c};
   for (int p = 0; p < 4; ++p) {
     int found = -1;
     for (int v = 0; v < kPencilCands && found < 0; ++v)
-      if (tune_value(c->N, p, v) == in[p] && in[p] > 0) found = v;
+      if (tune_value(c->geom, p, v) == in[p] && in[p] > 0) found = v;
     if (found < 0) return fail(-1, "cpfft_set_tune: shape is not among the candidates for this N");
     *knob[p] = found;
   }

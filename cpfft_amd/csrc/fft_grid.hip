@@ -764,7 +764,7 @@ __global__ __launch_bounds__(1024) void k_fwd(Grid g, FwdArgs a) {
 template <int NC, bool PAIR>
 __global__ __launch_bounds__(1024) void k_mid(Grid g, MidArgs a) {
   extern __shared__ cplx lds[];
-  constexpr int NL = PAIR ? 2 : 3;  // x lines per (kz, y)
+  constexpr int NL = PAIR ? 2 : 3;  // x lines per (kz, y), as mid_lines
   const int rhs = blockIdx.z, row = blockIdx.y, tid = threadIdx.x, T = blockDim.x;
   int tile = blockIdx.x;
   if (a.cs) {
@@ -1171,6 +1171,9 @@ static void plan(int n, int* best, int& nb, int* cur, int nc, int from) {
     }
 }
 
+// x lines per (kz, y) and tensor row (see k_mid)
+static int mid_lines(int N, int gamma_mode) { return N <= kSlabN && gamma_mode == 1 ? 2 : 3; }
+
 static Grid make_grid(const SpecGeom& s) {
   Grid g;
   g.N = s.N;
@@ -1178,7 +1181,7 @@ static Grid make_grid(const SpecGeom& s) {
   g.nzk = s.gamma_mode == 1 && s.N % 2 == 0 ? s.Nz - 1 : s.Nz;
   g.NN = s.N * s.N;
   g.gamma_mode = s.gamma_mode;
-  g.pair = s.N <= kSlabN && s.gamma_mode == 1;
+  g.pair = mid_lines(s.N, s.gamma_mode) == 2;
   g.V = s.V;
   g.S1 = s.S1;
   g.dN = Div(s.N);
@@ -1263,7 +1266,7 @@ static void middle(const Grid& g, const MidArgs& a, int nrhs, int cand, hipStrea
   if (NC != kAnyRadix || g.N <= kSlabN) {
     const int tiles = (g.nzk * g.N + kML - 1) / kML;
     const dim3 grid(tiles + (a.pqp ? 1 : 0), 3, nrhs);
-    const int nl = g.pair ? 2 : 3;
+    const int nl = mid_lines(g.N, g.gamma_mode);
     auto k = g.pair ? k_mid<NC, true> : k_mid<NC, false>;
     k<<<grid, mid_threads(g.N, nl, cand), lds_lines(g.N, nl * kML), s>>>(g, a);
   } else if constexpr (NC == kAnyRadix) {
@@ -1469,10 +1472,10 @@ int grid_rr_parts(int N, bool projection) {
 bool grid_fused_check(int N) { return grid_parts(N) <= 2304; }
 long grid_spec_len(const SpecGeom& g) { return gp::spec_stride(gp::make_grid(g)); }
 
-int grid_candidate(int N, int pass, int v) {
+int grid_candidate(int N, int gamma_mode, int pass, int v) {
   if (N != 16 && N != 32 && N != 48) return 0;
   if (v < 0 || v > 1) return 0;
-  return (pass == 3 ? gp::mid_threads(N, 2, v) : gp::slab_threads(N, v)) / 64;
+  return (pass == 3 ? gp::mid_threads(N, gp::mid_lines(N, gamma_mode), v) : gp::slab_threads(N, v)) / 64;
 }
 void launch_grid_pass(const SpecGeom& g, int pass, int v, const double* F, const double* K4,
                       cplx* spec, const cplx* tw, hipStream_t s) {

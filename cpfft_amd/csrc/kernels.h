@@ -127,7 +127,7 @@ int grid_rr_parts(int N, bool projection);
 bool grid_fused_check(int N);  // whether chk may be used at this edge
 long grid_spec_len(const SpecGeom& g);
 // autotuner support for N = 16, 32, 48 (see pencil_candidate)
-int grid_candidate(int N, int pass, int v);
+int grid_candidate(int N, int gamma_mode, int pass, int v);
 void launch_grid_pass(const SpecGeom& g, int pass, int v, const double* F, const double* K4,
                       cplx* spec, const cplx* tw, hipStream_t s);
 

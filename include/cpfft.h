@@ -213,9 +213,9 @@ int cpfft_set_cg_maxit(cpfft_ctx* ctx, int maxit);
 /* Autotuner of the compile-time-planned FFT paths (N in 16, 32, 48, 64, 96,
  * 128, 256): times the candidate launch shapes of each of the forward pass
  * with K4, without K4, the y passes (N <= 48: the inverse pass) and the x
- * pass on this context's buffers (reps launches each) and keeps the fastest.  The choice is cached per
- * device and N for every context of the process (force != 0 measures
- * again).  Only shapes that compute bit-identical results are candidates
+ * pass on this context's buffers (reps launches each) and keeps the fastest.
+ * The choice is cached per device and N (N <= 48: and operator) for every
+ * context of the process (force != 0 measures again).  Only shapes that compute bit-identical results are candidates
  * (which block transforms which lines; never the radix order or a
  * reduction), so tuning changes speed, not results.  Returns 1 (nothing to
  * tune) for other N.                                                      */

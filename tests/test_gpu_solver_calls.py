@@ -221,3 +221,67 @@ def test_times_count_applications(N, mode):
     assert cnt[3] == 9
     assert 0.0 < avg[3] < 1.5 * one[3]
     s.close()
+
+
+def _shapes(s):
+    """every shape cpfft_set_tune takes that differs from the one set in one place"""
+    now = s.tune()
+    for k in range(4):
+        for v in range(1, 65):
+            shape = list(now)
+            shape[k] = v
+            if v == now[k]:
+                continue
+            try:
+                s.set_tune(shape)
+            except C.CpfftError:
+                continue
+            assert s.tune() == shape
+            yield shape
+    s.set_tune(now)
+
+
+@pytest.mark.parametrize("N,mode,waves", [(16, 1, 2), (32, 1, 2), (48, 1, 3), (16, 0, 3), (32, 0, 3),
+                                          (48, 0, 5)])
+def test_reported_shapes_are_the_launched_ones(N, mode, waves):
+    """out[3] of cpfft_get_tune: wavefronts of the x pass, whose blocks take eight
+    x lines of two (textbook operator) or three (reference's) components, two
+    points a thread below N = 32, else four; and with the reference's operator
+    the shapes change no result either"""
+    s = _solver(N, mode)
+    assert s.tune()[3] == waves
+    if mode == 0:
+        _rhs(s, N)
+        s.set_cg_maxit(20)
+
+        def run():
+            s.gkdf(C.DFM, C.WORK, 0)
+            g = s.download(C.WORK)
+            C.lib().cpfft_pcg(s.h, s.field(C.B), s.field(C.WORK), 1e-8, None, None)
+            return g, s.download(C.WORK)
+
+        ref = run()
+        tried = 0
+        for shape in _shapes(s):
+            got = run()
+            assert np.array_equal(got[0], ref[0]) and np.array_equal(got[1], ref[1]), shape
+            tried += 1
+        assert tried >= 3
+    s.close()
+
+
+def test_shapes_are_tuned_for_each_operator():
+    """a choice timed with one operator, whose x pass is another kernel, is not
+    taken over by the other: 200 repetitions of eight or more launches take
+    longer than a millisecond, a look at the stored choice does not"""
+    a, b = _solver(48, 1), _solver(48, 0)
+    t0 = time.perf_counter()
+    a.autotune(reps=200, force=True)
+    t1 = time.perf_counter()
+    b.autotune(reps=200)
+    t2 = time.perf_counter()
+    b.autotune(reps=200)
+    t3 = time.perf_counter()
+    assert t1 - t0 > 1e-3 and t2 - t1 > 1e-3 and t3 - t2 < 1e-3
+    a.close()
+    b.close()
