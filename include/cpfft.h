@@ -226,8 +226,9 @@ int cpfft_autotune(cpfft_ctx* ctx, int reps, int force);
  * lines, transforms in registers) for N = 64, 128, 256, else 18 or 9 (all
  * nine components of 2 or 1 y lines).  N = 16, 32, 48: wavefronts per block
  * of the forward pass with K4, without K4, the inverse pass and the x pass
- * (the first and third of plain G_K_dF applications; solves take the
- * default there).  0 where N has no planned path                          */
+ * (the first three of plain G_K_dF applications; solves take the default
+ * there, and tangent_homo at 64 and 96 everywhere).  0 where N has no planned
+ * path                                                                    */
 int cpfft_get_tune(cpfft_ctx* ctx, int out[4]);
 /* set them (each must be one of the candidates; -1 otherwise)             */
 int cpfft_set_tune(cpfft_ctx* ctx, const int in[4]);

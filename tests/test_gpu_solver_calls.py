@@ -285,3 +285,14 @@ def test_shapes_are_tuned_for_each_operator():
     assert t1 - t0 > 1e-3 and t2 - t1 > 1e-3 and t3 - t2 < 1e-3
     a.close()
     b.close()
+
+
+@pytest.mark.parametrize("N", [16, 48, 64, 96])
+def test_tangent_homo_under_every_shape(N):
+    """No shape changes a tangent (the large grids: their systems take none of them)."""
+    s = _solver(N)
+    s.drive_eps_sig(1, 0)
+    ref = s.tangent_homo(1e-6)
+    for shape in _shapes(s):
+        assert np.array_equal(s.tangent_homo(1e-6), ref), shape
+    s.close()
