@@ -24,11 +24,11 @@ const char* make_spec_geom(int N, int gamma_mode, SpecGeom& g) {
   g.S1 = (long)N * N * g.Nz;
   g.gamma_mode = gamma_mode;
   if (gkdf_grid_edge(N)) {
-    if (N > 227) return "grid edge too large for the LDS of this device";
+    if (N > 227) return "no grid edge above 227 but 256 is served";
     int m = N;
     for (int p : {2, 3, 5, 7, 11})
       while (m % p == 0) m /= p;
-    if (m > 13) return "N has a prime factor above 16";
+    if (m > 13) return "N has a prime factor above 13, or 13 twice";
   }
   return nullptr;
 }

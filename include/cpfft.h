@@ -184,8 +184,8 @@ int cpfft_f2disp(cpfft_ctx* ctx, const double* F, const double lengths[3], doubl
  * serialise them.  Its address is resolved once per device (by
  * cpfft_create, or by the first call there); the call itself makes no
  * allocation.  Returns 0; -1 for a bad argument, N above the maximum
- * included; -3 for an N the operator cannot serve (prime factor above 16);
- * -100 or below for a HIP error (cpfft_last_error() describes each).     */
+ * included; -3 for an N the operator does not serve (a prime factor above
+ * 13); -100 or below for a HIP error (cpfft_last_error() describes each). */
 #define CPFFT_NOALLOC_MAX_N 48
 int cpfft_gkdf_noalloc(int N, int gamma_mode, const double* F, const double* K4, double* GKF,
                        void* stream);

@@ -296,3 +296,18 @@ def test_tangent_homo_under_every_shape(N):
     for shape in _shapes(s):
         assert np.array_equal(s.tangent_homo(1e-6), ref), shape
     s.close()
+
+
+@pytest.mark.parametrize("N,why", [(17, "prime factor above 13"), (34, "prime factor above 13"),
+                                   (169, "13 twice"), (228, "above 227 but 256"),
+                                   (250, "above 227 but 256")])
+def test_refused_edges_and_why(N, why):
+    """edges that no kernel serves are refused with -3 and the true reason"""
+    m = C.Material()
+    cm = C.CMaterial(**{k: getattr(m, k) for k, _ in C.CMaterial._fields_})
+    ang = np.zeros((3, N ** 3))
+    h = ctypes.c_void_p()
+    assert C.lib().cpfft_create(N, ctypes.byref(cm), C._p(ang), 0.25, 1, ctypes.byref(h)) == -3
+    assert why in C.lib().cpfft_last_error().decode()
+    if N <= 48:
+        assert C.lib().cpfft_gkdf_noalloc(N, 1, 8, None, 16, None) == -3
