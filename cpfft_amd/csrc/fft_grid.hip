@@ -1239,8 +1239,11 @@ static size_t lds_lines(int N, int lines) {
 // against 3.38), and radices 11 and 13 leave no registers for it.
 template <int NC, int ME, bool HASK, bool DIR>
 static void fwd_slab(const Grid& g, const FwdArgs& a, int threads, hipStream_t s) {
-  auto k = k_fwd<NC, ME, HASK, DIR, false>;
-  if constexpr (HASK && NC != kAnyRadix) {
+  constexpr bool ahead = HASK && NC != kAnyRadix;
+  // several systems have the contraction in this kernel below edge 40 only
+  constexpr bool several = !ahead || (DIR && NC != 48 && ME != kMaxE);
+  auto k = k_fwd<NC, ME, HASK, DIR, !several>;
+  if constexpr (ahead && several) {
     if (a.nrhs == 1) k = k_fwd<NC, ME, HASK, DIR, true>;
   }
   const size_t lds = lds_slab(g.N);
@@ -1261,13 +1264,19 @@ static void forward(const Grid& g, const FwdArgs& a, int cand, hipStream_t s) {
   }
 }
 
+// Edges of fft_pencil.hip: only tangent_homo's systems come here, with the
+// textbook operator and K4:p formed by a launch of its own
+constexpr bool tangent_only(int NC) { return NC == 64 || NC == 96; }
+
 template <int NC>
 static void middle(const Grid& g, const MidArgs& a, int nrhs, int cand, hipStream_t s) {
   if (NC != kAnyRadix || g.N <= kSlabN) {
     const int tiles = (g.nzk * g.N + kML - 1) / kML;
     const dim3 grid(tiles + (a.pqp ? 1 : 0), 3, nrhs);
     const int nl = mid_lines(g.N, g.gamma_mode);
-    auto k = g.pair ? k_mid<NC, true> : k_mid<NC, false>;
+    auto k = k_mid<NC, true>;
+    if constexpr (!tangent_only(NC))
+      if (!g.pair) k = k_mid<NC, false>;
     k<<<grid, mid_threads(g.N, nl, cand), lds_lines(g.N, nl * kML), s>>>(g, a);
   } else if constexpr (NC == kAnyRadix) {
     const int yb = x_lines(g.N);
@@ -1369,15 +1378,15 @@ static void run_cg(const SpecGeom& sg, const GridCG& c, int part, hipStream_t s)
     if (c.q[0]) {
       for (int k = 0; k < c.nrhs; ++k) a.f.F.p[k] = const_cast<double*>(c.q[k]);
       forward<NC, false, false>(g, a.f, 0, s);
-    } else {
+    } else if constexpr (!tangent_only(NC)) {
       forward<NC, true, true>(g, a.f, ct, s);
     }
     middle<NC>(g, a.m, c.nrhs, mid_shape(sg), s);
   } else if (part == 1) {
-    if (plain)
-      inverse<NC, 1>(g, a.i, c.nrhs, ct, s);
-    else
+    if (!plain)
       inverse<NC, 2>(g, a.i, c.nrhs, ct, s);
+    else if constexpr (!tangent_only(NC))
+      inverse<NC, 1>(g, a.i, c.nrhs, ct, s);
   } else if (plain) {
     StepArgs t{};
     t.p = a.i.pd;
@@ -1430,13 +1439,12 @@ static void run_pass(const SpecGeom& sg, int pass, int v, const double* F, const
 bool gkdf_slab_edge(int N) { return N <= gp::kSlabN; }
 bool gkdf_grid_edge(int N) { return !(N == 64 || N == 96 || N == 128 || N == 256); }
 
-#define CPFFT_EDGE(call)            \
+#define CPFFT_EDGE(call, large)     \
   switch (g.N) {                    \
     case 16: gp::call<16> CPFFT_ARGS; break; \
     case 32: gp::call<32> CPFFT_ARGS; break; \
     case 48: gp::call<48> CPFFT_ARGS; break; \
-    case 64: gp::call<64> CPFFT_ARGS; break; \
-    case 96: gp::call<96> CPFFT_ARGS; break; \
+    large                           \
     default:                        \
       if (gp::smooth(g.N))          \
         gp::call<gp::kSmooth> CPFFT_ARGS; \
@@ -1444,23 +1452,27 @@ bool gkdf_grid_edge(int N) { return !(N == 64 || N == 96 || N == 128 || N == 256
         gp::call<gp::kAnyRadix> CPFFT_ARGS; \
       break;                        \
   }
+// with the edges of tangent_only
+#define CPFFT_EDGE_ALL(call)                         \
+  CPFFT_EDGE(call, case 64: gp::call<64> CPFFT_ARGS; break; \
+             case 96: gp::call<96> CPFFT_ARGS; break;)
 
 void launch_gkdf_grid(const SpecGeom& g, const double* F, const double* K4, double* out,
                       cplx* spec, const cplx* tw, hipStream_t s) {
 #define CPFFT_ARGS (g, F, K4, out, spec, tw, s)
-  CPFFT_EDGE(run_gkdf)
+  CPFFT_EDGE(run_gkdf, )
 #undef CPFFT_ARGS
 }
 void launch_cg_grid(const SpecGeom& g, const GridCG& c, int part, hipStream_t s) {
 #define CPFFT_ARGS (g, c, part, s)
-  CPFFT_EDGE(run_cg)
+  CPFFT_EDGE_ALL(run_cg)
 #undef CPFFT_ARGS
 }
 
 void launch_homo_rhs_grid(const SpecGeom& g, const double* K4, int i0, int n, double* const* r,
                           cplx* spec, const cplx* tw, double* rr, hipStream_t s) {
 #define CPFFT_ARGS (g, K4, i0, n, r, spec, tw, rr, s)
-  CPFFT_EDGE(run_homo_rhs)
+  CPFFT_EDGE_ALL(run_homo_rhs)
 #undef CPFFT_ARGS
 }
 

@@ -799,12 +799,6 @@ constexpr int dot_parts() { return (N / tile_z(N)) * N * 9; }
 
 }  // namespace fp
 
-bool gkdf_pencil_supported(int N) {
-  switch (N) {
-    default: return false;
-  }
-}
-
 bool launch_gkdf_pencil(const SpecGeom& g, const double* F, const double* K4, double* out,
                         cplx* spec, const cplx* tw, hipStream_t s, const CGFuse* fuse) {
   cplx* T1 = spec;

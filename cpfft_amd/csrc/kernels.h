@@ -132,7 +132,6 @@ void launch_grid_pass(const SpecGeom& g, int pass, int v, const double* F, const
                       cplx* spec, const cplx* tw, hipStream_t s);
 
 // ---- fft_pencil.hip
-bool gkdf_pencil_supported(int N);
 // returns false (and launches nothing) when N has no compile-time plan
 bool launch_gkdf_pencil(const SpecGeom& g, const double* F, const double* K4, double* out,
                         cplx* spec, const cplx* tw, hipStream_t s, const CGFuse* fuse = nullptr);
