@@ -13,6 +13,7 @@ import numpy as np
 import pytest
 
 import cpfft_amd as C
+import oracle_lib as O
 from cpfft_amd.microstructure import polycrystal
 
 pytestmark = pytest.mark.gpu
@@ -105,4 +106,32 @@ def test_tangent_homo_edges(N, mode):
         x[i] += 1.0
         want = np.array([(K[9 * j:9 * j + 9] * x).sum(0).mean() for j in range(9)])
         assert abs(got[:, i] - want).max() <= 1e-9 * abs(want).max()
+    s.close()
+
+
+@pytest.mark.parametrize("N,tol", [(20, 1e-2), (40, 1e-2), (48, 1e-1)])
+def test_solves_with_the_references_even_operator(N, tol):
+    """The reference's operator on even edges, where it is no projection (CG
+    converges to a loose tolerance only): p.q from the inverse pass and an
+    update of its own, for one system and for nine, these with the contraction in
+    the forward pass (20) and in a launch of its own whose result the inverse
+    pass overwrites (40, 48), over two host round trips (20, 40).  Against the
+    oracle: equal iteration counts, 1e-9 as test_pcg_and_tangent_homo."""
+    V = N ** 3
+    _, ang = polycrystal(N, 4, 5 * N)
+    s = C.Solver(N, ang, C.Material(), dt=0.25, gamma_mode=0)
+    s.drive_eps_sig(1, 0)
+    K = s.download(C.K4)
+    fo = O.FFT(N, 0)
+    b = -fo.gkdf(np.ascontiguousarray(K.reshape(9, 9, V)[:, 1]))
+    xo, rco, ito, _ = fo.pcg(K, b, tol)
+    s.upload(C.B, b)
+    rc, it, _ = s.pcg(C.B, C.DFM, tol)
+    x = s.download(C.DFM)
+    assert rc == rco == 0 and it == ito
+    assert abs(x - xo).max() <= 1e-9 * abs(xo).max()
+    want = fo.tangent_homo(K, tol)
+    for graphs in (False, True):
+        s.set_graphs(graphs)
+        assert abs(s.tangent_homo(tol) - want).max() <= 1e-9 * abs(want).max()
     s.close()
