@@ -73,6 +73,7 @@ struct cpfft_ctx {
   // yet, see homo_prepare) and their spectra (nullptr: spec holds them)
   int homo_group = 0;
   cplx* hspec = nullptr;
+  int tune_as[4] = {0, 0, 0, 0};  // shapes that cpfft_set_tune took as former_shape
   // tangent_homo keeps no x: per right-hand side i,
   // hdc[9i..9i+9) receives the voxel sums of K4:p_i from pass C and
   // hm[9i..9i+9) the running sum of alpha * mean(K4:p_i) = mean(K4:x_i)
@@ -823,7 +824,21 @@ static int tune_value(const SpecGeom& g, int p, int v) {
   return gkdf_grid_edge(g.N) ? grid_candidate(g.N, g.gamma_mode, p, v) : pencil_candidate(g.N, p, v);
 }
 
+// Whether v was a shape of pass p at the edges 16, 32 and 48 while
+// fft_pencil.hip served them (pencils per block of pass A, lines per block of
+// the y passes, component lines of pass C).  A program may have kept one:
+// cpfft_set_tune takes it, for the default, and cpfft_get_tune returns it.
+static bool former_shape(int N, int p, int v) {
+  if (N != 16 && N != 32 && N != 48) return false;
+  static constexpr int a[3][3] = {{16, 8, 4}, {32, 16, 8}, {16, 12, 8}};
+  static constexpr int y[3][3] = {{8, 4, 2}, {8, 4, 2}, {8, 6, 4}};
+  if (p == 3) return v == 18 || v == 9;
+  const int(&l)[3] = p == 2 ? y[N / 16 - 1] : a[N / 16 - 1];
+  return v == l[0] || v == l[1] || v == l[2];
+}
+
 static void apply_tune(cpfft_ctx* c, const PencilTune& t) {
+  std::fill(c->tune_as, c->tune_as + 4, 0);
   const bool changed = t.a != c->geom.tune.a || t.a0 != c->geom.tune.a0 || t.b != c->geom.tune.b ||
                        t.c != c->geom.tune.c;
   c->geom.tune = t;
@@ -893,7 +908,7 @@ extern "C" int cpfft_get_tune(cpfft_ctx* c, int out[4]) {
   if (!c) return fail(-1, "cpfft_get_tune: null context");
   const PencilTune& t = c->geom.tune;
   const int idx[4] = {t.a, t.a0, t.b, t.c};
-  for (int p = 0; p < 4; ++p) out[p] = tune_value(c->geom, p, idx[p]);
+  for (int p = 0; p < 4; ++p) out[p] = c->tune_as[p] ? c->tune_as[p] : tune_value(c->geom, p, idx[p]);
   return 0;
 }
 
@@ -902,14 +917,20 @@ extern "C" int cpfft_set_tune(cpfft_ctx* c, const int in[4]) {
   if (!tune_value(c->geom, 0, 0)) return fail(-1, "cpfft_set_tune: no tunable shapes for this N");
   PencilTune t;
   int* knob[4] = {&t.a, &t.a0, &t.b, &t.c};
+  int as[4] = {0, 0, 0, 0};
   for (int p = 0; p < 4; ++p) {
     int found = -1;
     for (int v = 0; v < kPencilCands && found < 0; ++v)
       if (tune_value(c->geom, p, v) == in[p] && in[p] > 0) found = v;
+    if (found < 0 && former_shape(c->N, p, in[p])) {
+      found = 0;
+      as[p] = in[p];
+    }
     if (found < 0) return fail(-1, "cpfft_set_tune: shape is not among the candidates for this N");
     *knob[p] = found;
   }
   apply_tune(c, t);
+  std::copy(as, as + 4, c->tune_as);
   return 0;
 }
 

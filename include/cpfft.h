@@ -215,10 +215,10 @@ int cpfft_set_cg_maxit(cpfft_ctx* ctx, int maxit);
  * with K4, without K4, the y passes (N <= 48: the inverse pass) and the x
  * pass on this context's buffers (reps launches each) and keeps the fastest.
  * The choice is cached per device and N (N <= 48: and operator) for every
- * context of the process (force != 0 measures again).  Only shapes that compute bit-identical results are candidates
- * (which block transforms which lines; never the radix order or a
- * reduction), so tuning changes speed, not results.  Returns 1 (nothing to
- * tune) for other N.                                                      */
+ * context of the process (force != 0 measures again).  Only shapes that
+ * compute bit-identical results are candidates (which block transforms which
+ * lines; never the radix order or a reduction), so tuning changes speed, not
+ * results.  Returns 1 (nothing to tune) for other N.                      */
 int cpfft_autotune(cpfft_ctx* ctx, int reps, int force);
 /* shapes in use: out[0] pencils per block of pass A with K4, out[1]
  * without K4, out[2] lines per block of the y passes, out[3] component
@@ -230,7 +230,8 @@ int cpfft_autotune(cpfft_ctx* ctx, int reps, int force);
  * there, and tangent_homo at 64 and 96 everywhere).  0 where N has no planned
  * path                                                                    */
 int cpfft_get_tune(cpfft_ctx* ctx, int out[4]);
-/* set them (each must be one of the candidates; -1 otherwise)             */
+/* set them (each must be one of the candidates; -1 otherwise).  N = 16, 32,
+ * 48: the pencils and lines per block of earlier versions select the default */
 int cpfft_set_tune(cpfft_ctx* ctx, const int in[4]);
 
 /* ---- diagnostics ------------------------------------------------------ */

@@ -311,3 +311,26 @@ def test_refused_edges_and_why(N, why):
     assert why in C.lib().cpfft_last_error().decode()
     if N <= 48:
         assert C.lib().cpfft_gkdf_noalloc(N, 1, 8, None, 16, None) == -3
+
+
+@pytest.mark.parametrize("N,former", [(16, [16, 8, 4, 18]), (32, [32, 16, 2, 9]), (48, [16, 12, 6, 18])])
+def test_shapes_a_program_kept_are_taken(N, former):
+    """launch shapes of 16, 32 and 48 from before these edges had kernels of their
+    own: taken, returned, without a change of results, and gone once tuned"""
+    s = _solver(N)
+    now = s.tune()
+    _rhs(s, N)
+    s.gkdf(C.B, C.WORK, 1)
+    ref = s.download(C.WORK)
+    s.set_tune(former)
+    assert s.tune() == former
+    s.gkdf(C.B, C.WORK, 1)
+    assert np.array_equal(s.download(C.WORK), ref)
+    s.set_tune(now)
+    assert s.tune() == now
+    with pytest.raises(C.CpfftError):
+        s.set_tune([7, *now[1:]])
+    assert s.tune() == now
+    s.set_tune(former)
+    assert s.autotune(reps=1, force=True)[3] < 9
+    s.close()
