@@ -1254,14 +1254,17 @@ static void fwd_slab(const Grid& g, const FwdArgs& a, int threads, hipStream_t s
 template <int NC, bool HASK, bool DIR>
 static void forward(const Grid& g, const FwdArgs& a, int cand, hipStream_t s) {
   const int t = slab_threads(g.N, cand);
-  if (NC == kAnyRadix && g.N > kSlabN) {
-    k_zf<HASK, DIR><<<8 * ((g.nzb + 7) / 8) * 3 * a.nrhs, 256,
-                      lds_lines(g.N, 3 * (g.TL / 2)), s>>>(g, a);
-  } else if (NC <= 0 && g.N > kE4N) {
-    fwd_slab<NC, kMaxE, HASK, DIR>(g, a, t, s);
-  } else {
-    fwd_slab<NC, NC == 96 ? 5 : 4, HASK, DIR>(g, a, t, s);
+  if constexpr (NC == kAnyRadix) {
+    if (g.N > kSlabN) {
+      k_zf<HASK, DIR><<<8 * ((g.nzb + 7) / 8) * 3 * a.nrhs, 256,
+                        lds_lines(g.N, 3 * (g.TL / 2)), s>>>(g, a);
+      return;
+    }
   }
+  if constexpr (NC <= 0) {
+    if (g.N > kE4N) return fwd_slab<NC, kMaxE, HASK, DIR>(g, a, t, s);
+  }
+  fwd_slab<NC, NC == 96 ? 5 : 4, HASK, DIR>(g, a, t, s);
 }
 
 // Edges of fft_pencil.hip: only tangent_homo's systems come here, with the
@@ -1298,12 +1301,16 @@ static void inv_slab(const Grid& g, const InvArgs& a, int nrhs, int threads, hip
 template <int NC, int MODE>
 static void inverse(const Grid& g, const InvArgs& a, int nrhs, int cand, hipStream_t s) {
   const int t = slab_threads(g.N, cand);
-  if (NC == kAnyRadix && g.N > kSlabN)
-    k_zi<MODE><<<dim3(g.nzb, 9, nrhs), 256, lds_lines(g.N, g.TL / 2), s>>>(g, a);
-  else if (NC <= 0 && g.N > kE4N)
-    inv_slab<NC, kMaxE, MODE>(g, a, nrhs, t, s);
-  else
-    inv_slab<NC, NC == 96 ? 5 : 4, MODE>(g, a, nrhs, t, s);
+  if constexpr (NC == kAnyRadix) {
+    if (g.N > kSlabN) {
+      k_zi<MODE><<<dim3(g.nzb, 9, nrhs), 256, lds_lines(g.N, g.TL / 2), s>>>(g, a);
+      return;
+    }
+  }
+  if constexpr (NC <= 0) {
+    if (g.N > kE4N) return inv_slab<NC, kMaxE, MODE>(g, a, nrhs, t, s);
+  }
+  inv_slab<NC, NC == 96 ? 5 : 4, MODE>(g, a, nrhs, t, s);
 }
 
 // spectrum entries per right-hand side; above kSlabN T2 follows T1
