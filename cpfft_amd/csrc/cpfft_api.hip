@@ -998,14 +998,15 @@ extern "C" int cpfft_pcg(cpfft_ctx* c, const double* b, double* x, double tol, i
       c->pcg_graphs.emplace_back(x, ge);
     }
   }
-  // (The first chunk is launched kernel by kernel also with graphs: zero_rhs.)
+  // (With graphs too, the first chunk is launched kernel by kernel where
+  // zero_rhs is asked within it.)
   int launched = 0;
   // the events of this solve follow the first ev0[f] of family f
   int ev0[cpfft_ctx::kFam];
   std::copy(c->ev_n, c->ev_n + cpfft_ctx::kFam, ev0);
   for (;;) {
-    if (graph && launched > 0) {
-      HIP_OK(hipGraphLaunch(ge, c->stream));
+    if (graph && (launched > 0 || zero_at(c) == 0)) {
+      if (launched > 0 || !zero_rhs(c)) HIP_OK(hipGraphLaunch(ge, c->stream));
     } else {
       if (c->timing && (c->ev_n[0] + kChunk > cpfft_ctx::kRing || c->ev_n[2] + kChunk > cpfft_ctx::kRing)) {
         flush_events(c);
