@@ -1448,28 +1448,22 @@ bool gkdf_grid_edge(int N) { return !(N == 64 || N == 96 || N == 128 || N == 256
 
 #define CPFFT_EDGE(call, large)     \
   switch (g.N) {                    \
-    case 16: gp::call<16> CPFFT_ARGS; break; \
-    case 32: gp::call<32> CPFFT_ARGS; break; \
-    case 48: gp::call<48> CPFFT_ARGS; break; \
-    large                           \
     default:                        \
       if (gp::smooth(g.N))          \
         gp::call<gp::kSmooth> CPFFT_ARGS; \
       else                          \
         gp::call<gp::kAnyRadix> CPFFT_ARGS; \
       break;                        \
+    case 16: gp::call<16> CPFFT_ARGS; break; \
+    case 32: gp::call<32> CPFFT_ARGS; break; \
+    case 48: gp::call<48> CPFFT_ARGS; break; \
+    large                           \
   }
 // with the edges of tangent_only
 #define CPFFT_EDGE_ALL(call)                         \
   CPFFT_EDGE(call, case 64: gp::call<64> CPFFT_ARGS; break; \
              case 96: gp::call<96> CPFFT_ARGS; break;)
 
-void launch_gkdf_grid(const SpecGeom& g, const double* F, const double* K4, double* out,
-                      cplx* spec, const cplx* tw, hipStream_t s) {
-#define CPFFT_ARGS (g, F, K4, out, spec, tw, s)
-  CPFFT_EDGE(run_gkdf, )
-#undef CPFFT_ARGS
-}
 void launch_cg_grid(const SpecGeom& g, const GridCG& c, int part, hipStream_t s) {
 #define CPFFT_ARGS (g, c, part, s)
   CPFFT_EDGE_ALL(run_cg)
@@ -1483,6 +1477,12 @@ void launch_homo_rhs_grid(const SpecGeom& g, const double* K4, int i0, int n, do
 #undef CPFFT_ARGS
 }
 
+void launch_gkdf_grid(const SpecGeom& g, const double* F, const double* K4, double* out,
+                      cplx* spec, const cplx* tw, hipStream_t s) {
+#define CPFFT_ARGS (g, F, K4, out, spec, tw, s)
+  CPFFT_EDGE(run_gkdf, )
+#undef CPFFT_ARGS
+}
 int grid_parts(int N) {
   SpecGeom s{};
   s.N = N;
