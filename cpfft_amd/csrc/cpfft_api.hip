@@ -149,7 +149,7 @@ static bool homo_grid(const SpecGeom& g) {
 // Chooses the systems per launch of tangent_homo on fft_grid.hip's kernels and
 // allocates their spectra, once, before the first solve or graph needs them: a
 // context that only solves does not hold them (585 MB at 96^3).  As many
-// systems as 700 MB hold, so all nine up to 96^3 (1.4 GB above 126^3, where a
+// systems as 700 MB hold, so all nine up to 103^3 (1.4 GB above 126^3, where a
 // transposed copy follows each), evenly over the launches; fewer if the device
 // has less.  (That the spectra outgrow the 256 MB memory-side cache costs less
 // than the launches: at 96^3 one, three and nine a launch took 85.0, 73.3 and
@@ -1096,15 +1096,13 @@ extern "C" int cpfft_drive_eps_sig(cpfft_ctx* c, int step, int iiter) {
 // K4 forms K4 : p_i for every solve still running, then each solve applies
 // the projection and its own CG update.  Each solve's arithmetic is that of
 // fftPcg on its own, so iterates and iteration counts are unchanged.
-// kChunk iterations of tangent_homo's nine CG solves (scalars in c->dcg9):
-// one K4 pass forms K4 : p_i for every running solve (and on the planned
-// path first p_i = r_i + beta_i p_i), then each solve applies the operator
-// without K4 in place and its own alpha, update and test.  Kernels of
-// finished solves return at once, so the chunk can be replayed from a graph.
+
 // Whether tangent_homo's K4:p_i are formed by a launch of their own, which
-// reads r and p once instead of once per component: from 40^3 on (48^3:
-// 10.7 against 12.8 ms a call; 32^3: 3.7 against 3.5, its blocks too few to
-// fill the chip).
+// reads r and p once instead of once per component, but has too few blocks to
+// fill the chip on the smaller grids: from 40^3 on.  A call took, with it and
+// without, 12.3 and 14.9 ms at 45^3, 8.7 and 12.1 at 48^3, but 3.7 and 3.1 at
+// 32^3, 7.2 and 5.2 at 36^3, and still 8.1 and 6.3 at 40^3 itself, so the line
+// would lie better just above it.
 static bool homo_contract(const cpfft_ctx* c) {
   return c->N >= 40 && gkdf_slab_edge(c->N);
 }
@@ -1186,6 +1184,11 @@ static void enqueue_homo_grid(cpfft_ctx* c) {
   }
 }
 
+// kChunk iterations of tangent_homo's nine CG solves (scalars in c->dcg9).  On
+// the planned path one K4 pass forms p_i = r_i + beta_i p_i and K4 : p_i for
+// every running solve, then each solve applies the operator without K4 in
+// place and its own alpha, update and test.  Kernels of finished solves return
+// at once, so the chunk can be replayed from a graph.
 static void enqueue_homo_chunk(cpfft_ctx* c) {
   if (homo_grid(c->geom))
     return homo_contract(c) ? enqueue_homo_slab(c) : enqueue_homo_grid(c);

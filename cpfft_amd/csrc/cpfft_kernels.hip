@@ -448,10 +448,14 @@ void launch_k4_contract_multi(long V, const double* K4, const Ptr9& pp, const CG
 // kilobyte a lane and run 1.7 times as long).  So what is not needed is left
 // out of each instantiation: EXPL the explicit update of iteration 0, WARM
 // the warm-start candidates, MatParamsInt the calls to pow; scratch falls from 640
-// to 148 bytes a lane.  At 128^3, about five local iterations a voxel: 3.31 ms
-// for fcc (61% of the cycles issue) against 5.83 with the stages of the local
-// solve, their line searches and the general parameters inlined one after
-// another and slip systems taken one at a time (45%).
+// to 148 bytes a lane (with the candidates 512, and 720 with the general
+// parameters, which always have them).  At 128^3, about five local iterations
+// a voxel: 3.31 ms for fcc (60% of a wave's cycles issue a vector instruction,
+// 28% wait) against 5.83 with the stages of the local solve, their line
+// searches and the general parameters inlined one after another and slip
+// systems taken one at a time.  The candidates' registers cost what they save:
+// from the previous iterate 2.86 ms a call against 2.75 over load steps 6 to 25
+// of the 128^3 workload, with 1.68 local iterations a voxel instead of 3.01.
 template <int NS, bool EXPL, bool WARM, class MP>
 __global__ __launch_bounds__(64) void k_drive_eps_sig(long V, MP P,
                                                       const Orient<NS>* __restrict__ orients,
@@ -531,7 +535,7 @@ void launch_drive_eps_sig(long V, const MatParams& P, const Orient<NS>* orients,
   };
   const std::true_type yes;
   const std::false_type no;
-  // the narrowest instantiation that covers the call
+  // (other materials' Newton iterations have one form, with the candidates)
   const bool simple = P.int_rate && P.m_is_one, warm = ws || warm_prev;
   if (iter == 0)
     update(yes, no, P);

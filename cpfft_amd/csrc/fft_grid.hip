@@ -688,10 +688,13 @@ __device__ __forceinline__ void form_alpha(const MidArgs& a, int rhs) {
 // k_fwd: block = (x, component, right-hand side); blockIdx.x as where().
 // One buffer: the line pairs [m][z], after the z transforms (through
 // registers) the half spectrum [kz][y].  One component a block: three (F read
-// three times instead of nine) took as long at 32^3 and 48^3, and with the
-// contraction in it the kernel is slower than fft_pencil.hip's pass A from
-// 64^3 on (56 against 41 us), where the F of the slabs in flight outgrows an
-// XCD's L2.
+// three times instead of nine) took as long for one system at 32^3 and 48^3.
+// The blocks of a slab share F through their XCD's L2 (798 B a voxel are
+// fetched at 32^3, 855 at 90^3, 865 at 126^3, of the 792 that K4, r and p are),
+// but with the contraction in it the kernel is slower than fft_pencil.hip's
+// pass A from 64^3 on (56 against 41 us): loads, transforms and stores of a
+// block follow one another, and from 64^3 its threads and LDS leave room for
+// one block a CU, so the stream stops meanwhile (2.6 TB/s at 90^3).
 template <int NC, int ME, bool HASK, bool DIR, bool AHEAD>
 __global__ __launch_bounds__(1024) void k_fwd(Grid g, FwdArgs a) {
   extern __shared__ cplx lds[];

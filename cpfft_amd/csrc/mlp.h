@@ -84,7 +84,7 @@ void mlp_stats(const MlpBuffers& b, long count, hipStream_t s);
 // Inference over all voxels in one launch: ws[k][e] = the network's output
 // k for the normalised inputs Xv[e] (row stride mlp_nin_pad(nin)),
 // denormalised (the weights must be in pbf).  BF16 operands, FP32
-// accumulation, the the rounding points of mlp_forward.
+// accumulation, the rounding points of mlp_forward.
 void mlp_infer(const MlpBuffers& b, long V, hipStream_t s);
 
 }  // namespace cpfft

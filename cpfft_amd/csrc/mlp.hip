@@ -12,7 +12,7 @@
 // needs in the registers of the lanes that made them, and writes what the
 // weight gradients read with the rows contiguous.  k_mlp_grad gives each
 // 16 x 16 tile of a weight gradient to one wave, which sums over all rows in
-// order, and applies Adam to it.  A step on 4096 rows takes 33 us (21 + 13)
+// order, and applies Adam to it.  A step on 4096 rows takes 33 us (20 + 13)
 // where one launch per product and reduction took 505 us, 381 of them in the
 // three weight gradients (6 to 64 waves, two-byte loads across the rows).
 #include "mlp.h"
